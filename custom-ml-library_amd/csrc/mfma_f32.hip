@@ -23,6 +23,19 @@
 // is half the banks and the segment reads take two passes).  Tiles reach LDS
 // by direct buffer loads (DMA), each lane fetching the global chunk its
 // swizzled position holds; rows past the buffer range arrive as zeros.
+//
+// Masks (template MK): 0 = none, or a [B,1,1,K] key mask reduced to kv_len /
+// kv_prefix; 1 = any other boolean mask; 2 / 3 = an additive f32 / (f16 or
+// bf16) mask, each of any broadcast strides.  A wave reads its next tile's
+// 32 x 32 mask elements into registers while it multiplies the current one
+// (an fp32 tile is thousands of MFMA cycles, so the loads never wait), and
+// skips the products of a tile that no element of the mask allows -- most of
+// a packed-documents mask.  Additive masks keep the softmax in natural units
+// (x = s scale + mask, P = exp2((x - m) log2 e)): a mask of -FLT_MAX times
+// log2 e would overflow to -inf and turn a row of such keys, whose softmax is
+// their mean, into an empty one.  B4 H8 S777 D64, a [B,1,S,S] mask of three
+// documents a row and the causal flag, forward + backward: on the generic
+// kernels these problems ran on before 1455 us, here 180 us.
 #include "mfma_common.h"
 
 namespace tsattn {
@@ -85,11 +98,100 @@ int device_cus() {
   return cus[dev];
 }
 
+// The general mask over a wave's 32 x 32 tile, read one tile ahead.
+//
+// Query rows in lanes (forward, dQ): lane (c, h) wants row c at the 16 keys
+// crow(i, h).  Boolean elements are loaded with the keys across the lanes --
+// load k takes rows 2 k + h, two whole row pieces per instruction -- and a
+// ballot per load gives the rows' bits, of which each lane keeps its own row's
+// (its bit j = key j).  Additive elements are loaded where they are used.
+// Keys in lanes (dK/dV): lane (c, h) wants key c at the 16 rows crow(i, h),
+// which is one load of two row pieces per element; boolean ones pack to bit i.
+// Offsets past the mask's extent read as zero; elements the kernel does not
+// allow are not used.
+template <int MK>
+struct F32Mask {
+  uint32_t raw[16];
+  uint32_t bits;  // MK 1: the current tile's bits
+  float add[16];  // MK 2, 3: the current tile's elements
+  bool any;       // the mask allows some element of the current tile
+  static constexpr int ES = MK == 1 ? 1 : (MK == 2 ? 4 : 2);
+
+  __device__ __forceinline__ uint32_t load(rsrc_t r, uint32_t off) const {
+    if constexpr (MK == 1) return __builtin_amdgcn_raw_buffer_load_b8(r, static_cast<int>(off), 0, 0);
+    else if constexpr (MK == 2) return __builtin_amdgcn_raw_buffer_load_b32(r, static_cast<int>(off), 0, 0);
+    else return __builtin_amdgcn_raw_buffer_load_b16(r, static_cast<int>(off), 0, 0);
+  }
+  // the (b, hq) slice of the mask
+  __device__ __forceinline__ static rsrc_t slice(const Problem &p, int b, int hq) {
+    const int64_t extent = ((p.Sq - 1) * p.mask.s2 + (p.Sk - 1) * p.mask.s3 + 1) * ES;
+    return make_rsrc(static_cast<const char *>(p.mask.data) + (b * p.mask.s0 + hq * p.mask.s1) * ES,
+                     static_cast<uint32_t>(extent));
+  }
+  // rows in lanes: tile of rows row0 .. + 31, keys key0 .. + 31
+  __device__ __forceinline__ void issue_rows(const Problem &p, rsrc_t r, int row0, int key0, int c, int h) {
+    const uint32_t s2 = static_cast<uint32_t>(p.mask.s2) * ES, s3 = static_cast<uint32_t>(p.mask.s3) * ES;
+    if constexpr (MK == 1) {
+      const uint32_t off = static_cast<uint32_t>(row0 + h) * s2 + static_cast<uint32_t>(key0 + c) * s3;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) raw[k] = load(r, off + static_cast<uint32_t>(2 * k) * s2);
+    } else {
+      const uint32_t off = static_cast<uint32_t>(row0 + c) * s2 + static_cast<uint32_t>(key0 + 4 * h) * s3;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) raw[i] = load(r, off + static_cast<uint32_t>(8 * (i >> 2) + (i & 3)) * s3);
+    }
+  }
+  // keys in lanes: the same tile, this lane's key key0 + c
+  __device__ __forceinline__ void issue_keys(const Problem &p, rsrc_t r, int row0, int key0, int c, int h) {
+    const uint32_t s2 = static_cast<uint32_t>(p.mask.s2) * ES, s3 = static_cast<uint32_t>(p.mask.s3) * ES;
+    const uint32_t off = static_cast<uint32_t>(row0 + 4 * h) * s2 + static_cast<uint32_t>(key0 + c) * s3;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) raw[i] = load(r, off + static_cast<uint32_t>(8 * (i >> 2) + (i & 3)) * s2);
+  }
+  // the issued tile becomes the current one
+  template <bool ROWS>
+  __device__ __forceinline__ void take(const Problem &p, int c, int h) {
+    if constexpr (MK == 1) {
+      bits = 0;
+      if constexpr (ROWS) {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+          const uint64_t two = __ballot(raw[k] != 0u);
+          const uint32_t lo = static_cast<uint32_t>(two), hi = static_cast<uint32_t>(two >> 32);
+          bits = c == 2 * k ? lo : bits;
+          bits = c == 2 * k + 1 ? hi : bits;
+        }
+        any = __ballot(bits != 0u) != 0ull;
+        bits >>= 4 * h;  // bit 8 (i / 4) + i % 4 is element i's key
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) bits |= raw[i] != 0u ? 1u << (8 * (i >> 2) + (i & 3)) : 0u;
+        any = __ballot(bits != 0u) != 0ull;
+      }
+    } else {
+      float mx = -INFINITY;
+      bool nan = false;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        if constexpr (MK == 2) add[i] = __builtin_bit_cast(float, raw[i]);
+        else if (p.mask.dtype == TSATTN_BF16) add[i] = __builtin_bit_cast(float, raw[i] << 16);
+        else add[i] = static_cast<float>(__builtin_bit_cast(f16, static_cast<uint16_t>(raw[i])));
+        mx = fmaxf(mx, add[i]);
+        nan |= add[i] != add[i];
+      }
+      any = __ballot(mx > -INFINITY || nan) != 0ull;
+    }
+  }
+};
+
 struct F32Args {
   Problem p;
   View q, k, v, o, dout, dq, dk, dv;
   float *lse;
-  float *rows;  // backward row values: [rows] -delta, then [rows] -safe(lse) / scale
+  // backward row values: [rows] -delta, then [rows] -safe(lse) / scale (additive
+  // masks: -safe(lse), their scores being scaled already)
+  float *rows;
+  int lse_scaled;
   float sl;     // scale * log2(e)
   float scale;
 };
@@ -110,7 +212,7 @@ struct F32Args {
 // online softmax merges tiles: the key loop of a row block runs 4 ways
 // parallel.  One workgroup per CU.
 // ---------------------------------------------------------------------------
-template <int D, bool SPLIT>
+template <int D, bool SPLIT, int MK>
 __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
   using TL = FTile<D>;
   constexpr int HD = D / 2;             // MFMA steps over the head dimension
@@ -140,7 +242,7 @@ __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
   const int b = bh / p.Hq, hq = bh - b * p.Hq, hk = hq / p.rep;
   const int q0 = qb * ROWS, qw = SPLIT ? q0 : q0 + 32 * w, qrow = qw + c;
   const int kv_end = kv_end_for(p, b);
-  const bool keymask = p.mask.kind == TSATTN_MASK_BOOL && !(p.kv_prefix && p.kv_prefix[b]);
+  const bool keymask = MK == 0 && p.mask.kind == TSATTN_MASK_BOOL && !(p.kv_prefix && p.kv_prefix[b]);
 
   int64_t lim = kv_end, wlim = kv_end;
   if (p.causal) {
@@ -211,7 +313,13 @@ __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
 #pragma unroll
   for (int dt = 0; dt < PDT; ++dt) oacc[dt] = f32x16{};
   float m = -INFINITY, l = 0.f, thr = -INFINITY, nbase = 0.f;
-  const float sl = a.sl, inv_sl = 1.f / sl;
+  // Units of the running maximum and the exponent: log2 (scores times sl), or
+  // with an additive mask natural (the masked score is scaled already).
+  constexpr bool ADD = MK >= 2;
+  const float sl = ADD ? 1.f : a.sl, inv_sl = 1.f / sl;
+  const float tau = ADD ? kTau * kLn2 : kTau;
+  // exp of a difference in those units
+  auto exp_u = [](float x) { return fast_exp2(ADD ? x * kLog2e : x); };
   int klim = kv_end;
   if (p.causal) {
     const int64_t cl = static_cast<int64_t>(qrow) + p.offset + 1;
@@ -219,12 +327,17 @@ __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
   }
   const uint8_t *kmask_b = keymask ? static_cast<const uint8_t *>(p.mask.data) + b * p.mask.s0 : nullptr;
   int j_edge = kv_end / BN;
-  if (keymask) j_edge = 0;
+  if (MK != 0 || keymask) j_edge = 0;
   if (p.causal) {
     const int64_t dd = static_cast<int64_t>(qw) + p.offset - (BN - 1);
     const int jc = dd < 0 ? 0 : static_cast<int>(min(dd / BN + 1, static_cast<int64_t>(INT32_MAX)));
     j_edge = min(j_edge, jc);
   }
+
+  // general mask: this wave's next tile in flight beside the tile it multiplies
+  F32Mask<MK> mask;
+  const rsrc_t mrs = F32Mask<MK>::slice(p, b, hq);
+  if constexpr (MK != 0) mask.issue_rows(p, mrs, qw, first * BN, c, h);
 
 #pragma unroll
   for (int u = 0; u < PARTS; ++u) issue_part(0, u);
@@ -246,7 +359,13 @@ __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
     const int j = first + STRIDE * jj;
     const char *kt = ring_p + (jj & 1) * STAGE;
     const char *vt = kt + TL::BYTES;
-    if (SPLIT || j < w_tiles) {
+    bool work = SPLIT || j < w_tiles;
+    if constexpr (MK != 0) {
+      mask.template take<true>(p, c, h);
+      mask.issue_rows(p, mrs, qw, (j + STRIDE) * BN, c, h);  // (past the last tile: not used)
+      work = work && mask.any;
+    }
+    if (work) {
       // S^T = K Q^T, the next tile's parts spread over the steps; each
       // 16-byte chunk of K serves four steps, read one chunk ahead
       f32x16 s = f32x16{};
@@ -279,9 +398,11 @@ __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
           const bool ok = key < p.Sk && kmask_b[static_cast<int64_t>(key) * p.mask.s3];
           kbits = static_cast<unsigned>(__ballot(ok) >> (4 * h));
         }
+        if constexpr (MK == 1) kbits = mask.bits;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const int kc_ = 8 * (i >> 2) + (i & 3);
+          if constexpr (ADD) s[i] = fmaf(s[i], a.scale, mask.add[i]);
           s[i] = ((kc_ < lm) & (((kbits >> kc_) & 1u) != 0)) ? s[i] : -INFINITY;
         }
       }
@@ -291,9 +412,9 @@ __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
       const float mxr = half_swap_max3(mx);
       if (__ballot(mxr > thr) != 0ull) {
         const float m_new = fmaxf(m, mxr * sl);
-        const float corr = m_new == -INFINITY ? 1.f : fast_exp2(m - m_new);
+        const float corr = m_new == -INFINITY ? 1.f : exp_u(m - m_new);
         m = m_new;
-        thr = (m + kTau) * inv_sl;
+        thr = (m + tau) * inv_sl;
         nbase = m == -INFINITY ? 0.f : -m;
         l *= corr;
 #pragma unroll
@@ -301,7 +422,7 @@ __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
       }
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        s[i] = fast_exp2(fmaf(s[i], sl, nbase));
+        s[i] = exp_u(ADD ? s[i] + nbase : fmaf(s[i], sl, nbase));
         l += s[i];
       }
       // O^T += V^T P^T: step i takes keys crow(i, h) (register i of P^T); the
@@ -354,7 +475,7 @@ __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
                      oacc[dt][4 * g + 3] * inv};
       if (a.lse && h == 0)
         a.lse[(static_cast<int64_t>(b) * p.Hq + hq) * p.Sq + qrow] =
-            lt > 0.f ? (m + log2f(lt)) * kLn2 : -INFINITY;
+            lt > 0.f ? (ADD ? fmaf(log2f(lt), kLn2, m) : (m + log2f(lt)) * kLn2) : -INFINITY;
     }
   } else {
     // Merge the waves' partial rows: max mf = max_w m_w, sum L = sum_w l_w
@@ -381,7 +502,7 @@ __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
 #pragma unroll
     for (int v = 0; v < NW; ++v) {
       const float mv = cm[v * 32 + c];
-      sc[v] = mv == -INFINITY ? 0.f : fast_exp2(mv - mf);
+      sc[v] = mv == -INFINITY ? 0.f : exp_u(mv - mf);
       lsum += cl[v * 32 + c] * sc[v];
     }
     const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
@@ -398,7 +519,7 @@ __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
       }
       if (a.lse && w == 0 && h == 0)
         a.lse[(static_cast<int64_t>(b) * p.Hq + hq) * p.Sq + qrow] =
-            lsum > 0.f ? (mf + log2f(lsum)) * kLn2 : -INFINITY;
+            lsum > 0.f ? (ADD ? fmaf(log2f(lsum), kLn2, mf) : (mf + log2f(lsum)) * kLn2) : -INFINITY;
     }
   }
 }
@@ -429,7 +550,7 @@ __global__ __launch_bounds__(NT) void rows_f32_kernel(F32Args a) {
   if (live && g == 0) {
     const float lse = a.lse[rr];
     a.rows[rr] = -d;
-    a.rows[rows + rr] = isfinite(lse) ? -lse / a.scale : 0.f;
+    a.rows[rows + rr] = isfinite(lse) ? (a.lse_scaled ? -lse : -lse / a.scale) : 0.f;
   }
 }
 
@@ -446,7 +567,7 @@ __global__ __launch_bounds__(NT) void rows_f32_kernel(F32Args a) {
 // tiles w, w + 4, ... through its own ring, and the waves' dQ^T partial sums
 // add up through LDS in wave order at the end.
 // ---------------------------------------------------------------------------
-template <int D, bool SPLIT>
+template <int D, bool SPLIT, int MK>
 __global__ __launch_bounds__(NT, 1) void dq_f32_kernel(F32Args a) {
   using TL = FTile<D>;
   constexpr int HD = D / 2, PDT = D / 32;
@@ -473,7 +594,7 @@ __global__ __launch_bounds__(NT, 1) void dq_f32_kernel(F32Args a) {
   const int b = bh / p.Hq, hq = bh - b * p.Hq, hk = hq / p.rep;
   const int q0 = qb * ROWS, qw = SPLIT ? q0 : q0 + 32 * w, qrow = qw + c;
   const int kv_end = kv_end_for(p, b);
-  const bool keymask = p.mask.kind == TSATTN_MASK_BOOL && !(p.kv_prefix && p.kv_prefix[b]);
+  const bool keymask = MK == 0 && p.mask.kind == TSATTN_MASK_BOOL && !(p.kv_prefix && p.kv_prefix[b]);
   int64_t lim = kv_end, wlim = kv_end;
   if (p.causal) {
     lim = min(lim, static_cast<int64_t>(min(q0 + ROWS, p.Sq) - 1) + p.offset + 1);
@@ -545,7 +666,7 @@ __global__ __launch_bounds__(NT, 1) void dq_f32_kernel(F32Args a) {
   }
   const uint8_t *kmask_b = keymask ? static_cast<const uint8_t *>(p.mask.data) + b * p.mask.s0 : nullptr;
   int j_edge = kv_end / BN;
-  if (keymask) j_edge = 0;
+  if (MK != 0 || keymask) j_edge = 0;
   if (p.causal) {
     const int64_t dd = static_cast<int64_t>(qw) + p.offset - (BN - 1);
     const int jc = dd < 0 ? 0 : static_cast<int>(min(dd / BN + 1, static_cast<int64_t>(INT32_MAX)));
@@ -555,6 +676,9 @@ __global__ __launch_bounds__(NT, 1) void dq_f32_kernel(F32Args a) {
   f32x16 acc[PDT];
 #pragma unroll
   for (int dt = 0; dt < PDT; ++dt) acc[dt] = f32x16{};
+  F32Mask<MK> mask;  // one tile ahead, as in the forward
+  const rsrc_t mrs = F32Mask<MK>::slice(p, b, hq);
+  if constexpr (MK != 0) mask.issue_rows(p, mrs, qw, first * BN, c, h);
 
 #pragma unroll
   for (int u = 0; u < PARTS; ++u) issue_part(0, u);
@@ -577,7 +701,13 @@ __global__ __launch_bounds__(NT, 1) void dq_f32_kernel(F32Args a) {
     const int j = first + STRIDE * jj;
     const char *kt = ring_p + (jj & 1) * STAGE;
     const char *vt = kt + TL::BYTES;
-    if (SPLIT || j < w_tiles) {
+    bool work = SPLIT || j < w_tiles;
+    if constexpr (MK != 0) {
+      mask.template take<true>(p, c, h);
+      mask.issue_rows(p, mrs, qw, (j + STRIDE) * BN, c, h);  // (past the last tile: not used)
+      work = work && mask.any;
+    }
+    if (work) {
       f32x16 s = f32x16{}, dp = f32x16{};
       {
         constexpr int NC = HD / 4;
@@ -620,11 +750,15 @@ __global__ __launch_bounds__(NT, 1) void dq_f32_kernel(F32Args a) {
           const bool ok = key < p.Sk && kmask_b[static_cast<int64_t>(key) * p.mask.s3];
           kbits = static_cast<unsigned>(__ballot(ok) >> (4 * h));
         }
+        if constexpr (MK == 1) kbits = mask.bits;
       }
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int kc_ = 8 * (i >> 2) + (i & 3);
-        const float pv = ((kc_ < lm) & (((kbits >> kc_) & 1u) != 0)) ? fast_exp2((s[i] + nl) * sl) : 0.f;
+        float x;  // log2 P
+        if constexpr (MK >= 2) x = (fmaf(s[i], a.scale, mask.add[i]) + nl) * kLog2e;
+        else x = (s[i] + nl) * sl;
+        const float pv = ((kc_ < lm) & (((kbits >> kc_) & 1u) != 0)) ? fast_exp2(x) : 0.f;
         s[i] = pv * (dp[i] + nd);
       }
       // dQ^T += K^T dS^T: step i takes keys crow(i, h) (register i of dS^T)
@@ -706,7 +840,7 @@ __global__ __launch_bounds__(NT, 1) void dq_f32_kernel(F32Args a) {
 // of the (query head, query tile) walk through its own ring, and the waves'
 // dK^T / dV^T partial sums add up through LDS in wave order at the end.
 // ---------------------------------------------------------------------------
-template <int D, bool SPLIT>
+template <int D, bool SPLIT, int MK>
 __global__ __launch_bounds__(NT, 1) void dkdv_f32_kernel(F32Args a) {
   using TL = FTile<D>;
   constexpr int HD = D / 2, PDT = D / 32;
@@ -732,7 +866,7 @@ __global__ __launch_bounds__(NT, 1) void dkdv_f32_kernel(F32Args a) {
   const int b = bh / p.Hkv, hk = bh - b * p.Hkv;
   const int k0 = kb * KEYS, kw = SPLIT ? k0 : k0 + 32 * w, key = kw + c;
   const int kv_end = kv_end_for(p, b);
-  const bool keymask = p.mask.kind == TSATTN_MASK_BOOL && !(p.kv_prefix && p.kv_prefix[b]);
+  const bool keymask = MK == 0 && p.mask.kind == TSATTN_MASK_BOOL && !(p.kv_prefix && p.kv_prefix[b]);
   const bool key_live = key < kv_end &&
                         (!keymask || static_cast<const uint8_t *>(p.mask.data)[b * p.mask.s0 + static_cast<int64_t>(key) * p.mask.s3]);
   int q_start = 0;
@@ -789,12 +923,15 @@ __global__ __launch_bounds__(NT, 1) void dkdv_f32_kernel(F32Args a) {
   const char *ring_p = lds + (SPLIT ? w * 2 * STAGE : 0);
   const uint32_t spare = lds0 + RINGS * 2 * STAGE;
   // the loads of local tile jj (tile first + STRIDE jj): this wave's share of
-  // its Q / dO blocks (split: all of them) and row values
+  // its Q / dO blocks (split: all of them) and row values, and its part of a
+  // general mask
+  F32Mask<MK> mask;
   auto issue = [&](int jj) {
     const int it = first + STRIDE * jj;
     const bool real = it < n_iter;
     const int r = real ? it / n_qt : 0, qi = real ? it - r * n_qt : 0;
     const int hq = hk * p.rep + r, q0 = q_start + qi * BN;
+    if constexpr (MK != 0) mask.issue_keys(p, F32Mask<MK>::slice(p, b, hq), q0, kw, c, h);
     const uint32_t st = real ? ring + (jj & 1) * STAGE : spare;
     const u32x4 qd = make_desc(f32_head<float>(a.q, b, hq), static_cast<uint32_t>(p.Sq) * qs_b);
     const u32x4 gd = make_desc(f32_head<float>(a.dout, b, hq), static_cast<uint32_t>(p.Sq) * gs_b);
@@ -844,7 +981,13 @@ __global__ __launch_bounds__(NT, 1) void dkdv_f32_kernel(F32Args a) {
     const float *rvl = reinterpret_cast<const float *>(qt + 2 * TL::BYTES);  // nl [32] | nd [32]
     const int r = it / n_qt, qi = it - r * n_qt;
     const int q0 = q_start + qi * BN;
+    bool work = true;
+    if constexpr (MK != 0) {
+      mask.template take<false>(p, c, h);
+      work = mask.any;
+    }
     issue(jj + 1);
+    if (work) {
     // S = Q K^T, dP = dO V^T over the tile's 32 rows x this wave's 32 keys
     f32x16 s = f32x16{}, dp = f32x16{};
     {
@@ -876,8 +1019,12 @@ __global__ __launch_bounds__(NT, 1) void dkdv_f32_kernel(F32Args a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int rr = 8 * (i >> 2) + 4 * h + (i & 3);
-      const bool ok = key_live && (q0 + rr < p.Sq) && (!p.causal || kdiff <= q0 + rr);
-      const float pv = ok ? fast_exp2((s[i] + rvl[rr]) * sl) : 0.f;
+      bool ok = key_live && (q0 + rr < p.Sq) && (!p.causal || kdiff <= q0 + rr);
+      if constexpr (MK == 1) ok = ok && ((mask.bits >> (8 * (i >> 2) + (i & 3))) & 1u);
+      float x;  // log2 P
+      if constexpr (MK >= 2) x = (fmaf(s[i], a.scale, mask.add[i]) + rvl[rr]) * kLog2e;
+      else x = (s[i] + rvl[rr]) * sl;
+      const float pv = ok ? fast_exp2(x) : 0.f;
       s[i] = pv;
       dp[i] = pv * (dp[i] + rvl[BN + rr]);
     }
@@ -901,6 +1048,7 @@ __global__ __launch_bounds__(NT, 1) void dkdv_f32_kernel(F32Args a) {
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    }  // work
     wait_vm_n<0>();
     if constexpr (SPLIT) wait_lgkm0();  // (this wave's ring only)
     else __syncthreads();
@@ -955,7 +1103,7 @@ __global__ __launch_bounds__(NT, 1) void dkdv_f32_kernel(F32Args a) {
   }
 }
 
-template <int D>
+template <int D, int MK>
 void launch_bwd_dims(const F32Args &a, hipStream_t st) {
   const Problem &p = a.p;
   {
@@ -973,37 +1121,51 @@ void launch_bwd_dims(const F32Args &a, hipStream_t st) {
   }
   if (split_q) {
     if constexpr (D <= 64) {
-      Probe pr_("bwd_dq_mfma_f32_split", st);
-      dq_f32_kernel<D, true><<<dim3(static_cast<unsigned>((p.Sq + 31) / 32 * qheads)), dim3(NT), 0, st>>>(a);
+      Probe pr_(MK ? "bwd_dq_mfma_f32_masked_split" : "bwd_dq_mfma_f32_split", st);
+      dq_f32_kernel<D, true, MK><<<dim3(static_cast<unsigned>((p.Sq + 31) / 32 * qheads)), dim3(NT), 0, st>>>(a);
     }
   } else {
-    Probe pr_("bwd_dq_mfma_f32", st);
-    dq_f32_kernel<D, false><<<dim3(static_cast<unsigned>(n_qb * qheads)), dim3(NT), 0, st>>>(a);
+    Probe pr_(MK ? "bwd_dq_mfma_f32_masked" : "bwd_dq_mfma_f32", st);
+    dq_f32_kernel<D, false, MK><<<dim3(static_cast<unsigned>(n_qb * qheads)), dim3(NT), 0, st>>>(a);
   }
   if (split_k) {
     if constexpr (D <= 64) {
-      Probe pr_("bwd_dkdv_mfma_f32_split", st);
-      dkdv_f32_kernel<D, true><<<dim3(static_cast<unsigned>((p.Sk + 31) / 32 * kheads)), dim3(NT), 0, st>>>(a);
+      Probe pr_(MK ? "bwd_dkdv_mfma_f32_masked_split" : "bwd_dkdv_mfma_f32_split", st);
+      dkdv_f32_kernel<D, true, MK><<<dim3(static_cast<unsigned>((p.Sk + 31) / 32 * kheads)), dim3(NT), 0, st>>>(a);
     }
   } else {
-    Probe pr_("bwd_dkdv_mfma_f32", st);
-    dkdv_f32_kernel<D, false><<<dim3(static_cast<unsigned>(n_kb * kheads)), dim3(NT), 0, st>>>(a);
+    Probe pr_(MK ? "bwd_dkdv_mfma_f32_masked" : "bwd_dkdv_mfma_f32", st);
+    dkdv_f32_kernel<D, false, MK><<<dim3(static_cast<unsigned>(n_kb * kheads)), dim3(NT), 0, st>>>(a);
   }
 }
 
-template <int D>
+template <int D, int MK>
 void launch_fwd_dims(const F32Args &a, hipStream_t st) {
   const int64_t heads = static_cast<int64_t>(a.p.Hq) * a.p.B;
   const int64_t n_qb = (a.p.Sq + BM - 1) / BM;
   if constexpr (D <= 64) {  // (the split rings of D = 128 would not fit in LDS)
     if (n_qb * heads < device_cus()) {
-      Probe pr_("fwd_mfma_f32_split", st);
-      fwd_f32_kernel<D, true><<<dim3(static_cast<unsigned>((a.p.Sq + 31) / 32 * heads)), dim3(NT), 0, st>>>(a);
+      Probe pr_(MK ? "fwd_mfma_f32_masked_split" : "fwd_mfma_f32_split", st);
+      fwd_f32_kernel<D, true, MK><<<dim3(static_cast<unsigned>((a.p.Sq + 31) / 32 * heads)), dim3(NT), 0, st>>>(a);
       return;
     }
   }
-  Probe pr_("fwd_mfma_f32", st);
-  fwd_f32_kernel<D, false><<<dim3(static_cast<unsigned>(n_qb * heads)), dim3(NT), 0, st>>>(a);
+  Probe pr_(MK ? "fwd_mfma_f32_masked" : "fwd_mfma_f32", st);
+  fwd_f32_kernel<D, false, MK><<<dim3(static_cast<unsigned>(n_qb * heads)), dim3(NT), 0, st>>>(a);
+}
+
+template <int MK>
+void launch_fwd_mask(const F32Args &a, hipStream_t st) {
+  if (a.p.Dqk == 128) launch_fwd_dims<128, MK>(a, st);
+  else if (a.p.Dqk == 64) launch_fwd_dims<64, MK>(a, st);
+  else launch_fwd_dims<32, MK>(a, st);
+}
+
+template <int MK>
+void launch_bwd_mask(const F32Args &a, hipStream_t st) {
+  if (a.p.Dqk == 128) launch_bwd_dims<128, MK>(a, st);
+  else if (a.p.Dqk == 64) launch_bwd_dims<64, MK>(a, st);
+  else launch_bwd_dims<32, MK>(a, st);
 }
 
 }  // namespace
@@ -1018,9 +1180,12 @@ hipError_t launch_mfma_f32_backward(const Problem &p, View q, View k, View v, Vi
   a.rows = rows;
   a.sl = static_cast<float>(p.scale) * kLog2e;
   a.scale = static_cast<float>(p.scale);
-  if (p.Dqk == 128) launch_bwd_dims<128>(a, st);
-  else if (p.Dqk == 64) launch_bwd_dims<64>(a, st);
-  else launch_bwd_dims<32>(a, st);
+  const int mk = mfma_mask_mode(p);
+  a.lse_scaled = mk >= 2;
+  if (mk == 0) launch_bwd_mask<0>(a, st);
+  else if (mk == 1) launch_bwd_mask<1>(a, st);
+  else if (mk == 2) launch_bwd_mask<2>(a, st);
+  else launch_bwd_mask<3>(a, st);
   return hipGetLastError();
 }
 
@@ -1028,9 +1193,13 @@ bool mfma_f32_supported(const Problem &p, int dtype) {
   if (dtype != TSATTN_F32 || p.Dqk != p.Dv) return false;
   if (p.Dqk != 32 && p.Dqk != 64 && p.Dqk != 128) return false;
   if (!(p.scale > 0.0) || p.drop.on || p.rope.R > 0) return false;
-  // masks: none, or a [B,1,1,K] boolean key mask reduced to lengths
-  return p.mask.kind == TSATTN_MASK_NONE ||
-         (p.mask.kind == TSATTN_MASK_BOOL && p.mask.s1 == 0 && p.mask.s2 == 0 && p.kv_len != nullptr);
+  // masks: any boolean one, or an additive one in f32 / f16 / bf16, read with
+  // 32-bit offsets (f64 masks keep their precision on the generic kernels).
+  // Additive masks over fewer than 128 query rows (one workgroup's) stay on
+  // the generic kernels, where such problems are checked to run: not for
+  // speed (B1 H2 S96 D64 forward + backward 137 us there, 45 us here).
+  if (p.mask.kind == TSATTN_MASK_ADDITIVE && p.Sq < BM) return false;
+  return mfma_mask_ok(p);
 }
 
 hipError_t launch_mfma_f32_forward(const Problem &p, View q, View k, View v, View o, float *lse,
@@ -1041,9 +1210,11 @@ hipError_t launch_mfma_f32_forward(const Problem &p, View q, View k, View v, Vie
   a.lse = lse;
   a.sl = static_cast<float>(p.scale) * kLog2e;
   a.scale = static_cast<float>(p.scale);
-  if (p.Dqk == 128) launch_fwd_dims<128>(a, st);
-  else if (p.Dqk == 64) launch_fwd_dims<64>(a, st);
-  else launch_fwd_dims<32>(a, st);
+  const int mk = mfma_mask_mode(p);
+  if (mk == 0) launch_fwd_mask<0>(a, st);
+  else if (mk == 1) launch_fwd_mask<1>(a, st);
+  else if (mk == 2) launch_fwd_mask<2>(a, st);
+  else launch_fwd_mask<3>(a, st);
   return hipGetLastError();
 }
 

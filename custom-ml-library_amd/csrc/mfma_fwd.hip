@@ -594,17 +594,7 @@ bool mfma_supported(const Problem &p, int dtype) {
   // the backward reads each (b, h) slice of the dropout keep bits with 32-bit offsets
   if (p.drop.on && static_cast<int64_t>((p.Sk + 31) / 32) * ((p.Sq + 3) / 4 * 4) * 4 >= (int64_t(1) << 31))
     return false;
-  if (p.mask.kind == TSATTN_MASK_ADDITIVE && p.mask.dtype != TSATTN_F32 &&
-      p.mask.dtype != TSATTN_F16 && p.mask.dtype != TSATTN_BF16)
-    return false;
-  const int mk = mfma_mask_mode(p);
-  if (mk == 0) return true;
-  // General masks are read with 32-bit byte offsets inside each (b, h) slice,
-  // rows and keys padded to whole tiles.
-  const MaskDesc &m = p.mask;
-  if (m.s0 < 0 || m.s1 < 0 || m.s2 < 0 || m.s3 < 0) return false;
-  const int64_t es = mk == 1 ? 1 : (mk == 2 ? 4 : 2);
-  return ((p.Sq + 128) * m.s2 + (p.Sk + 128) * m.s3 + 1) * es < (int64_t(1) << 31);
+  return mfma_mask_ok(p);
 }
 
 hipError_t launch_mfma_forward(const Problem &p, int dtype, View q, View k, View v, View o,

@@ -116,6 +116,20 @@ inline int mfma_mask_mode(const Problem &p) {
   if (p.mask.kind != TSATTN_MASK_ADDITIVE) return 0;
   return p.mask.dtype == TSATTN_F32 ? 2 : 3;
 }
+// Whether the MFMA kernels can read the problem's mask: not an f64 one, and a
+// general mask with 32-bit byte offsets inside each (b, h) slice, rows and
+// keys padded to whole tiles.
+inline bool mfma_mask_ok(const Problem &p) {
+  if (p.mask.kind == TSATTN_MASK_ADDITIVE && p.mask.dtype != TSATTN_F32 &&
+      p.mask.dtype != TSATTN_F16 && p.mask.dtype != TSATTN_BF16)
+    return false;
+  const int mk = mfma_mask_mode(p);
+  if (mk == 0) return true;
+  const MaskDesc &m = p.mask;
+  if (m.s0 < 0 || m.s1 < 0 || m.s2 < 0 || m.s3 < 0) return false;
+  const int64_t es = mk == 1 ? 1 : (mk == 2 ? 4 : 2);
+  return ((p.Sq + 128) * m.s2 + (p.Sk + 128) * m.s3 + 1) * es < (int64_t(1) << 31);
+}
 // The same, read as 16-byte row pieces (modes 4..6) where the keys are
 // contiguous and every row starts 16-byte aligned.
 inline int mfma_mask_mode_vec(const Problem &p) {
@@ -190,7 +204,7 @@ int mfma_ds_chunk_groups(const Problem &p);
 size_t mfma_rope_stage_offset(const Problem &p);
 
 // fp32 MFMA kernels (mfma_f32.hip): fp32, Dqk = Dv in {32, 64, 128}, no
-// dropout / folded RoPE, masks none or a key mask reduced to lengths.
+// dropout / folded RoPE, any boolean mask or an additive one in f32 / f16 / bf16.
 bool mfma_f32_supported(const Problem &p, int dtype);
 hipError_t launch_mfma_f32_forward(const Problem &p, View q, View k, View v, View o, float *lse,
                                    hipStream_t st);
