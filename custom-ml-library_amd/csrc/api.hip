@@ -9,6 +9,7 @@
 #include <stdio.h>
 
 #include <atomic>
+#include <initializer_list>
 
 #include "mfma_common.h"
 
@@ -352,6 +353,31 @@ int decode_forward(const tsattn_problem *p, const tsattn_rope_desc *rope, const 
                     "decode launch");
 }
 
+// Arrays of the layer kernels: f32 / f16 / bf16, given and 16-byte aligned.
+int check_flat(int32_t dtype, int64_t n, std::initializer_list<const void *> arrays) {
+  if (dtype != TSATTN_F32 && dtype != TSATTN_F16 && dtype != TSATTN_BF16)
+    return fail(TSATTN_ERR_INVALID, "the layer kernels take dtype f32, f16 or bf16 (got dtype %d)", dtype);
+  if (n <= 0) return fail(TSATTN_ERR_INVALID, "the layer kernels need positive sizes");
+  for (const void *p : arrays) {
+    if (!p) return fail(TSATTN_ERR_INVALID, "data pointer is NULL");
+    if (reinterpret_cast<uintptr_t>(p) % 16)
+      return fail(TSATTN_ERR_UNSUPPORTED, "the layer kernels need 16-byte aligned arrays");
+  }
+  if (n % 8) return fail(TSATTN_ERR_UNSUPPORTED, "the layer kernels take multiples of 8 elements");
+  return TSATTN_OK;
+}
+
+int check_norm(int32_t dtype, int32_t w_dtype, int64_t rows, int32_t dim,
+               std::initializer_list<const void *> arrays, std::initializer_list<const void *> optional) {
+  if (rows <= 0) return fail(TSATTN_ERR_INVALID, "the layer kernels need positive sizes");
+  int rc = check_flat(dtype, dim, arrays);
+  if (!rc) rc = check_flat(w_dtype, dim, {});
+  for (const void *p : optional)
+    if (!rc && p) rc = check_flat(w_dtype, dim, {p});
+  if (!rc && dim > 8192) return fail(TSATTN_ERR_UNSUPPORTED, "norm rows above 8192 elements are not supported");
+  return rc;
+}
+
 }  // namespace
 
 extern "C" {
@@ -598,6 +624,55 @@ int tsattn_qkv_rope_append(int32_t dtype, int32_t batch, int32_t len, int32_t em
                                                    v_scale ? &vs : nullptr, cos, sin, pos,
                                                    static_cast<hipStream_t>(stream)),
                     "fused projection launch");
+}
+
+int tsattn_norm_forward(int32_t dtype, int32_t w_dtype, int64_t rows, int32_t dim, int32_t rms,
+                        const void *x, const void *w, const void *bias, void *out, float *mean,
+                        float *rstd, double eps, void *stream) {
+  int rc = check_norm(dtype, w_dtype, rows, dim, {x, w, out}, {bias});
+  if (rc) return rc;
+  if (!(eps > 0.0)) return fail(TSATTN_ERR_INVALID, "eps must be positive");
+  if (rstd && !rms && !mean) return fail(TSATTN_ERR_INVALID, "layer norm saves its mean beside rstd");
+  return hip_status(tsattn::launch_norm_forward(dtype, w_dtype, rows, dim, rms != 0, x, w, bias, out,
+                                                mean, rstd, eps, static_cast<hipStream_t>(stream)),
+                    "norm launch");
+}
+
+size_t tsattn_norm_backward_workspace(int64_t rows, int32_t dim, int32_t rms) {
+  return rows > 0 && dim > 0 ? tsattn::norm_workspace_bytes(rows, dim, rms != 0) : 0;
+}
+
+int tsattn_norm_backward(int32_t dtype, int32_t w_dtype, int64_t rows, int32_t dim, int32_t rms,
+                         const void *x, const void *w, const void *g, const float *mean,
+                         const float *rstd, void *dx, void *dw, void *db, void *workspace,
+                         size_t workspace_bytes, void *stream) {
+  int rc = check_norm(dtype, w_dtype, rows, dim, {x, w, g, dx, dw, workspace}, {db});
+  if (rc) return rc;
+  if (!rstd || (!rms && !mean)) return fail(TSATTN_ERR_INVALID, "norm backward needs the saved statistics");
+  const size_t need = tsattn::norm_workspace_bytes(rows, dim, rms != 0);
+  if (workspace_bytes < need)
+    return fail(TSATTN_ERR_INVALID, "norm workspace too small: %zu < %zu bytes", workspace_bytes, need);
+  return hip_status(tsattn::launch_norm_backward(dtype, w_dtype, rows, dim, rms != 0, x, w, g, mean, rstd,
+                                                 dx, dw, rms ? nullptr : db, static_cast<float *>(workspace),
+                                                 static_cast<hipStream_t>(stream)),
+                    "norm backward launch");
+}
+
+int tsattn_silu_mul(int32_t dtype, int64_t n, const void *gate, const void *up, void *out, void *stream) {
+  int rc = check_flat(dtype, n, {gate, up, out});
+  if (rc) return rc;
+  return hip_status(tsattn::launch_silu_mul(dtype, n, gate, up, nullptr, out, nullptr,
+                                            static_cast<hipStream_t>(stream)),
+                    "SwiGLU launch");
+}
+
+int tsattn_silu_mul_backward(int32_t dtype, int64_t n, const void *gate, const void *up, const void *g,
+                             void *dgate, void *dup, void *stream) {
+  int rc = check_flat(dtype, n, {gate, up, g, dgate, dup});
+  if (rc) return rc;
+  return hip_status(tsattn::launch_silu_mul(dtype, n, gate, up, g, dgate, dup,
+                                            static_cast<hipStream_t>(stream)),
+                    "SwiGLU backward launch");
 }
 
 int tsattn_key_mask_lengths(const uint8_t *mask, int64_t stride_b, int64_t stride_k,

@@ -259,6 +259,22 @@ inline size_t dropout_bits_bytes(const Problem &p) {
          sizeof(uint32_t);
 }
 
+// Layer (rms = false) or RMS norm of `rows` contiguous rows of `dim` elements
+// (a multiple of 8, at most 8192; 16-byte aligned), statistics in fp32; mean /
+// rstd [rows] saved for the VJP when given.  The VJP's workspace holds the
+// partial weight (and bias) gradients.
+hipError_t launch_norm_forward(int dtype, int w_dtype, int64_t rows, int dim, bool rms, const void *x,
+                               const void *w, const void *bias, void *out, float *mean, float *rstd,
+                               double eps, hipStream_t st);
+size_t norm_workspace_bytes(int64_t rows, int dim, bool rms);
+hipError_t launch_norm_backward(int dtype, int w_dtype, int64_t rows, int dim, bool rms, const void *x,
+                                const void *w, const void *g, const float *mean, const float *rstd,
+                                void *dx, void *dw, void *db, float *ws, hipStream_t st);
+// out = silu(gate) * up over n elements (a multiple of 8), or with g its VJP:
+// out = d gate, dup = d up.
+hipError_t launch_silu_mul(int dtype, int64_t n, const void *gate, const void *up, const void *g,
+                           void *out, void *dup, hipStream_t st);
+
 hipError_t launch_key_mask_lengths(const uint8_t *mask, int64_t sb, int64_t sk, int B, int K,
                                    int32_t *kv_len, int32_t *kv_prefix, hipStream_t st);
 

@@ -130,6 +130,21 @@ SIGNATURES = {
          c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, _PV, _PV, _PV, _PV, _PV, c_void_p,
          c_void_p, c_int64, c_void_p],
     ),
+    "tsattn_norm_forward": (
+        c_int,
+        [c_int32, c_int32, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p,
+         c_void_p, c_void_p, c_double, c_void_p],
+    ),
+    "tsattn_norm_backward_workspace": (c_size_t, [c_int64, c_int32, c_int32]),
+    "tsattn_norm_backward": (
+        c_int,
+        [c_int32, c_int32, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p,
+         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p],
+    ),
+    "tsattn_silu_mul": (
+        c_int, [c_int32, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "tsattn_silu_mul_backward": (
+        c_int, [c_int32, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "tsattn_key_mask_lengths": (
         c_int,
         [c_void_p, c_int64, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_void_p],

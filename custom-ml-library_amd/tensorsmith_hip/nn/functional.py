@@ -1,18 +1,22 @@
 """Tape ops around the attention path, on hip tensors.
 
 Each op is one autograd node with the reference's semantics
-(``src/tensorsmith/nn/functional.py`` and ``nn/primitives.py``); the array
-math runs as PyTorch-ROCm library calls on the device tensors (GEMMs in
-hipBLASLt).  Only attention itself has hand-written HIP kernels.
+(``src/tensorsmith/nn/functional.py`` and ``nn/primitives.py``).  The norms and
+the SwiGLU activation run as one HIP kernel a pass (``csrc/layers.hip``) where
+their operands allow; the rest of the array math, and operands outside those
+kernels, as PyTorch-ROCm library calls on the device tensors (GEMMs in
+hipBLASLt).
 """
 
 from __future__ import annotations
 
+import ctypes
 import math
 
+from .. import _lib
 from ..amp import _cast_inputs
-from ..device import random_uniform
-from ..tensor import Tensor, _sum_to_shape, is_torch
+from ..device import current_stream, random_uniform
+from ..tensor import Tensor, _sum_to_shape, is_grad_enabled, is_torch
 from .attention import rotary_embedding, scaled_dot_product_attention
 
 __all__ = [
@@ -24,6 +28,23 @@ __all__ = [
 def _require_hip(t: Tensor, op: str):
     if not is_torch(t._data):
         raise RuntimeError(f"{op}: tensorsmith_hip computes on hip devices only")
+
+
+def _code(raw) -> int:
+    """The C ABI's code of a dtype the layer kernels take, or -1."""
+    import torch
+
+    return {torch.float32: _lib.F32, torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}.get(raw.dtype, -1)
+
+
+def _flat(raw):
+    """``raw`` as the layer kernels read it: contiguous, 16-byte aligned."""
+    raw = raw.contiguous()
+    return raw if raw.data_ptr() % 16 == 0 else raw.clone()
+
+
+def _ptr(raw):
+    return None if raw is None else ctypes.c_void_p(raw.data_ptr())
 
 
 def _compute(raw):
@@ -92,6 +113,10 @@ def _norm(input: Tensor, weight: Tensor, bias: Tensor | None, eps: float, rms: b
     if any(p.device != input.device for p in parents):
         raise ValueError("normalization tensors must be on the same device")
     _require_hip(input, "rms_norm" if rms else "layer_norm")
+    dim = math.prod(weight.shape)
+    if (_code(input._data) >= 0 and _code(weight._data) >= 0 and 0 < dim <= 8192 and dim % 8 == 0
+            and input.size > 0 and (bias is None or bias.dtype == weight.dtype)):
+        return _norm_kernel(input, weight, bias, eps, rms, dim, parents)
     axes = tuple(range(input.ndim - weight.ndim, input.ndim))
     x = _compute(input._data)
     w = weight._data.to(x.dtype)
@@ -113,6 +138,40 @@ def _norm(input: Tensor, weight: Tensor, bias: Tensor | None, eps: float, rms: b
         if bias is not None:
             grads.append(_sum_to_shape(g, bias.shape).to(bias.dtype))
         return tuple(grads)
+
+    return Tensor._from_op(out, parents, backward, "rms_norm" if rms else "layer_norm")
+
+
+def _norm_kernel(input, weight, bias, eps, rms, dim, parents) -> Tensor:
+    """``_norm`` in one kernel, and its VJP (``tsattn_norm_forward`` / ``_backward``)."""
+    import torch
+
+    lib = _lib.load()
+    x, w = _flat(input._data), _flat(weight._data)
+    b = None if bias is None else _flat(bias._data)
+    code, w_code, rows = _code(x), _code(w), x.numel() // dim
+    out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+    mean = rstd = None
+    if is_grad_enabled() and any(p.requires_grad for p in parents):
+        rstd = torch.empty(rows, dtype=torch.float32, device=x.device)
+        mean = None if rms else torch.empty(rows, dtype=torch.float32, device=x.device)
+    _lib.check(lib.tsattn_norm_forward(code, w_code, rows, dim, rms, _ptr(x), _ptr(w), _ptr(b),
+                                       _ptr(out), _ptr(mean), _ptr(rstd), eps,
+                                       ctypes.c_void_p(current_stream(input.device))), "norm")
+
+    def backward(g):
+        g = _flat(g.to(x.dtype))
+        dx = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+        dw = torch.empty(w.shape, dtype=w.dtype, device=x.device)
+        db = None if b is None else torch.empty(b.shape, dtype=b.dtype, device=x.device)
+        nbytes = lib.tsattn_norm_backward_workspace(rows, dim, rms)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+        _lib.check(lib.tsattn_norm_backward(code, w_code, rows, dim, rms, _ptr(x), _ptr(w), _ptr(g),
+                                            _ptr(mean), _ptr(rstd), _ptr(dx), _ptr(dw), _ptr(db),
+                                            _ptr(ws), nbytes,
+                                            ctypes.c_void_p(current_stream(input.device))),
+                   "norm backward")
+        return (dx, dw) if b is None else (dx, dw, db)
 
     return Tensor._from_op(out, parents, backward, "rms_norm" if rms else "layer_norm")
 
@@ -140,6 +199,34 @@ def silu(input: Tensor) -> Tensor:
         return ((g.to(x.dtype) * (sig + x * sig * (1 - sig))).to(input.dtype),)
 
     return Tensor._from_op(out, (input,), backward, "silu")
+
+
+def _silu_mul(gate: Tensor, up: Tensor) -> Tensor:
+    """``silu(gate) * up``, the SwiGLU activation (reference
+    ``transformer.py:190-205``): one kernel forward and one backward, rounding
+    where the two ops would."""
+    a, b = gate._data, up._data
+    if (not is_torch(a) or not is_torch(b) or a.dtype != b.dtype or a.shape != b.shape
+            or gate.device != up.device or _code(a) < 0 or a.numel() == 0 or a.numel() % 8):
+        return silu(gate) * up
+    import torch
+
+    lib, code = _lib.load(), _code(a)
+    a, b = _flat(a), _flat(b)
+    out = torch.empty(a.shape, dtype=a.dtype, device=a.device)
+    _lib.check(lib.tsattn_silu_mul(code, a.numel(), _ptr(a), _ptr(b), _ptr(out),
+                                   ctypes.c_void_p(current_stream(gate.device))), "SwiGLU")
+
+    def backward(g):
+        g = _flat(g.to(a.dtype))
+        da, db = torch.empty_like(a), torch.empty_like(b)
+        _lib.check(lib.tsattn_silu_mul_backward(code, a.numel(), _ptr(a), _ptr(b), _ptr(g), _ptr(da),
+                                                _ptr(db),
+                                                ctypes.c_void_p(current_stream(gate.device))),
+                   "SwiGLU backward")
+        return da, db
+
+    return Tensor._from_op(out, (gate, up), backward, "silu_mul")
 
 
 def embedding(indices: Tensor, weight: Tensor) -> Tensor:

@@ -178,7 +178,7 @@ class SwiGLU(Module):
         self.dropout = Dropout(dropout)
 
     def forward(self, input: Tensor) -> Tensor:
-        return self.dropout(self.down(F.silu(self.gate(input)) * self.up(input)))
+        return self.dropout(self.down(F._silu_mul(self.gate(input), self.up(input))))
 
 
 class TransformerDecoderBlock(Module):

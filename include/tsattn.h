@@ -390,6 +390,44 @@ int tsattn_qkv_rope_append(int32_t dtype, int32_t batch, int32_t len, int32_t em
                            void *stream);
 
 /*
+ * Layer norm (rms = 0) or RMS norm (rms != 0) of `rows` rows of `dim`
+ * contiguous elements (src/tensorsmith/nn/primitives.py:67-136): out = n w (+
+ * bias), n = (x - mean) / sqrt(var + eps) or x / sqrt(mean(x^2) + eps), in
+ * fp32 and rounded to dtype once.  dtype / w_dtype (of w and bias): f32, f16
+ * or bf16; dim a multiple of 8 up to 8192, every array contiguous and 16-byte
+ * aligned (others: TSATTN_ERR_UNSUPPORTED).  bias may be NULL.  rstd (and with
+ * rms = 0 mean): fp32 [rows] kept for the VJP, or NULL.
+ */
+int tsattn_norm_forward(int32_t dtype, int32_t w_dtype, int64_t rows, int32_t dim, int32_t rms,
+                        const void *x, const void *w, const void *bias, void *out, float *mean,
+                        float *rstd, double eps, void *stream);
+
+/* Bytes of scratch tsattn_norm_backward needs (partial weight gradients). */
+size_t tsattn_norm_backward_workspace(int64_t rows, int32_t dim, int32_t rms);
+
+/*
+ * Its VJP from the saved statistics (primitives.py:100-131): dx in dtype, dw
+ * (and with rms = 0 and db non-NULL, db) in w_dtype.  Deterministic: partial
+ * sums add up in a fixed order.
+ */
+int tsattn_norm_backward(int32_t dtype, int32_t w_dtype, int64_t rows, int32_t dim, int32_t rms,
+                         const void *x, const void *w, const void *g, const float *mean,
+                         const float *rstd, void *dx, void *dw, void *db, void *workspace,
+                         size_t workspace_bytes, void *stream);
+
+/*
+ * The SwiGLU activation over n contiguous elements (src/tensorsmith/nn/
+ * transformer.py:190-205): out = silu(gate) * up, silu (primitives.py:52-64)
+ * rounded to dtype before the product.  n a multiple of 8, 16-byte aligned
+ * arrays (others: TSATTN_ERR_UNSUPPORTED).
+ */
+int tsattn_silu_mul(int32_t dtype, int64_t n, const void *gate, const void *up, void *out, void *stream);
+
+/* Its VJP for the upstream gradient g: dgate and dup. */
+int tsattn_silu_mul_backward(int32_t dtype, int64_t n, const void *gate, const void *up, const void *g,
+                             void *dgate, void *dup, void *stream);
+
+/*
  * Boolean key mask [B, K] (strides in bytes-as-elements) -> kv_len[b] = 1 +
  * last allowed key (0 if none) and kv_prefix[b] = 1 iff the allowed keys are
  * exactly [0, kv_len[b]).  Serves the reference's key-padding masks
