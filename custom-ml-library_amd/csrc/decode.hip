@@ -26,7 +26,7 @@
 #include <mutex>
 #include <type_traits>
 
-#include "mfma_common.h"
+#include "decode_internal.h"
 #include "rope_math.h"
 
 namespace tsattn {
@@ -35,25 +35,6 @@ namespace {
 constexpr int NT = 256;
 constexpr int kU = 4;  // key instructions in flight per batch (per operand, 16-byte loads)
 constexpr int kMaxRows = 8;
-
-struct DecArgs {
-  Problem p;
-  View q, k, v, o;
-  View ks, vs;  // int8 caches: fp32 row scales [B, Hkv, capacity, 1]
-  float *ws;
-  int split_len, max_splits, rows;  // rows = rep * Sq query rows per KV head
-  float sl;                         // scale * log2(e)
-};
-
-// Keys any row may attend to: [0, eff_end).
-__device__ __forceinline__ int eff_end(const Problem &p, int b) {
-  int e = kv_end_for(p, b);
-  if (p.causal) {
-    const int64_t lim = static_cast<int64_t>(p.Sq) - 1 + p.offset + 1;
-    if (lim < e) e = static_cast<int>(lim < 0 ? 0 : lim);
-  }
-  return e;
-}
 
 __device__ __forceinline__ void merge_state(float &m, float &l, float *acc, float m2, float l2,
                                             const float *acc2) {
@@ -425,7 +406,9 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(DecArgs a) {
 template <typename T, int D, int R, bool Q8>
 hipError_t launch_rows(const DecArgs &a, hipStream_t st) {
   const Problem &p = a.p;
-  {
+  if (a.mfma) {
+    launch_decode_mfma(a, std::is_same_v<T, bf16> ? TSATTN_BF16 : TSATTN_F16, Q8, st);
+  } else {
     Probe pr_(Q8 ? "decode_split_int8" : "decode_split", st);
     decode_split_kernel<T, D, R, Q8><<<dim3(a.max_splits, p.Hkv, p.B), dim3(NT), 0, st>>>(a);
   }
@@ -472,6 +455,26 @@ int choose_split(const Problem &p, int split_len) {
   int s = 640;
   while (s > 80 && static_cast<int64_t>(p.B) * p.Hkv * ((p.Sk + s - 1) / s) < 4096) s >>= 1;
   return s;
+}
+
+// The split kernel and the length of its splits.  The matrix-core kernel has
+// a longer prologue and merge per workgroup and needs fewer workgroups: its
+// splits halve only until the grid has one per CU (never shorter than the
+// others', which the workspace is sized for).  Split + merge times: B64 Hkv8
+// 1025 keys 640 (1024 workgroups) 56 us, 160 67 us, 80 100 us; B1 Hkv8 16000
+// keys 640 (200) 28, 320 (400) 27, 160 (800) 35, 80 49 us.
+void choose_kernel(DecArgs &a, int dtype, bool q8, int split_len) {
+  const Problem &p = a.p;
+  a.split_len = split_len > 0 ? split_len : 640;
+  a.mfma = decode_mfma_applies(a, dtype, q8);
+  if (!a.mfma) {
+    a.split_len = choose_split(p, split_len);
+  } else if (split_len <= 0) {
+    while (a.split_len > 80 &&
+           static_cast<int64_t>(p.B) * p.Hkv * ((p.Sk + a.split_len - 1) / a.split_len) < 256)
+      a.split_len >>= 1;
+  }
+  a.max_splits = (p.Sk + a.split_len - 1) / a.split_len;
 }
 
 }  // namespace
@@ -528,18 +531,16 @@ hipError_t decode_scratch(void **ptr) {
 hipError_t launch_decode(const Problem &p, int dtype, View q, View k, View v, View o,
                          int split_len, void *workspace, hipStream_t st) {
   DecArgs a{p, q, k, v, o, View{}, View{}, static_cast<float *>(workspace), 0, 0, p.rep * p.Sq,
-            static_cast<float>(p.scale) * kLog2e};
-  a.split_len = choose_split(p, split_len);
-  a.max_splits = (p.Sk + a.split_len - 1) / a.split_len;
+            static_cast<float>(p.scale) * kLog2e, false};
+  choose_kernel(a, dtype, false, split_len);
   return launch_any<false>(a, dtype, st);
 }
 
 hipError_t launch_decode_int8(const Problem &p, int dtype, View q, View k, View v, View ks,
                               View vs, View o, int split_len, void *workspace, hipStream_t st) {
   DecArgs a{p, q, k, v, o, ks, vs, static_cast<float *>(workspace), 0, 0, p.rep * p.Sq,
-            static_cast<float>(p.scale) * kLog2e};
-  a.split_len = choose_split(p, split_len);
-  a.max_splits = (p.Sk + a.split_len - 1) / a.split_len;
+            static_cast<float>(p.scale) * kLog2e, false};
+  choose_kernel(a, dtype, true, split_len);
   return launch_any<true>(a, dtype, st);
 }
 

@@ -1,0 +1,114 @@
+"""The matrix-core decode split kernel (2 .. 8 query rows per KV head) against
+attention in float64.
+
+Sizes at the edges of its work split: a cache that ends one key before, at and
+after a 32-key tile and a wave's second tile, splits shorter than one tile per
+wave, every row count the routing sends here, caches whose rows are not
+contiguous ([B,S,H,D] memory), general and key-padding masks, an empty row.
+The bound is the rounding of the result to its dtype: the probabilities enter
+the value product with 22 (f16) or 24 (bf16) bits and the sums are fp32, so
+2e-6 of the row's largest value on top of half an ulp.
+"""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+if not torch.cuda.is_available():  # pragma: no cover - CPU containers
+    pytest.skip("no GPU", allow_module_level=True)
+
+import abi  # noqa: E402
+from tensorsmith_hip import _lib  # noqa: E402
+
+ULP = {torch.float16: 2.0**-11, torch.bfloat16: 2.0**-8}
+
+CASES = [
+    # (B, Hkv, rep, Sq, keys, D, dtype, split, layout, mask)
+    (2, 2, 2, 1, 31, 64, torch.float16, 0, "bhsd", None),
+    (1, 3, 4, 1, 33, 128, torch.bfloat16, 0, "bhsd", None),
+    (3, 2, 8, 1, 641, 128, torch.float16, 0, "bhsd", None),
+    (2, 2, 1, 5, 200, 128, torch.bfloat16, 40, "bhsd", None),
+    (2, 1, 3, 2, 257, 64, torch.bfloat16, 96, "bshd", None),
+    (1, 2, 7, 1, 320, 256, torch.float16, 0, "bhsd", None),
+    (2, 2, 2, 3, 130, 256, torch.bfloat16, 33, "bshd", None),
+    (3, 2, 4, 1, 300, 128, torch.float16, 0, "bhsd", "lengths"),
+    (2, 2, 4, 1, 300, 64, torch.bfloat16, 64, "bhsd", "bool"),
+    (2, 2, 2, 2, 190, 128, torch.float16, 0, "bhsd", "additive"),
+]
+
+
+def _reference(q, k, v, causal_off, mask):
+    rep = q.shape[1] // k.shape[1]
+    k, v = (t.double().repeat_interleave(rep, dim=1) for t in (k, v))
+    x = q.double() @ k.transpose(-1, -2).contiguous() / math.sqrt(q.shape[-1])
+    n, sq = k.shape[2], q.shape[2]
+    seen = torch.arange(n, device=q.device)[None, :] <= torch.arange(sq, device=q.device)[:, None] + causal_off
+    x = x.masked_fill(~seen, -math.inf)
+    if mask is not None:
+        x = x.masked_fill(~mask, -math.inf) if mask.dtype == torch.bool else x + mask.double()
+    p = torch.exp(x - x.amax(-1, keepdim=True).clamp_min(-1e300))
+    return (p @ v) / p.sum(-1, keepdim=True).clamp_min(1e-300)
+
+
+def _check(got, want, dtype):
+    scale = want.abs().amax(-1, keepdim=True).clamp_min(1e-30)
+    err = (got.double() - want).abs() - ULP[dtype] * want.abs()
+    assert (err / scale).max().item() <= 4e-6, (err / scale).max().item()
+
+
+def _caches(gen, b, h, n, d, layout):
+    out = []
+    for _ in range(2):
+        t = torch.randn((b, n + 7, h, d) if layout == "bshd" else (b, h, n + 7, d), generator=gen, device="cuda")
+        out.append(t.transpose(1, 2) if layout == "bshd" else t)
+    return out
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(x).split(".")[-1] for x in c))
+def test_decode_rows_match_float64(case):
+    b, hkv, rep, sq, n, d, dt, split, layout, mkind = case
+    print("decode rows", case, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(n + d)
+    q = torch.randn(b, hkv * rep, sq, d, generator=gen, device="cuda").to(dt)
+    k, v = (t.to(dt)[:, :, :n] for t in _caches(gen, b, hkv, n, d, layout))
+    kw, mask = dict(causal=True, offset=n - sq), None
+    if mkind == "lengths":
+        lens = torch.tensor([n, 0, n - 37][:b], dtype=torch.int32, device="cuda")
+        kw["kv_len"] = lens
+        mask = (torch.arange(n, device="cuda")[None] < lens[:, None])[:, None, None]
+    elif mkind == "bool":
+        mask = torch.rand(b, hkv * rep, 1, n, generator=gen, device="cuda") > 0.4
+        mask[0, 1] = False  # a row that sees nothing
+        kw["mask"] = mask
+    elif mkind == "additive":
+        mask = torch.randn(b, 1, sq, n, generator=gen, device="cuda")
+        mask[..., 32:96] = -math.inf
+        kw["mask"] = mask
+    got = abi.decode(q, k, v, split_len=split, **kw)
+    assert _lib.last_kernel_path() == _lib.PATH_DECODE
+    _check(got, _reference(q, k, v, n - sq, mask), dt)
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,rep,d,split", [(33, 2, 64, 0), (129, 4, 128, 0), (645, 8, 128, 0), (700, 3, 64, 96),
+                                           (130, 4, 256, 0)])
+def test_int8_decode_rows_match_float64(n, rep, d, split, dt):
+    """The codes are exact in the 16-bit tiles and the row scales enter in fp32;
+    one key's scale is far from the others'."""
+    print("int8 decode rows", n, rep, d, dt, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    b, hkv = 2, 2
+    q = torch.randn(b, hkv * rep, 1, d, generator=gen, device="cuda").to(dt)
+    k8, v8 = (torch.randint(-127, 128, (b, hkv, n + 5, d), generator=gen, device="cuda", dtype=torch.int8)
+              for _ in range(2))
+    ks, vs = (torch.rand(b, hkv, n + 5, 1, generator=gen, device="cuda") * 0.02 + 1e-4 for _ in range(2))
+    vs[:, :, 7] = 30.0
+    out, path = abi.decode_int8(q, k8, v8, ks, vs, n, split_len=split, causal=True, offset=n - 1)
+    assert path == _lib.PATH_DECODE
+    k, v = ((c.double() * s.double())[:, :, :n] for c, s in ((k8, ks), (v8, vs)))
+    _check(out, _reference(q, k, v, n - 1, None), dt)
