@@ -378,6 +378,173 @@ int check_norm(int32_t dtype, int32_t w_dtype, int64_t rows, int32_t dim,
   return rc;
 }
 
+// Operands of the few-row linear kernels.
+int check_rows(int32_t dtype, int32_t rows, int32_t k, int32_t n, int64_t xs, int64_t os,
+               std::initializer_list<const void *> arrays, std::initializer_list<const void *> optional) {
+  if (dtype != TSATTN_F16 && dtype != TSATTN_BF16)
+    return fail(TSATTN_ERR_INVALID, "few-row linear layers take dtype f16 or bf16 (got dtype %d)", dtype);
+  if (rows <= 0 || k <= 0 || n <= 0) return fail(TSATTN_ERR_INVALID, "linear layers need positive sizes");
+  for (const void *p : arrays)
+    if (!p) return fail(TSATTN_ERR_INVALID, "data pointer is NULL");
+  uintptr_t al = 0;
+  for (const void *p : arrays) al |= reinterpret_cast<uintptr_t>(p);
+  for (const void *p : optional) al |= reinterpret_cast<uintptr_t>(p);
+  if (rows > 64 || k % 8 || n % 4 || xs % 8 || os % 4 || xs < 0 || os < 0 || al % 16 ||
+      (static_cast<int64_t>(rows) * xs + k) * 2 >= (int64_t(1) << 31) ||
+      static_cast<int64_t>(k) * 64 >= (int64_t(1) << 31))
+    return fail(TSATTN_ERR_UNSUPPORTED,
+                "few-row linear layers take up to 64 rows, k %% 8 == 0, n %% 4 == 0 and 16-byte aligned arrays");
+  return TSATTN_OK;
+}
+
+// A cached step: the workspace's layout and the attention problem.
+struct StepPlan {
+  int rows, width;  // batch len, heads_q dim
+  bool q8;
+  tsattn::Problem pr;
+  size_t normed, q, attn, hidden, act, split, bytes;  // offsets, then the total
+};
+
+int plan_step(const tsattn_step_desc *d, StepPlan *out) {
+  if (!d) return fail(TSATTN_ERR_INVALID, "step descriptor is NULL");
+  if (d->dtype != TSATTN_F16 && d->dtype != TSATTN_BF16)
+    return fail(TSATTN_ERR_INVALID, "the cached step takes dtype f16 or bf16 (got dtype %d)", d->dtype);
+  if (d->batch <= 0 || d->len <= 0 || d->embed <= 0 || d->heads_q <= 0 || d->heads_kv <= 0 || d->pos < 0 ||
+      (d->norm2 && d->hidden <= 0))
+    return fail(TSATTN_ERR_INVALID, "the cached step needs positive sizes and a nonnegative position");
+  if (d->heads_q % d->heads_kv) return fail(TSATTN_ERR_INVALID, "query heads must divide into KV groups");
+  if (!d->x || !d->out || !d->wq || !d->wk || !d->wv || !d->wo || !d->k_cache.data || !d->v_cache.data ||
+      (d->norm2 && (!d->gate || !d->up || !d->down)))
+    return fail(TSATTN_ERR_INVALID, "data pointer is NULL");
+  if (!d->cos != !d->sin) return fail(TSATTN_ERR_INVALID, "RoPE needs both cos and sin tables");
+  if (!d->k_scale.data != !d->v_scale.data)
+    return fail(TSATTN_ERR_INVALID, "an int8 cache needs both key and value scales");
+  int rc;
+  if ((rc = check_view(&d->k_cache, "key cache")) || (rc = check_view(&d->v_cache, "value cache")) ||
+      (d->k_scale.data &&
+       ((rc = check_view(&d->k_scale, "key scales")) || (rc = check_view(&d->v_scale, "value scales")))))
+    return rc;
+  const int64_t rows = static_cast<int64_t>(d->batch) * d->len, width = static_cast<int64_t>(d->heads_q) * d->dim;
+  uintptr_t al = 0;
+  for (const void *p : {d->x, d->norm1, d->wq, d->wk, d->wv, d->wo, d->bq, d->bk, d->bv, d->bo, d->norm2, d->gate,
+                        d->up, d->down, d->cos, d->sin, static_cast<const void *>(d->out)})
+    al |= reinterpret_cast<uintptr_t>(p);
+  if (rows > 64 || d->heads_q / d->heads_kv * static_cast<int64_t>(d->len) > 8 || (d->dim != 64 && d->dim != 128) ||
+      d->embed % 16 || d->embed > 8192 || width > 65536 || d->hidden > (1 << 20) ||
+      (d->norm2 && d->hidden % 8) || al % 16 || d->pos + d->len > INT32_MAX / 2)
+    return fail(TSATTN_ERR_UNSUPPORTED,
+                "the cached step takes up to 64 rows, 8 query rows per KV head, head dims 64 and 128, embed %% 16 == "
+                "0 and 16-byte aligned arrays");
+  StepPlan s{};
+  s.rows = static_cast<int>(rows);
+  s.width = static_cast<int>(width);
+  s.q8 = d->k_scale.data != nullptr;
+  const tsattn::View vk = tsattn::make_view(&d->k_cache), vv = tsattn::make_view(&d->v_cache);
+  auto rows_ok = [&](const tsattn::View &v) {
+    return s.q8 ? reinterpret_cast<uintptr_t>(v.data) % 8 == 0 && v.s0 % 8 == 0 && v.s1 % 8 == 0 && v.s2 % 8 == 0
+                : tsattn::aligned16(v);
+  };
+  if (!rows_ok(vk) || !rows_ok(vv)) return fail(TSATTN_ERR_UNSUPPORTED, "the cached step needs aligned cache rows");
+  tsattn::Problem &p = s.pr;
+  p.B = d->batch, p.Hq = d->heads_q, p.Hkv = d->heads_kv, p.Sq = d->len;
+  p.Sk = static_cast<int>(d->pos) + d->len;
+  p.Dqk = p.Dv = d->dim;
+  p.rep = d->heads_q / d->heads_kv;
+  p.scale = 1.0 / sqrt(static_cast<double>(d->dim));
+  p.causal = d->is_causal ? 1 : 0;
+  p.offset = d->pos;
+  if (s.q8 && d->cos) p.rope = tsattn::RopeDesc{d->cos, d->sin, d->dim, d->pos, 0, nullptr};
+  size_t at = 0;
+  auto take = [&](size_t n) {
+    const size_t o = at;
+    at = round256(at + n);
+    return o;
+  };
+  const size_t es = 2, re = static_cast<size_t>(rows) * d->embed * es;
+  const size_t qkv = static_cast<size_t>(rows) * (d->heads_q + (s.q8 ? 2 * d->heads_kv : 0)) * d->dim * es;
+  s.normed = take(d->norm1 || d->norm2 ? re : 0);
+  s.q = take(qkv);
+  s.attn = take(static_cast<size_t>(rows) * width * es);
+  s.hidden = take(d->norm2 ? re : 0);
+  s.act = take(d->norm2 ? static_cast<size_t>(rows) * d->hidden * es : 0);
+  s.split = take(tsattn::decode_workspace_bytes(p, 0));
+  s.bytes = at;
+  *out = s;
+  return TSATTN_OK;
+}
+
+int run_step(const tsattn_step_desc &d, const StepPlan &s, char *ws, hipStream_t st) {
+  const int rows = s.rows, E = d.embed, D = d.dim, L = d.len;
+  const int64_t W = s.width;
+  const void *none[3] = {nullptr, nullptr, nullptr};
+  const void *x = d.x;
+  int rc;
+  if (d.norm1) {
+    if ((rc = hip_status(tsattn::launch_norm_forward(d.dtype, d.dtype, rows, E, true, x, d.norm1, nullptr,
+                                                     ws + s.normed, nullptr, nullptr, d.eps1, st),
+                         "step norm launch")))
+      return rc;
+    x = ws + s.normed;
+  }
+  const tsattn::View vk = tsattn::make_view(&d.k_cache), vv = tsattn::make_view(&d.v_cache);
+  const tsattn::View vks = tsattn::make_view(&d.k_scale), vvs = tsattn::make_view(&d.v_scale);
+  const void *w[3] = {d.wq, d.wk, d.wv}, *bias[3] = {d.bq, d.bk, d.bv};
+  char *q = ws + s.q;
+  tsattn::View vq;
+  if (!s.q8) {
+    vq = tsattn::View{q, static_cast<int64_t>(L) * W, D, W};
+    rc = hip_status(tsattn::launch_qkv_rope_append(d.dtype, d.batch, L, E, d.heads_q, d.heads_kv, D,
+                                                   tsattn::View{x, static_cast<int64_t>(L) * E, 0, E}, w, bias, vq,
+                                                   vk, vv, nullptr, nullptr, d.cos, d.sin, d.pos, st),
+                    "step projection launch");
+    if (rc) return rc;
+  } else {
+    // int8 caches: the quantiser needs a whole row, which a 32-channel tile of
+    // the projection does not have: all rows first, then rotate and append
+    // (the decode kernel rotates the queries)
+    tsattn::Probe pr_("qkv_rope_append_int8", st);
+    const int kvw = d.heads_kv * D, n[3] = {static_cast<int>(W), kvw, kvw};
+    const int64_t N = W + 2 * kvw;
+    if ((rc = hip_status(tsattn::launch_rows_linear(d.dtype, rows, E, n, x, E, w, bias, nullptr, 0, q, N, st, false),
+                         "step projection launch")))
+      return rc;
+    vq = tsattn::View{q, L * N, D, N};
+    const tsattn::View nk{q + W * 2, L * N, D, N}, nv{q + (W + kvw) * 2, L * N, D, N};
+    rc = hip_status(tsattn::launch_rope_append(d.dtype, d.batch, d.heads_kv, L, D, d.cos ? D : 0, nk, nv, vk, vv,
+                                               &vks, &vvs, d.cos, d.sin, d.pos, st, false),
+                    "step append launch");
+    if (rc) return rc;
+  }
+  g_last_path = 3;
+  char *attn = ws + s.attn;
+  const tsattn::View vo{attn, static_cast<int64_t>(L) * W, D, W};
+  rc = s.q8 ? hip_status(tsattn::launch_decode_int8(s.pr, d.dtype, vq, vk, vv, vks, vvs, vo, 0, ws + s.split, st),
+                         "step int8 decode launch")
+            : hip_status(tsattn::launch_decode(s.pr, d.dtype, vq, vk, vv, vo, 0, ws + s.split, st),
+                         "step decode launch");
+  if (rc) return rc;
+  const bool block = d.norm1 || d.norm2;
+  void *h = d.norm2 ? ws + s.hidden : d.out;
+  const int ne[3] = {E, 0, 0};
+  const void *wo[3] = {d.wo, nullptr, nullptr}, *bo[3] = {d.bo, nullptr, nullptr};
+  if ((rc = hip_status(tsattn::launch_rows_linear(d.dtype, rows, static_cast<int>(W), ne, attn, W, wo, bo,
+                                                  block ? d.x : nullptr, E, h, E, st),
+                       "step output projection launch")) ||
+      !d.norm2)
+    return rc;
+  if ((rc = hip_status(tsattn::launch_norm_forward(d.dtype, d.dtype, rows, E, true, h, d.norm2, nullptr,
+                                                   ws + s.normed, nullptr, nullptr, d.eps2, st),
+                       "step norm launch")) ||
+      (rc = hip_status(tsattn::launch_rows_swiglu(d.dtype, rows, E, d.hidden, ws + s.normed, E, d.gate, d.up,
+                                                  ws + s.act, d.hidden, st),
+                       "step SwiGLU launch")))
+    return rc;
+  const void *wd[3] = {d.down, nullptr, nullptr};
+  return hip_status(tsattn::launch_rows_linear(d.dtype, rows, d.hidden, ne, ws + s.act, d.hidden, wd, none, h, E,
+                                               d.out, E, st),
+                    "step down projection launch");
+}
+
 }  // namespace
 
 extern "C" {
@@ -673,6 +840,45 @@ int tsattn_silu_mul_backward(int32_t dtype, int64_t n, const void *gate, const v
   return hip_status(tsattn::launch_silu_mul(dtype, n, gate, up, g, dgate, dup,
                                             static_cast<hipStream_t>(stream)),
                     "SwiGLU backward launch");
+}
+
+int tsattn_rows_linear(int32_t dtype, int32_t rows, int32_t k, int32_t n, const void *x, int64_t x_stride,
+                       const void *w, const void *bias, const void *residual, int64_t residual_stride,
+                       void *out, int64_t out_stride, void *stream) {
+  int rc = check_rows(dtype, rows, k, n, x_stride, out_stride, {x, w, out}, {bias, residual});
+  if (rc) return rc;
+  if (residual && (residual_stride % 4 || residual_stride < 0))
+    return fail(TSATTN_ERR_UNSUPPORTED, "residual rows need 4-element aligned strides");
+  const int ns[3] = {n, 0, 0};
+  const void *ws[3] = {w, nullptr, nullptr}, *bs[3] = {bias, nullptr, nullptr};
+  return hip_status(tsattn::launch_rows_linear(dtype, rows, k, ns, x, x_stride, ws, bs, residual,
+                                               residual_stride, out, out_stride,
+                                               static_cast<hipStream_t>(stream)),
+                    "rows linear launch");
+}
+
+int tsattn_rows_swiglu(int32_t dtype, int32_t rows, int32_t k, int32_t n, const void *x, int64_t x_stride,
+                       const void *gate, const void *up, void *out, int64_t out_stride, void *stream) {
+  int rc = check_rows(dtype, rows, k, n, x_stride, out_stride, {x, gate, up, out}, {});
+  if (rc) return rc;
+  return hip_status(tsattn::launch_rows_swiglu(dtype, rows, k, n, x, x_stride, gate, up, out, out_stride,
+                                               static_cast<hipStream_t>(stream)),
+                    "rows SwiGLU launch");
+}
+
+size_t tsattn_cached_step_workspace(const tsattn_step_desc *d) {
+  StepPlan s;
+  return plan_step(d, &s) ? 0 : s.bytes;
+}
+
+int tsattn_cached_step(const tsattn_step_desc *d, void *workspace, size_t workspace_bytes, void *stream) {
+  StepPlan s;
+  int rc = plan_step(d, &s);
+  if (rc) return rc;
+  if (!workspace || reinterpret_cast<uintptr_t>(workspace) % 256 || workspace_bytes < s.bytes)
+    return fail(TSATTN_ERR_INVALID, "step workspace too small or misaligned: %zu < %zu bytes", workspace_bytes,
+                s.bytes);
+  return run_step(*d, s, static_cast<char *>(workspace), static_cast<hipStream_t>(stream));
 }
 
 int tsattn_key_mask_lengths(const uint8_t *mask, int64_t stride_b, int64_t stride_k,

@@ -71,6 +71,46 @@ class RopeDesc(ctypes.Structure):
     ]
 
 
+class StepDesc(ctypes.Structure):
+    """``tsattn_step_desc``: one cached step of an attention layer or decoder block."""
+
+    _fields_ = [
+        ("dtype", c_int32),
+        ("batch", c_int32),
+        ("len", c_int32),
+        ("embed", c_int32),
+        ("heads_q", c_int32),
+        ("heads_kv", c_int32),
+        ("dim", c_int32),
+        ("hidden", c_int32),
+        ("is_causal", c_int32),
+        ("pos", c_int64),
+        ("eps1", c_double),
+        ("eps2", c_double),
+        ("x", c_void_p),
+        ("norm1", c_void_p),
+        ("wq", c_void_p),
+        ("wk", c_void_p),
+        ("wv", c_void_p),
+        ("wo", c_void_p),
+        ("bq", c_void_p),
+        ("bk", c_void_p),
+        ("bv", c_void_p),
+        ("bo", c_void_p),
+        ("norm2", c_void_p),
+        ("gate", c_void_p),
+        ("up", c_void_p),
+        ("down", c_void_p),
+        ("cos", c_void_p),
+        ("sin", c_void_p),
+        ("k_cache", View),
+        ("v_cache", View),
+        ("k_scale", View),
+        ("v_scale", View),
+        ("out", c_void_p),
+    ]
+
+
 _PV = POINTER(View)
 _PP = POINTER(Problem)
 _PR = POINTER(RopeDesc)
@@ -145,6 +185,18 @@ SIGNATURES = {
         c_int, [c_int32, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),
     "tsattn_silu_mul_backward": (
         c_int, [c_int32, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "tsattn_rows_linear": (
+        c_int,
+        [c_int32, c_int32, c_int32, c_int32, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64,
+         c_void_p, c_int64, c_void_p],
+    ),
+    "tsattn_rows_swiglu": (
+        c_int,
+        [c_int32, c_int32, c_int32, c_int32, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64,
+         c_void_p],
+    ),
+    "tsattn_cached_step_workspace": (c_size_t, [POINTER(StepDesc)]),
+    "tsattn_cached_step": (c_int, [POINTER(StepDesc), c_void_p, c_size_t, c_void_p]),
     "tsattn_key_mask_lengths": (
         c_int,
         [c_void_p, c_int64, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_void_p],

@@ -67,9 +67,11 @@ def linear(input: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
     _require_hip(input, "linear")
     w = weight._data
     x = input._data.reshape(-1, weight.shape[1])
-    out = x @ w.t()
-    if bias is not None:
-        out = out + bias._data.to(out.dtype)
+    out = _rows_linear(x, w, None if bias is None else bias._data, input.device)
+    if out is None:
+        out = x @ w.t()
+        if bias is not None:
+            out = out + bias._data.to(out.dtype)
     out = out.reshape(input.shape[:-1] + (weight.shape[0],))
 
     def backward(g):
@@ -80,6 +82,29 @@ def linear(input: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
         return tuple(grads)
 
     return Tensor._from_op(out, parents, backward, "linear")
+
+
+def _rows_linear(x, w, bias, dev):
+    """``x W^T (+ bias)`` of a few 16-bit rows in one kernel
+    (``tsattn_rows_linear``), or None outside it.  Over 32 rows each weight is
+    read by two row blocks, and wide layers are the library's (K 4096, 64 rows:
+    N 4096 13 us here and 12 there, N 16384 51 and 32)."""
+    import torch
+
+    rows, k = x.shape
+    n = w.shape[0]
+    if (x.dtype not in (torch.float16, torch.bfloat16) or w.dtype != x.dtype or not 0 < rows <= 64
+            or (rows > 32 and n > 8192) or k % 8 or n % 4 or k == 0 or n == 0 or x.stride(1) != 1
+            or x.stride(0) % 8 or not w.is_contiguous() or x.data_ptr() % 16 or w.data_ptr() % 16
+            or (bias is not None and (bias.dtype != x.dtype or not bias.is_contiguous()
+                                      or bias.data_ptr() % 16))):
+        return None
+    out = torch.empty((rows, n), dtype=x.dtype, device=x.device)
+    _lib.check(_lib.load().tsattn_rows_linear(
+        _code(x), rows, k, n, x.data_ptr(), x.stride(0), w.data_ptr(),
+        None if bias is None else bias.data_ptr(), None, 0, out.data_ptr(), n, current_stream(dev)),
+        "few-row linear")
+    return out
 
 
 def gelu(input: Tensor) -> Tensor:

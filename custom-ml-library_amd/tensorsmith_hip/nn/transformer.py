@@ -28,16 +28,115 @@ import numpy as np
 
 from dataclasses import dataclass
 
+from .. import _lib
 from .. import device as _device
+from ..device import current_stream
 from ..tensor import Tensor, cat, is_grad_enabled, no_grad
 from . import functional as F
-from .attention import BACKENDS, decode_int8_cache, rotary_embedding, scaled_dot_product_attention
+from .attention import (BACKENDS, DECODE_MIN_KEYS, _dtype_code, _view, decode_int8_cache, rope_tables,
+                        rotary_embedding, scaled_dot_product_attention)
 from .cache import KVCache
 from .checkpoint import checkpoint
 from .layers import Dropout, Embedding, Linear
 from .module import Module, Parameter
 
 random_uniform = _device.random_uniform
+_PROJECT_APPEND = KVCache._project_append
+
+
+def _plain(module, cls) -> bool:
+    """``module`` is a ``cls`` itself, its forward not replaced."""
+    return type(module) is cls and "forward" not in module.__dict__
+
+
+def _cached_step(x: Tensor, attention, cache, is_causal: bool = True, block=None):
+    """One inference step of ``attention`` over ``cache`` -- or of the decoder
+    ``block`` around it, norms, residuals and SwiGLU included -- in one library
+    call (``tsattn_cached_step``); the caller has validated ``x`` and the cache
+    mode.  Returns the raw result and advances ``cache.length``; or None,
+    writing nothing, where the call does not apply (many rows, fp32, a
+    replaced layer or cache method, a short cache): the layers then run one by
+    one.  Same values either way, rounded at the same places."""
+    import torch
+
+    raw = x._data
+    if (raw.dtype not in (torch.float16, torch.bfloat16) or type(cache) is not KVCache
+            or KVCache._project_append is not _PROJECT_APPEND or cache.dtype != raw.dtype
+            or cache.device != x.device or attention.backend == "native"):
+        return None
+    b, t, e = raw.shape
+    pos, stop = cache.length, cache.length + t
+    heads, kv_heads, dim = attention.num_heads, attention.num_kv_heads, attention.head_dim
+    if (stop > cache.max_seq_len or stop < DECODE_MIN_KEYS or b * t > 64 or (heads // kv_heads) * t > 8
+            or dim not in (64, 128) or b != cache.batch_size or kv_heads != cache.num_heads
+            or dim != cache.head_dim or dim != cache.value_dim or t == 0):
+        return None
+    linear = [attention.q_proj, attention.k_proj, attention.v_proj, attention.out_proj]
+    hidden, widest = 0, e
+    if block is not None:
+        ffn = block.ffn
+        mlp = [ffn.gate, ffn.up, ffn.down]
+        if (not all(_plain(m, Linear) and m.bias is None for m in mlp) or not _plain(ffn, SwiGLU)
+                or not _plain(attention, MultiHeadAttention) or not _plain(block.attention_norm, RMSNorm)
+                or not _plain(block.ffn_norm, RMSNorm)
+                or any(d.training and d.p for d in (block.residual_dropout, ffn.dropout))):
+            return None
+        hidden = ffn.gate.weight.shape[0]
+        widest = max(e, hidden)
+    # over 32 rows every weight is read by two row blocks: the library's products
+    # are the faster ones for wide layers (K 4096, N 16384, 64 rows: 32 us against 51)
+    if b * t > 32 and widest > 8192:
+        return None
+    if not all(_plain(m, Linear) for m in linear):
+        return None
+    desc = _lib.StepDesc()
+    keep = [raw] if raw.is_contiguous() else [raw.contiguous()]
+
+    def at(tensor, *shape):  # the pointer of a contiguous operand of the step's dtype, else 0
+        if tensor is None:
+            return None
+        data = tensor._data
+        if data.dtype != raw.dtype or not data.is_contiguous() or tuple(data.shape) != shape:
+            return 0
+        keep.append(data)
+        return data.data_ptr()
+
+    kv = kv_heads * dim
+    ptrs = {"wq": at(linear[0].weight, heads * dim, e), "wk": at(linear[1].weight, kv, e),
+            "wv": at(linear[2].weight, kv, e), "wo": at(linear[3].weight, e, heads * dim),
+            "bq": at(linear[0].bias, heads * dim), "bk": at(linear[1].bias, kv),
+            "bv": at(linear[2].bias, kv), "bo": at(linear[3].bias, e)}
+    if block is not None:
+        ptrs.update(norm1=at(block.attention_norm.weight, e), norm2=at(block.ffn_norm.weight, e),
+                    gate=at(ffn.gate.weight, hidden, e), up=at(ffn.up.weight, hidden, e),
+                    down=at(ffn.down.weight, e, hidden))
+        desc.eps1, desc.eps2 = block.attention_norm.eps, block.ffn_norm.eps
+    if 0 in ptrs.values():
+        return None
+    for name, value in ptrs.items():
+        setattr(desc, name, value)
+    desc.dtype = _dtype_code(raw.dtype)
+    desc.batch, desc.len, desc.embed = b, t, e
+    desc.heads_q, desc.heads_kv, desc.dim, desc.hidden = heads, kv_heads, dim, hidden
+    desc.is_causal, desc.pos = int(is_causal), pos
+    if attention.rotary:
+        tables = rope_tables(10000.0, dim, raw.dtype, raw.device, stop)
+        desc.cos, desc.sin = tables[0].data_ptr(), tables[1].data_ptr()
+    keys, values, key_scales, value_scales = cache.storage
+    desc.k_cache, desc.v_cache = _view(keys), _view(values)
+    if cache.quantized:
+        desc.k_scale, desc.v_scale = _view(key_scales), _view(value_scales)
+    out = torch.empty((b, t, e), dtype=raw.dtype, device=raw.device)
+    desc.x, desc.out = keep[0].data_ptr(), out.data_ptr()
+    lib = _lib.load()
+    nbytes = lib.tsattn_cached_step_workspace(desc)
+    if nbytes == 0:
+        return None
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=raw.device)
+    _lib.check(lib.tsattn_cached_step(desc, ws.data_ptr(), nbytes, current_stream(x.device)),
+               "cached step")
+    cache.length = stop
+    return out
 
 
 class MultiHeadAttention(Module):
@@ -94,6 +193,10 @@ class MultiHeadAttention(Module):
                     raise TypeError("attention masks must be boolean or floating point")
             except ValueError as error:
                 raise ValueError("attention mask is not broadcastable to [B,H,Q,K]") from error
+        if cache is not None and context is None and attn_mask is None:
+            stepped = _cached_step(input, self, cache, is_causal)
+            if stepped is not None:
+                return Tensor._from_op(stepped, (input,), None, "cached_step")
         # cached self-attention: projections, RoPE and the append in one kernel
         # where the operands allow (the queries come back rotated)
         q_fused = None
@@ -196,6 +299,12 @@ class TransformerDecoderBlock(Module):
         self.ffn = SwiGLU(dim, hidden_dim or 4 * dim, dropout, device)
 
     def forward(self, input: Tensor, *, cache=None, attn_mask=None) -> Tensor:
+        if (cache is not None and attn_mask is None and not is_grad_enabled()
+                and not self.attention.training and input.ndim == 3
+                and input.shape[-1] == self.attention.embed_dim):
+            stepped = _cached_step(input, self.attention, cache, block=self)
+            if stepped is not None:
+                return Tensor._from_op(stepped, (input,), None, "cached_step")
         hidden = input + self.residual_dropout(
             self.attention(self.attention_norm(input), cache=cache, attn_mask=attn_mask))
         return hidden + self.ffn(self.ffn_norm(hidden))

@@ -428,6 +428,60 @@ int tsattn_silu_mul_backward(int32_t dtype, int64_t n, const void *gate, const v
                              void *dgate, void *dup, void *stream);
 
 /*
+ * A linear layer over few rows (src/tensorsmith/nn/functional.py:63-90; the
+ * cached decode step): out[r][:] = x[r] W^T, rounded to dtype, (+ bias),
+ * (+ residual[r]), each sum rounded to dtype.  w: [n, k] row-major.  dtype f16
+ * or bf16, rows <= 64, k a multiple of 8 and n of 4, row strides (in elements)
+ * multiples of 8 for x and of 4 for residual and out, every array 16-byte
+ * aligned (others: TSATTN_ERR_UNSUPPORTED).  bias and residual may be NULL.
+ */
+int tsattn_rows_linear(int32_t dtype, int32_t rows, int32_t k, int32_t n, const void *x, int64_t x_stride,
+                       const void *w, const void *bias, const void *residual, int64_t residual_stride,
+                       void *out, int64_t out_stride, void *stream);
+
+/*
+ * silu(x gate^T) * (x up^T) over few rows, rounded where the separate layers
+ * round (src/tensorsmith/nn/transformer.py:190-205); gate, up: [n, k].  Limits
+ * as tsattn_rows_linear.
+ */
+int tsattn_rows_swiglu(int32_t dtype, int32_t rows, int32_t k, int32_t n, const void *x, int64_t x_stride,
+                       const void *gate, const void *up, void *out, int64_t out_stride, void *stream);
+
+/*
+ * One cached decode step of the attention layer, or of a whole pre-norm
+ * decoder block, as one call: MultiHeadAttention.forward with a cache
+ * (src/tensorsmith/nn/transformer.py:124-155) and TransformerDecoderBlock.forward
+ * (transformer.py:226-243).  Launches, in order: RMS norm (norm1 != NULL), the
+ * projections with RoPE and the cache append, the split decode attention, the
+ * output projection (+ x, when norm1 or norm2 is given), and with norm2 != NULL
+ * RMS norm, the SwiGLU pair and the down projection + the residual.  The
+ * results are those of the separate entry points on the same arrays.
+ */
+typedef struct tsattn_step_desc {
+  int32_t dtype; /* f16 or bf16: activations, weights, norms and 16-bit caches */
+  int32_t batch, len, embed, heads_q, heads_kv, dim, hidden; /* hidden: MLP width (norm2) */
+  int32_t is_causal;
+  int64_t pos;   /* cached positions before the step; the caches hold pos + len after it */
+  double eps1, eps2; /* of the two norms */
+  const void *x;     /* [batch, len, embed] contiguous, 16-byte aligned, like every array here */
+  const void *norm1; /* [embed] or NULL */
+  const void *wq, *wk, *wv, *wo, *bq, *bk, *bv, *bo; /* Linear.weight / bias (biases may be NULL) */
+  const void *norm2, *gate, *up, *down; /* norm2 NULL: no MLP */
+  const void *cos, *sin; /* RoPE tables, or NULL */
+  tsattn_view k_cache, v_cache, k_scale, v_scale; /* scales' data NULL: caches in dtype */
+  void *out; /* [batch, len, embed] contiguous */
+} tsattn_step_desc;
+
+/* Bytes of scratch tsattn_cached_step needs (0: a problem it does not take). */
+size_t tsattn_cached_step_workspace(const tsattn_step_desc *d);
+
+/*
+ * The step.  batch * len <= 64 rows, (heads_q / heads_kv) * len <= 8, dim 64 or
+ * 128, embed a multiple of 16 up to 8192 (others: TSATTN_ERR_UNSUPPORTED, nothing launched).
+ */
+int tsattn_cached_step(const tsattn_step_desc *d, void *workspace, size_t workspace_bytes, void *stream);
+
+/*
  * Boolean key mask [B, K] (strides in bytes-as-elements) -> kv_len[b] = 1 +
  * last allowed key (0 if none) and kv_prefix[b] = 1 iff the allowed keys are
  * exactly [0, kv_len[b]).  Serves the reference's key-padding masks
