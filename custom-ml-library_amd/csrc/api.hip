@@ -866,6 +866,32 @@ int tsattn_rows_swiglu(int32_t dtype, int32_t rows, int32_t k, int32_t n, const 
                     "rows SwiGLU launch");
 }
 
+size_t tsattn_linear_wgrad_workspace(int32_t tokens, int32_t m, int32_t n) {
+  return tokens > 0 && m > 0 && n > 0 ? tsattn::wgrad_workspace_bytes(tokens, m, n) : 0;
+}
+
+int tsattn_linear_wgrad(int32_t dtype, int32_t tokens, int32_t m, int32_t n, const void *g, int64_t g_stride,
+                        const void *x, int64_t x_stride, void *dw, void *workspace, size_t workspace_bytes,
+                        void *stream) {
+  if (dtype != TSATTN_F16 && dtype != TSATTN_BF16)
+    return fail(TSATTN_ERR_INVALID, "the weight gradient takes dtype f16 or bf16 (got dtype %d)", dtype);
+  if (tokens <= 0 || m <= 0 || n <= 0) return fail(TSATTN_ERR_INVALID, "linear layers need positive sizes");
+  if (!g || !x || !dw) return fail(TSATTN_ERR_INVALID, "data pointer is NULL");
+  const uintptr_t al = reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(x) |
+                       reinterpret_cast<uintptr_t>(dw) | reinterpret_cast<uintptr_t>(workspace);
+  if (m % 8 || n % 8 || g_stride % 8 || x_stride % 8 || g_stride < m || x_stride < n || al % 16 ||
+      static_cast<int64_t>(tokens) * (g_stride > x_stride ? g_stride : x_stride) * 2 >= (int64_t(1) << 31) ||
+      static_cast<int64_t>(m) * n >= (int64_t(1) << 31))
+    return fail(TSATTN_ERR_UNSUPPORTED,
+                "the weight gradient takes m and n %% 8 == 0, 16-byte aligned rows and operands below 2^31 bytes");
+  const size_t need = tsattn::wgrad_workspace_bytes(tokens, m, n);
+  if (!workspace || workspace_bytes < need)
+    return fail(TSATTN_ERR_INVALID, "weight gradient workspace too small: %zu < %zu bytes", workspace_bytes, need);
+  return hip_status(tsattn::launch_wgrad(dtype, tokens, m, n, g, g_stride, x, x_stride, dw,
+                                         static_cast<float *>(workspace), static_cast<hipStream_t>(stream)),
+                    "weight gradient launch");
+}
+
 size_t tsattn_cached_step_workspace(const tsattn_step_desc *d) {
   StepPlan s;
   return plan_step(d, &s) ? 0 : s.bytes;

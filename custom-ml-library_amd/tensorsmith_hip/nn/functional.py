@@ -76,12 +76,40 @@ def linear(input: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
 
     def backward(g):
         flat = g.reshape(-1, weight.shape[0])
-        grads = [(flat @ w).reshape(input.shape).to(input.dtype), (flat.t() @ x).to(weight.dtype)]
+        grads = [(flat @ w).reshape(input.shape).to(input.dtype),
+                 _weight_grad(flat, x, input.device).to(weight.dtype)]
         if bias is not None:
             grads.append(flat.sum(0).to(bias.dtype))
         return tuple(grads)
 
     return Tensor._from_op(out, parents, backward, "linear")
+
+
+def _weight_grad(g, x, dev):
+    """``g^T x`` over the tokens: one split contraction kernel
+    (``tsattn_linear_wgrad``) where the product is long and its output small
+    enough to leave most of the chip idle otherwise -- 4096 tokens and up to
+    3072 x 768 outputs (512 x 512, 8192 tokens: 53 us as a library product, 20
+    here; 3072 x 768, 4096 tokens: 45 and 43; 4096 x 1024: 48 and 51; at 2048
+    tokens both take about 19 us)."""
+    import torch
+
+    tokens, m = g.shape
+    n = x.shape[1]
+    if (g.dtype not in (torch.float16, torch.bfloat16) or x.dtype != g.dtype or tokens < 4096
+            or -(-m // 128) * -(-n // 128) > 144 or m % 8 or n % 8 or m == 0 or n == 0
+            or tokens * max(g.stride(0), x.stride(0)) * 2 >= 2**31
+            or any(t.stride(1) != 1 or t.stride(0) % 8 or t.stride(0) < t.shape[1] or t.data_ptr() % 16
+                   for t in (g, x))):
+        return g.t() @ x
+    lib = _lib.load()
+    out = torch.empty((m, n), dtype=g.dtype, device=g.device)
+    nbytes = lib.tsattn_linear_wgrad_workspace(tokens, m, n)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=g.device)
+    _lib.check(lib.tsattn_linear_wgrad(_code(g), tokens, m, n, g.data_ptr(), g.stride(0), x.data_ptr(),
+                                       x.stride(0), out.data_ptr(), ws.data_ptr(), nbytes,
+                                       current_stream(dev)), "linear weight gradient")
+    return out
 
 
 def _rows_linear(x, w, bias, dev):

@@ -448,6 +448,20 @@ int tsattn_rows_swiglu(int32_t dtype, int32_t rows, int32_t k, int32_t n, const 
                        const void *gate, const void *up, void *out, int64_t out_stride, void *stream);
 
 /*
+ * Weight gradient of a linear layer (src/tensorsmith/nn/functional.py:63-90, the
+ * VJP): dw [m, n] = g^T x over `tokens` rows, g [tokens, m] and x [tokens, n]
+ * with row strides in elements; fp32 sums, rounded to dtype once.  f16 or
+ * bf16, m, n and the strides multiples of 8, 16-byte aligned arrays (others:
+ * TSATTN_ERR_UNSUPPORTED).  Deterministic.
+ */
+int tsattn_linear_wgrad(int32_t dtype, int32_t tokens, int32_t m, int32_t n, const void *g, int64_t g_stride,
+                        const void *x, int64_t x_stride, void *dw, void *workspace, size_t workspace_bytes,
+                        void *stream);
+
+/* Bytes of scratch tsattn_linear_wgrad needs (partial sums). */
+size_t tsattn_linear_wgrad_workspace(int32_t tokens, int32_t m, int32_t n);
+
+/*
  * One cached decode step of the attention layer, or of a whole pre-norm
  * decoder block, as one call: MultiHeadAttention.forward with a cache
  * (src/tensorsmith/nn/transformer.py:124-155) and TransformerDecoderBlock.forward
