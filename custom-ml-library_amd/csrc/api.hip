@@ -156,7 +156,7 @@ int rope_unsupported() {
 
 int sdpa_forward(const tsattn_problem *p, const tsattn_rope_desc *rope, const tsattn_view *q,
                  const tsattn_view *k, const tsattn_view *v, const tsattn_view *out, void *lse,
-                 void *stream) {
+                 void *workspace, size_t workspace_bytes, void *stream) {
   tsattn::Problem pr;
   int rc = check_problem(p, &pr);
   if (rc) return rc;
@@ -170,8 +170,12 @@ int sdpa_forward(const tsattn_problem *p, const tsattn_rope_desc *rope, const ts
   if (g_policy.load() == 0 && tsattn::mfma_supported(pr, p->dtype) && mfma_view_ok(vq, pr.Sq) &&
       mfma_view_ok(vk, pr.Sk) && mfma_view_ok(vv, pr.Sk) && mfma_view_ok(vo, pr.Sq)) {
     g_last_path = 2;
+    const size_t split = tsattn::mfma_forward_workspace(pr);
+    float *ws = workspace && split && workspace_bytes >= split && reinterpret_cast<uintptr_t>(workspace) % 16 == 0
+                    ? static_cast<float *>(workspace)
+                    : nullptr;
     return hip_status(tsattn::launch_mfma_forward(pr, p->dtype, vq, vk, vv, vo,
-                                                  static_cast<float *>(lse), st),
+                                                  static_cast<float *>(lse), ws, st),
                       "mfma forward launch");
   }
   if (rope) return rope_unsupported();
@@ -563,14 +567,26 @@ int tsattn_last_kernel_path(void) { return g_last_path; }
 
 int tsattn_sdpa_forward(const tsattn_problem *p, const tsattn_view *q, const tsattn_view *k,
                         const tsattn_view *v, const tsattn_view *out, void *lse, void *stream) {
-  return sdpa_forward(p, nullptr, q, k, v, out, lse, stream);
+  return sdpa_forward(p, nullptr, q, k, v, out, lse, nullptr, 0, stream);
 }
 
 int tsattn_sdpa_forward_rope(const tsattn_problem *p, const tsattn_rope_desc *rope,
                              const tsattn_view *q, const tsattn_view *k, const tsattn_view *v,
                              const tsattn_view *out, void *lse, void *stream) {
   if (!rope) return fail(TSATTN_ERR_INVALID, "RoPE descriptor is NULL");
-  return sdpa_forward(p, rope, q, k, v, out, lse, stream);
+  return sdpa_forward(p, rope, q, k, v, out, lse, nullptr, 0, stream);
+}
+
+size_t tsattn_sdpa_forward_workspace(const tsattn_problem *p) {
+  tsattn::Problem pr;
+  if (check_problem(p, &pr) || !tsattn::mfma_supported(pr, p->dtype)) return 0;
+  return tsattn::mfma_forward_workspace(pr);
+}
+
+int tsattn_sdpa_forward_split(const tsattn_problem *p, const tsattn_rope_desc *rope, const tsattn_view *q,
+                              const tsattn_view *k, const tsattn_view *v, const tsattn_view *out, void *lse,
+                              void *workspace, size_t workspace_bytes, void *stream) {
+  return sdpa_forward(p, rope, q, k, v, out, lse, workspace, workspace_bytes, stream);
 }
 
 size_t tsattn_sdpa_backward_workspace(const tsattn_problem *p) { return backward_workspace(p); }

@@ -46,6 +46,15 @@
 // entering as scores * scale + mask (attention.py:105-107) in log2 units
 // (MK = 2 for an f32 mask, 3 for f16 / bf16; 4..6 the same read as 16-byte
 // row pieces when the keys are contiguous and the rows aligned).
+//
+// Key splits (template SPLIT): a problem with fewer row blocks than the chip
+// runs at once (a chunk of a prompt against a long cache, a short prompt of one
+// sequence) gives each row block to several workgroups, every one a contiguous
+// part of the block's key tiles; they store (max, sum, unnormalised O) in fp32 and
+// fwd_merge_kernel combines them as the recurrence combines tiles.  128 row
+// blocks leave half of the CUs idle and the others with one wave per SIMD, whose
+// MFMA and softmax phases then do not overlap: B1 Hq32 Hkv8 Sq 500 against 8192
+// keys, D128: 145 us, split in four 76 us.
 #include <type_traits>
 
 #include "mfma_common.h"
@@ -70,6 +79,10 @@ struct FwdArgs {
   float sl;  // scale * log2(e)
   int n_qblocks;
   int total;
+  // key splits: partial O [splits][B Hq Sq][Dv], then [splits][B Hq Sq][2] (max
+  // in log2 units, sum)
+  int splits;
+  float *ws;
 };
 
 template <typename T>
@@ -78,8 +91,9 @@ __device__ __forceinline__ const T *head_ptr(View v, int b, int h) {
 }
 
 // DK = head dim of q / k, DV = of v / o (each 64 or 128).
-template <typename T, int DK, int DV, int MK, bool DR>
+template <typename T, int DK, int DV, int MK, bool DR, bool SPLIT>
 __global__ __launch_bounds__(NT, 2) void fwd_kernel(FwdArgs a) {
+  static_assert(!SPLIT || (MK == 0 && !DR), "split problems have no general mask and no dropout");
   constexpr int TILE_K = BN * DK * 2, TILE_V = BN * DV * 2;  // bytes per K / V tile
   constexpr int STAGE = TILE_K + TILE_V;
   // 1 KiB DMA blocks of a K / V tile; wave w loads blocks w, w + NW, ... of
@@ -108,14 +122,17 @@ __global__ __launch_bounds__(NT, 2) void fwd_kernel(FwdArgs a) {
   const Problem &p = a.p;
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, h = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, in an SGPR
-  const int logical = xcd_remap(blockIdx.x, a.total);
+  // (split: the parts of one row block follow each other, on one XCD)
+  const int logical_all = xcd_remap(blockIdx.x, SPLIT ? a.total * a.splits : a.total);
+  const int part = SPLIT ? logical_all % a.splits : 0;
+  const int logical = SPLIT ? logical_all / a.splits : logical_all;
   int bh, rank;
-  heavy_first(logical, a.n_qblocks, a.total / a.n_qblocks, 64, bh, rank);  // 2 WG per CU
+  heavy_first(logical, a.n_qblocks, a.total / a.n_qblocks, SPLIT ? max(1, 64 / a.splits) : 64, bh, rank);  // 2 WG per CU
   const int qb = a.n_qblocks - 1 - rank;  // long causal rows first
   const int b = bh / p.Hq, hq = bh - b * p.Hq, hk = hq / p.rep;
   const int q0 = qb * BM, qw = q0 + 32 * w, qrow = qw + c;
 
-  const int kv_end = kv_end_for(p, b);
+  int kv_end = kv_end_for(p, b);
   const bool keymask =
       MK == 0 && p.mask.kind == TSATTN_MASK_BOOL && !(p.kv_prefix && p.kv_prefix[b]);
 
@@ -129,17 +146,28 @@ __global__ __launch_bounds__(NT, 2) void fwd_kernel(FwdArgs a) {
   }
   if (qw >= p.Sq) wlim = 0;
   // wave-uniform by construction; readfirstlane keeps them in SGPRs
-  const int n_tiles =
+  int n_tiles =
       __builtin_amdgcn_readfirstlane(lim > 0 ? static_cast<int>((lim + BN - 1) / BN) : 0);
-  const int w_tiles =
+  int w_tiles =
       __builtin_amdgcn_readfirstlane(wlim > 0 ? static_cast<int>((wlim + BN - 1) / BN) : 0);
+  // Split: this workgroup's tiles [t0, t1) are a problem of their own whose first
+  // key is k_base; everything below counts keys from there.
+  int k_base = 0;
+  if constexpr (SPLIT) {
+    const int t0 = static_cast<int>(static_cast<int64_t>(n_tiles) * part / a.splits);
+    const int t1 = static_cast<int>(static_cast<int64_t>(n_tiles) * (part + 1) / a.splits);
+    k_base = t0 * BN;
+    kv_end = max(0, min(kv_end, t1 * BN) - k_base);
+    w_tiles = max(0, min(w_tiles, t1) - t0);
+    n_tiles = t1 - t0;
+  }
 
   const uint32_t qs_b = static_cast<uint32_t>(a.q.s2) * 2;
   const uint32_t ks_b = static_cast<uint32_t>(a.k.s2) * 2;
   const uint32_t vs_b = static_cast<uint32_t>(a.v.s2) * 2;
   const rsrc_t qrs = make_rsrc(head_ptr<T>(a.q, b, hq), static_cast<uint32_t>(p.Sq) * qs_b);
-  const u32x4 kdesc = make_desc(head_ptr<T>(a.k, b, hk), static_cast<uint32_t>(kv_end) * ks_b);
-  const u32x4 vdesc = make_desc(head_ptr<T>(a.v, b, hk), static_cast<uint32_t>(kv_end) * vs_b);
+  const u32x4 kdesc = make_desc(head_ptr<T>(a.k, b, hk) + k_base * a.k.s2, static_cast<uint32_t>(kv_end) * ks_b);
+  const u32x4 vdesc = make_desc(head_ptr<T>(a.v, b, hk) + k_base * a.v.s2, static_cast<uint32_t>(kv_end) * vs_b);
 
   // Q fragments (B operand of S^T = K Q^T): lane holds Q[qrow][16ks + 8h .. +7].
   // When the workgroup's 128 Q rows fit in ring stages 2 and 3 (DK <= DV)
@@ -242,11 +270,11 @@ __global__ __launch_bounds__(NT, 2) void fwd_kernel(FwdArgs a) {
   // further thinned by the key mask row kmask_b when there is one.
   int klim = kv_end;
   if (p.causal) {
-    const int64_t cl = static_cast<int64_t>(qrow) + p.offset + 1;
+    const int64_t cl = static_cast<int64_t>(qrow) + p.offset + 1 - k_base;
     if (cl < kv_end) klim = cl < 0 ? 0 : static_cast<int>(cl);
   }
   const uint8_t *kmask_b =
-      keymask ? static_cast<const uint8_t *>(p.mask.data) + b * p.mask.s0 : nullptr;
+      keymask ? static_cast<const uint8_t *>(p.mask.data) + b * p.mask.s0 + k_base * p.mask.s3 : nullptr;
   // General mask: the (b, hq) slice as a buffer; this lane reads row qrow.
   // Rows past Sq use none of what they read.
   constexpr int mes = mask_bytes<MK>();
@@ -320,7 +348,7 @@ __global__ __launch_bounds__(NT, 2) void fwd_kernel(FwdArgs a) {
   int j_edge = kv_end / BN;
   if (MK != 0 || keymask) j_edge = 0;
   if (p.causal) {
-    const int64_t d = static_cast<int64_t>(qw) + p.offset - (BN - 1);
+    const int64_t d = static_cast<int64_t>(qw) + p.offset - (BN - 1) - k_base;
     const int jc = d < 0 ? 0 : static_cast<int>(min(d / BN + 1, static_cast<int64_t>(INT32_MAX)));
     j_edge = min(j_edge, jc);
   }
@@ -381,7 +409,7 @@ __global__ __launch_bounds__(NT, 2) void fwd_kernel(FwdArgs a) {
         unsigned kbits = ~0u;
         if (keymask) {
           const int key = kv0 + lane;
-          const bool ok = key < p.Sk && kmask_b[static_cast<int64_t>(key) * p.mask.s3];
+          const bool ok = key < p.Sk - k_base && kmask_b[static_cast<int64_t>(key) * p.mask.s3];
           kbits = static_cast<unsigned>(__ballot(ok) >> (4 * h));
         }
 #pragma unroll
@@ -510,6 +538,40 @@ __global__ __launch_bounds__(NT, 2) void fwd_kernel(FwdArgs a) {
   }
 
   const float lt = xor32_sum(l);  // lanes c and c+32 share a query row
+  if constexpr (SPLIT) {
+    // The partial rows, fp32, through LDS as below (Dqk < Dv: in two halves of
+    // their channels, the ring being smaller): row r at r 4 DH bytes, its 16-byte
+    // chunk q at q ^ (r % CPF).
+    constexpr int HALVES = NW * 32 * 4 * DV <= NS * STAGE ? 1 : 2;
+    constexpr int DH = DV / HALVES, CPF = DH / 4;
+    static_assert(NW * 32 * 4 * DH <= NS * STAGE, "partial slices fit in the ring");
+    char *fs = lds + w * 32 * 4 * DH;
+    const int64_t rows = static_cast<int64_t>(p.B) * p.Hq * p.Sq, row0 = (static_cast<int64_t>(b) * p.Hq + hq) * p.Sq;
+    float *po = a.ws + (part * rows + row0) * DV;
+#pragma unroll
+    for (int hf = 0; hf < HALVES; ++hf) {
+#pragma unroll
+      for (int dt = 0; dt < PDT / HALVES; ++dt) {
+        const f32x16 &ac = oacc[hf * (PDT / HALVES) + dt];
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<float4 *>(fs + c * 4 * DH + (((8 * dt + 2 * g + h) ^ (c % CPF)) * 16)) =
+              float4{ac[4 * g], ac[4 * g + 1], ac[4 * g + 2], ac[4 * g + 3]};
+      }
+#pragma unroll
+      for (int u = 0; u < 32 * CPF / 64; ++u) {
+        const int idx = u * 64 + lane, r = idx / CPF, q = idx % CPF;
+        const float4 x = *reinterpret_cast<const float4 *>(fs + r * 4 * DH + ((q ^ (r % CPF)) * 16));
+        if (qw + r < p.Sq) *reinterpret_cast<float4 *>(po + static_cast<int64_t>(qw + r) * DV + hf * DH + 4 * q) = x;
+      }
+    }
+    if (h == 0 && qrow < p.Sq) {
+      float *ml = a.ws + a.splits * rows * DV + 2 * (part * rows + row0 + qrow);
+      ml[0] = m;
+      ml[1] = lt;
+    }
+    return;
+  }
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
   // O rows leave through LDS (free after the last barrier, all loads waited
   // for): each wave rounds its 32 rows into its own slice -- row r at r * 2D
@@ -549,23 +611,59 @@ __global__ __launch_bounds__(NT, 2) void fwd_kernel(FwdArgs a) {
         lt > 0.f ? (m + log2f(lt)) * kLn2 : -INFINITY;
 }
 
+// O and the LSE of the split rows: DV / 4 lanes a row, 4 channels a lane.
+template <typename T, int DV>
+__global__ __launch_bounds__(NT) void fwd_merge_kernel(FwdArgs a) {
+  constexpr int LPR = DV / 4, RPB = NT / LPR;
+  const Problem &p = a.p;
+  const int64_t rows = static_cast<int64_t>(p.B) * p.Hq * p.Sq;
+  const int q = threadIdx.x % LPR;
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * RPB + threadIdx.x / LPR;
+  if (row >= rows) return;
+  const float *ml = a.ws + a.splits * rows * DV + 2 * row;
+  float M = -INFINITY;
+  for (int s = 0; s < a.splits; ++s) M = fmaxf(M, ml[2 * s * rows]);
+  const float base = M == -INFINITY ? 0.f : M;
+  float L = 0.f;
+  float4 o{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = 0; s < a.splits; ++s) {
+    const float c = fast_exp2(ml[2 * s * rows] - base);
+    L = fmaf(ml[2 * s * rows + 1], c, L);
+    const float4 x = *reinterpret_cast<const float4 *>(a.ws + (s * rows + row) * DV + 4 * q);
+    o.x = fmaf(x.x, c, o.x), o.y = fmaf(x.y, c, o.y), o.z = fmaf(x.z, c, o.z), o.w = fmaf(x.w, c, o.w);
+  }
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  const int64_t bh = row / p.Sq, i = row - bh * p.Sq, b = bh / p.Hq, hq = bh - b * p.Hq;
+  T *op = static_cast<T *>(const_cast<void *>(a.o.data)) + b * a.o.s0 + hq * a.o.s1 + i * a.o.s2 + 4 * q;
+  *reinterpret_cast<u32x2 *>(op) = u32x2{pack2<T>(o.x * inv, o.y * inv), pack2<T>(o.z * inv, o.w * inv)};
+  if (a.lse && q == 0) a.lse[row] = L > 0.f ? (M + log2f(L)) * kLn2 : -INFINITY;
+}
+
 template <typename T, int DK, int DV, bool DR>
 void launch_dr(const FwdArgs &a, int mk, hipStream_t st) {
   const dim3 g(a.total), blk(NT);
   switch (mk) {
-    case 1: fwd_kernel<T, DK, DV, 1, DR><<<g, blk, 0, st>>>(a); break;
-    case 2: fwd_kernel<T, DK, DV, 2, DR><<<g, blk, 0, st>>>(a); break;
-    case 3: fwd_kernel<T, DK, DV, 3, DR><<<g, blk, 0, st>>>(a); break;
-    case 4: fwd_kernel<T, DK, DV, 4, DR><<<g, blk, 0, st>>>(a); break;
-    case 5: fwd_kernel<T, DK, DV, 5, DR><<<g, blk, 0, st>>>(a); break;
-    case 6: fwd_kernel<T, DK, DV, 6, DR><<<g, blk, 0, st>>>(a); break;
-    default: fwd_kernel<T, DK, DV, 0, DR><<<g, blk, 0, st>>>(a); break;
+    case 1: fwd_kernel<T, DK, DV, 1, DR, false><<<g, blk, 0, st>>>(a); break;
+    case 2: fwd_kernel<T, DK, DV, 2, DR, false><<<g, blk, 0, st>>>(a); break;
+    case 3: fwd_kernel<T, DK, DV, 3, DR, false><<<g, blk, 0, st>>>(a); break;
+    case 4: fwd_kernel<T, DK, DV, 4, DR, false><<<g, blk, 0, st>>>(a); break;
+    case 5: fwd_kernel<T, DK, DV, 5, DR, false><<<g, blk, 0, st>>>(a); break;
+    case 6: fwd_kernel<T, DK, DV, 6, DR, false><<<g, blk, 0, st>>>(a); break;
+    default: fwd_kernel<T, DK, DV, 0, DR, false><<<g, blk, 0, st>>>(a); break;
   }
 }
 
 template <typename T, int DK, int DV>
 void launch_dims(const FwdArgs &a, hipStream_t st) {
   const int mk = mfma_mask_mode_vec(a.p);
+  if (a.splits > 1) {
+    fwd_kernel<T, DK, DV, 0, false, true><<<dim3(a.total * a.splits), dim3(NT), 0, st>>>(a);
+    const int64_t rows = static_cast<int64_t>(a.p.B) * a.p.Hq * a.p.Sq;
+    constexpr int RPB = NT / (DV / 4);
+    fwd_merge_kernel<T, DV><<<dim3(static_cast<unsigned>((rows + RPB - 1) / RPB)), dim3(NT), 0, st>>>(a);
+    return;
+  }
   if (a.p.drop.on) launch_dr<T, DK, DV, true>(a, mk, st);
   else launch_dr<T, DK, DV, false>(a, mk, st);
 }
@@ -597,9 +695,32 @@ bool mfma_supported(const Problem &p, int dtype) {
   return mfma_mask_ok(p);
 }
 
+// Key splits of a forward: as many as fill the two workgroups a CU runs (512; so
+// none above 256 row blocks), each of 11 key tiles (352 keys) or more of an
+// average row.  Unsplit / split, bf16 D128 B1 causal: 32 heads, 16 rows over 8192
+// keys 137 / 25 us, 256 rows 149 / 51; 8 heads of 4096 x 4096 80 / 61; 16 heads
+// of 2048 x 2048 44 / 41; and with shorter parts the merge costs more than the
+// split gains: 32 heads of 1024 x 1024 (8 tiles a part) 27 / 32 us.
+int mfma_forward_splits(const Problem &p) {
+  if (p.drop.on || mfma_mask_mode(p) != 0) return 1;
+  const int64_t total = static_cast<int64_t>((p.Sq + BM - 1) / BM) * p.Hq * p.B;
+  int64_t keys = p.Sk;  // of an average row
+  if (p.causal && p.Sq / 2 + p.offset < keys) keys = p.Sq / 2 + p.offset;
+  const int64_t most = keys / (11 * BN);
+  int64_t s = 512 / total;
+  if (s > most) s = most;
+  return s < 2 ? 1 : static_cast<int>(s);
+}
+
+size_t mfma_forward_workspace(const Problem &p) {
+  const int s = mfma_forward_splits(p);
+  return s < 2 ? 0 : static_cast<size_t>(s) * p.B * p.Hq * p.Sq * (p.Dv + 2) * sizeof(float);
+}
+
 hipError_t launch_mfma_forward(const Problem &p, int dtype, View q, View k, View v, View o,
-                               float *lse, hipStream_t st) {
-  FwdArgs a{p, q, k, v, o, lse, static_cast<float>(p.scale) * kLog2e, (p.Sq + BM - 1) / BM, 0};
+                               float *lse, float *ws, hipStream_t st) {
+  FwdArgs a{p, q, k, v, o, lse, static_cast<float>(p.scale) * kLog2e, (p.Sq + BM - 1) / BM, 0,
+            ws ? mfma_forward_splits(p) : 1, ws};
   a.total = a.n_qblocks * p.Hq * p.B;
   return dtype == TSATTN_BF16 ? launch<bf16>(a, st) : launch<f16>(a, st);
 }

@@ -187,8 +187,11 @@ hipError_t launch_generic_backward(const Problem &p, int dtype, View q, View k, 
 // MFMA kernels: f16 / bf16, dim_qk and dim_v each in {64, 128}, scale > 0; any
 // boolean mask, or an additive mask in f32 / f16 / bf16.
 bool mfma_supported(const Problem &p, int dtype);
+// ws: NULL, or mfma_forward_workspace(p) bytes (0: none wanted) with which the
+// keys of a problem of few row blocks split over several workgroups.
+size_t mfma_forward_workspace(const Problem &p);
 hipError_t launch_mfma_forward(const Problem &p, int dtype, View q, View k, View v, View o,
-                               float *lse, hipStream_t st);
+                               float *lse, float *ws, hipStream_t st);
 // ds: NULL, or mfma_ds_bytes(p) bytes in which the dK/dV kernel stores dS
 // for the dQ product (then it runs first and dQ takes one GEMM).
 hipError_t launch_mfma_backward(const Problem &p, int dtype, View q, View k, View v, View o,

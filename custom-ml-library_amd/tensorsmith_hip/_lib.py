@@ -128,6 +128,9 @@ SIGNATURES = {
         [_PP, _PV, _PV, _PV, _PV, _PV, c_void_p, _PV, _PV, _PV, c_void_p, c_size_t, c_void_p],
     ),
     "tsattn_sdpa_forward_rope": (c_int, [_PP, _PR, _PV, _PV, _PV, _PV, c_void_p, c_void_p]),
+    "tsattn_sdpa_forward_workspace": (c_size_t, [_PP]),
+    "tsattn_sdpa_forward_split": (
+        c_int, [_PP, _PR, _PV, _PV, _PV, _PV, c_void_p, c_void_p, c_size_t, c_void_p]),
     "tsattn_sdpa_backward_rope_workspace": (c_size_t, [_PP]),
     "tsattn_dropout_keep": (c_int, [_PP, c_void_p, c_void_p]),
     "tsattn_dropout_bits_bytes": (c_size_t, [_PP]),

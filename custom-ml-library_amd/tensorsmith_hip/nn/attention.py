@@ -91,6 +91,18 @@ def _problem(b, hq, hkv, sq, sk, dqk, dv, dtype_code, scale, is_causal, offset):
     return p
 
 
+def _forward(lib, prob, rope, vq, vk, vv, vo, lse_ptr, tdev, stream) -> None:
+    """The forward, with scratch for splitting the keys where the problem has
+    too few query row blocks to fill the chip."""
+    import torch
+
+    nbytes = lib.tsattn_sdpa_forward_workspace(ctypes.byref(prob))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=tdev) if nbytes else None
+    _lib.check(lib.tsattn_sdpa_forward_split(
+        ctypes.byref(prob), rope, vq, vk, vv, vo, lse_ptr,
+        None if ws is None else ctypes.c_void_p(ws.data_ptr()), nbytes, stream), "attention forward")
+
+
 def scaled_dot_product_attention(
     query: Tensor,
     key: Tensor,
@@ -294,15 +306,13 @@ def scaled_dot_product_attention(
             rope[0].q_rotated = q_rot.data_ptr()
             keep.append(q_rot)
         try:
-            _lib.check(lib.tsattn_sdpa_forward_rope(ctypes.byref(prob), ctypes.byref(rope[0]), vq, vk,
-                                                    vv, vo, lse_ptr, stream), "attention forward")
+            _forward(lib, prob, ctypes.byref(rope[0]), vq, vk, vv, vo, lse_ptr, tdev, stream)
             fused = True
         except NotImplementedError:  # not an MFMA problem: rotate the queries separately
             q = _rope_rows(q, q_pos0, base, dim, False, query.device)
             vq = _view(q)
     if not fused:
-        _lib.check(lib.tsattn_sdpa_forward(ctypes.byref(prob), vq, vk, vv, vo, lse_ptr, stream),
-                   "attention forward")
+        _forward(lib, prob, None, vq, vk, vv, vo, lse_ptr, tdev, stream)
     if not recording:
         return Tensor._from_op(out, (query, key, value), None, "sdpa_hip")
 

@@ -209,6 +209,19 @@ int tsattn_sdpa_forward_rope(const tsattn_problem *p, const tsattn_rope_desc *ro
                              const tsattn_view *q, const tsattn_view *k, const tsattn_view *v,
                              const tsattn_view *out, void *lse, void *stream);
 
+/*
+ * The same two forwards (rope NULL or not) with scratch for splitting the keys:
+ * a 16-bit problem of few query row blocks against many keys (a chunk of a
+ * prompt over a long cache) then runs each block's keys on several workgroups
+ * and merges their partial rows in fp32 (attention.py:185-193 applied to
+ * whole parts).  tsattn_sdpa_forward_workspace: the bytes it wants (0: the
+ * problem is not split); less, or NULL, runs unsplit.
+ */
+size_t tsattn_sdpa_forward_workspace(const tsattn_problem *p);
+int tsattn_sdpa_forward_split(const tsattn_problem *p, const tsattn_rope_desc *rope, const tsattn_view *q,
+                              const tsattn_view *k, const tsattn_view *v, const tsattn_view *out, void *lse,
+                              void *workspace, size_t workspace_bytes, void *stream);
+
 /* Bytes of scratch tsattn_sdpa_backward_rope needs: the row values of
  * tsattn_sdpa_backward plus the rotated query rows the dK/dV kernel reads. */
 size_t tsattn_sdpa_backward_rope_workspace(const tsattn_problem *p);
