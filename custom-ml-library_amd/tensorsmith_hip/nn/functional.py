@@ -116,14 +116,16 @@ def _rows_linear(x, w, bias, dev):
     """``x W^T (+ bias)`` of a few 16-bit rows in one kernel
     (``tsattn_rows_linear``), or None outside it.  Over 32 rows each weight is
     read by two row blocks, and wide layers are the library's (K 4096, 64 rows:
-    N 4096 13 us here and 12 there, N 16384 51 and 32)."""
+    N 4096 13 us here and 12 there, N 16384 51 and 32).  The kernel's offsets are
+    32-bit: rows picked out of a tensor of 2^31 bytes and more are the library's."""
     import torch
 
     rows, k = x.shape
     n = w.shape[0]
     if (x.dtype not in (torch.float16, torch.bfloat16) or w.dtype != x.dtype or not 0 < rows <= 64
             or (rows > 32 and n > 8192) or k % 8 or n % 4 or k == 0 or n == 0 or x.stride(1) != 1
-            or x.stride(0) % 8 or not w.is_contiguous() or x.data_ptr() % 16 or w.data_ptr() % 16
+            or x.stride(0) % 8 or (rows * x.stride(0) + k) * 2 >= 2**31 or k >= 2**25
+            or not w.is_contiguous() or x.data_ptr() % 16 or w.data_ptr() % 16
             or (bias is not None and (bias.dtype != x.dtype or not bias.is_contiguous()
                                       or bias.data_ptr() % 16))):
         return None

@@ -24,6 +24,8 @@ step a one-token attention call over the caches (the split-K decode kernel).
 
 from __future__ import annotations
 
+import math
+
 import numpy as np
 
 from dataclasses import dataclass
@@ -79,7 +81,9 @@ def _cached_step(x: Tensor, attention, cache, is_causal: bool = True, block=None
         if (not all(_plain(m, Linear) and m.bias is None for m in mlp) or not _plain(ffn, SwiGLU)
                 or not _plain(attention, MultiHeadAttention) or not _plain(block.attention_norm, RMSNorm)
                 or not _plain(block.ffn_norm, RMSNorm)
-                or any(d.training and d.p for d in (block.residual_dropout, ffn.dropout))):
+                or any(d.training and d.p for d in (block.residual_dropout, ffn.dropout))
+                or not all(n.eps > 0 and math.isfinite(n.eps)
+                           for n in (block.attention_norm, block.ffn_norm))):
             return None
         hidden = ffn.gate.weight.shape[0]
         widest = max(e, hidden)
@@ -92,11 +96,11 @@ def _cached_step(x: Tensor, attention, cache, is_causal: bool = True, block=None
     desc = _lib.StepDesc()
     keep = [raw] if raw.is_contiguous() else [raw.contiguous()]
 
-    def at(tensor, *shape):  # the pointer of a contiguous operand of the step's dtype, else 0
+    def at(tensor, *shape):  # the pointer of a contiguous operand of the step's dtype and device, else 0
         if tensor is None:
             return None
         data = tensor._data
-        if data.dtype != raw.dtype or not data.is_contiguous() or tuple(data.shape) != shape:
+        if tensor.device != x.device or data.dtype != raw.dtype or not data.is_contiguous() or tuple(data.shape) != shape:
             return 0
         keep.append(data)
         return data.data_ptr()

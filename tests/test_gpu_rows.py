@@ -159,3 +159,23 @@ def test_block_step_leaves_replaced_layers_alone():
             block(x, cache=cache)
     assert not torch.equal(plain._data, changed._data)
     assert cache.length == 200
+
+
+def test_rows_of_a_large_tensor_and_bad_eps_stay_with_the_layers():
+    """The last position of a long batch (a row stride past the kernel's 32-bit
+    offsets) is multiplied all the same; a norm's eps is checked in a cached step."""
+    far = torch.empty(2, 2**20, 512, dtype=torch.float16, device="cuda")[:, -1]
+    far.copy_(torch.randn(2, 512, device="cuda"))
+    w = torch.randn(64, 512, device="cuda").half()
+    assert (far.shape[0] * far.stride(0) + 512) * 2 >= 2**31
+    got = F.linear(ts.Tensor(far, device="hip"), ts.Tensor(w, device="hip"))._data
+    _close(got, far.double() @ w.double().t(), torch.float16, 2)
+    block = nn.TransformerDecoderBlock(256, 4, 512, device="hip").eval()
+    block.to(dtype="float16")
+    cache = block.attention.new_cache(1, 256, dtype="float16")
+    x = ts.Tensor(torch.randn(1, 200, 256, device="cuda").half(), device="hip")
+    with ts.no_grad():
+        block(x, cache=cache)
+        block.ffn_norm.eps = 0.0
+        with pytest.raises(ValueError, match="eps"):
+            block(x[:, :1], cache=cache)
