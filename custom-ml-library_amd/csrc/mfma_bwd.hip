@@ -149,7 +149,7 @@ constexpr int KV_PD = 2;  // tiles in flight
 // and is still faster than alone on its CU: 0.88 against 1.07 ms at B16 H16
 // S2048 D128.)
 // Masks the dK/dV kernel stages through its LDS ring (modes 4 and 6: boolean
-// or 16-bit, key-contiguous with 16-byte aligned rows) hold no registers.
+// or 16-bit, key-contiguous with 4-byte aligned rows) hold no registers.
 constexpr bool mask_staged(int MK) { return MK == 4 || MK == 6; }
 
 template <int DK, int DV, int MK, bool DR>

@@ -92,7 +92,7 @@ struct MaskFetch {
     for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(v[i]));
   }
 
-  // Key-contiguous masks with 16-byte aligned rows: lane half h loads keys
+  // Key-contiguous masks with 4-byte aligned rows: lane half h loads keys
   // 16 h .. 16 h + 15 of the lane's row within the 32-key tile (NQ 16-byte
   // loads: bool 1, 16-bit 2, f32 4) into v[0 .. 4 NQ), resolve(), then
   // unpack<ES>(h) trades quarters with the partner lane (keys 4 m .. 4 m + 3
@@ -158,7 +158,7 @@ __device__ __forceinline__ void MaskFetch::unpack(int h) {
 
 // Mask modes MK: 1 boolean, 2 additive f32, 3 additive f16 / bf16, read
 // element by element; 4, 5, 6 the same kinds read as 16-byte row pieces
-// (key-contiguous, 16-byte aligned rows; the forward and dQ kernels).
+// (key-contiguous, 4-byte aligned rows; the forward and dQ kernels).
 constexpr int mask_kind(int MK) { return MK > 3 ? MK - 3 : MK; }
 constexpr bool mask_vec(int MK) { return MK > 3; }
 // Bytes per mask element.

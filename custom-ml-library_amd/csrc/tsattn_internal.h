@@ -131,14 +131,18 @@ inline bool mfma_mask_ok(const Problem &p) {
   return ((p.Sq + 128) * m.s2 + (p.Sk + 128) * m.s3 + 1) * es < (int64_t(1) << 31);
 }
 // The same, read as 16-byte row pieces (modes 4..6) where the keys are
-// contiguous and every row starts 16-byte aligned.
+// contiguous and every row starts 4-byte aligned, which is what a 16-byte
+// buffer load asks for (its range is checked per 4 bytes, so the piece at the
+// end of the last row keeps the elements inside): every f32 mask, 16-bit ones
+// of even and boolean ones of 4-fold row lengths.  An f32 [1,16,1111,1111] bias,
+// B3 Hkv4 D128 causal, bf16: forward 90 us by elements, 67 by pieces.
 inline int mfma_mask_mode_vec(const Problem &p) {
   const int mk = mfma_mask_mode(p);
   if (mk == 0) return 0;
   const int64_t es = mk == 1 ? 1 : (mk == 2 ? 4 : 2);
   const MaskDesc &m = p.mask;
-  const bool ok = m.s3 == 1 && (m.s0 * es) % 16 == 0 && (m.s1 * es) % 16 == 0 &&
-                  (m.s2 * es) % 16 == 0 && reinterpret_cast<uintptr_t>(m.data) % 16 == 0;
+  const bool ok = m.s3 == 1 && (m.s0 * es) % 4 == 0 && (m.s1 * es) % 4 == 0 &&
+                  (m.s2 * es) % 4 == 0 && reinterpret_cast<uintptr_t>(m.data) % 4 == 0;
   return ok ? mk + 3 : mk;
 }
 
