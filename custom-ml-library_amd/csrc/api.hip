@@ -886,11 +886,13 @@ size_t tsattn_linear_wgrad_workspace(int32_t tokens, int32_t m, int32_t n) {
   return tokens > 0 && m > 0 && n > 0 ? tsattn::wgrad_workspace_bytes(tokens, m, n) : 0;
 }
 
-int tsattn_linear_wgrad(int32_t dtype, int32_t tokens, int32_t m, int32_t n, const void *g, int64_t g_stride,
+int tsattn_linear_wgrad(int32_t dtype, int32_t out_dtype, int32_t tokens, int32_t m, int32_t n, const void *g, int64_t g_stride,
                         const void *x, int64_t x_stride, void *dw, void *workspace, size_t workspace_bytes,
                         void *stream) {
   if (dtype != TSATTN_F16 && dtype != TSATTN_BF16)
     return fail(TSATTN_ERR_INVALID, "the weight gradient takes dtype f16 or bf16 (got dtype %d)", dtype);
+  if (out_dtype != dtype && out_dtype != TSATTN_F32)
+    return fail(TSATTN_ERR_INVALID, "the weight gradient is in dtype or f32 (got dtype %d)", out_dtype);
   if (tokens <= 0 || m <= 0 || n <= 0) return fail(TSATTN_ERR_INVALID, "linear layers need positive sizes");
   if (!g || !x || !dw) return fail(TSATTN_ERR_INVALID, "data pointer is NULL");
   const uintptr_t al = reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(x) |
@@ -903,7 +905,7 @@ int tsattn_linear_wgrad(int32_t dtype, int32_t tokens, int32_t m, int32_t n, con
   const size_t need = tsattn::wgrad_workspace_bytes(tokens, m, n);
   if (!workspace || workspace_bytes < need)
     return fail(TSATTN_ERR_INVALID, "weight gradient workspace too small: %zu < %zu bytes", workspace_bytes, need);
-  return hip_status(tsattn::launch_wgrad(dtype, tokens, m, n, g, g_stride, x, x_stride, dw,
+  return hip_status(tsattn::launch_wgrad(dtype, out_dtype, tokens, m, n, g, g_stride, x, x_stride, dw,
                                          static_cast<float *>(workspace), static_cast<hipStream_t>(stream)),
                     "weight gradient launch");
 }

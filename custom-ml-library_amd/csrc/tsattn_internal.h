@@ -296,7 +296,7 @@ hipError_t launch_rows_swiglu(int dtype, int rows, int K, int N, const void *x, 
 // dw [M, N] = g^T x over `tokens` rows g [tokens, M], x [tokens, N] (f16 / bf16,
 // row strides gs / xs); ws: wgrad_workspace_bytes of partial sums.
 size_t wgrad_workspace_bytes(int tokens, int M, int N);
-hipError_t launch_wgrad(int dtype, int tokens, int M, int N, const void *g, int64_t gs, const void *x,
+hipError_t launch_wgrad(int dtype, int out_dtype, int tokens, int M, int N, const void *g, int64_t gs, const void *x,
                         int64_t xs, void *dw, float *ws, hipStream_t st);
 
 hipError_t launch_key_mask_lengths(const uint8_t *mask, int64_t sb, int64_t sk, int B, int K,

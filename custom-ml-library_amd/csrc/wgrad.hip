@@ -130,8 +130,11 @@ __global__ __launch_bounds__(NT, 2) void wgrad_kernel(WgradArgs a) {
 // thread adds them all.  More: the workgroup's four waves take every 4th split
 // of the same 64 pieces, eight loads in flight each, and add up in order (512 x
 // 512, 16 splits: 7 -> 4 us; at 4 splits the extra workgroups cost 2 us).
-template <typename T, int G>
-__global__ __launch_bounds__(NT) void wgrad_reduce_kernel(const float *part, int splits, int64_t n4, T *out) {
+//
+// O: T, or float for a parameter kept in fp32 -- the sum rounded to T all the
+// same, as a T gradient widened afterwards would be, without that pass.
+template <typename T, typename O, int G>
+__global__ __launch_bounds__(NT) void wgrad_reduce_kernel(const float *part, int splits, int64_t n4, O *out) {
   typedef float f4 __attribute__((ext_vector_type(4)));
   constexpr int PER = NT / G;  // pieces per workgroup
   __shared__ f4 red[G][PER];
@@ -156,7 +159,14 @@ __global__ __launch_bounds__(NT) void wgrad_reduce_kernel(const float *part, int
     for (int k = 1; k < G; ++k) s += red[k][lane];
   }
   if (i >= n4) return;
-  *reinterpret_cast<u32x2 *>(out + 4 * i) = u32x2{pack2<T>(s[0], s[1]), pack2<T>(s[2], s[3])};
+  if constexpr (sizeof(O) == 4) {
+    f4 r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = static_cast<float>(static_cast<T>(s[e]));
+    *reinterpret_cast<f4 *>(out + 4 * i) = r;
+  } else {
+    *reinterpret_cast<u32x2 *>(out + 4 * i) = u32x2{pack2<T>(s[0], s[1]), pack2<T>(s[2], s[3])};
+  }
 }
 
 // One workgroup a CU (256): at two a CU the partial tiles' traffic doubles and
@@ -178,7 +188,7 @@ size_t wgrad_workspace_bytes(int tokens, int M, int N) {
   return static_cast<size_t>(wgrad_splits(tokens, M, N)) * M * N * sizeof(float);
 }
 
-hipError_t launch_wgrad(int dtype, int tokens, int M, int N, const void *g, int64_t gs, const void *x,
+hipError_t launch_wgrad(int dtype, int out_dtype, int tokens, int M, int N, const void *g, int64_t gs, const void *x,
                         int64_t xs, void *dw, float *ws, hipStream_t st) {
   const int splits = wgrad_splits(tokens, M, N);
   const int per = ((tokens + splits - 1) / splits + BT - 1) / BT * BT;
@@ -192,16 +202,18 @@ hipError_t launch_wgrad(int dtype, int tokens, int M, int N, const void *g, int6
     else wgrad_kernel<f16><<<grid, blk, 0, st>>>(a);
   }
   Probe pr_("wgrad_reduce", st);
-  auto reduce = [&](auto tag) {
+  auto reduce = [&](auto tag, auto otag) {
     using T = decltype(tag);
-    T *out = static_cast<T *>(dw);
+    using O = decltype(otag);
+    O *out = static_cast<O *>(dw);
     if (splits > 8)
-      wgrad_reduce_kernel<T, 4><<<dim3(static_cast<unsigned>((n4 + 63) / 64)), blk, 0, st>>>(ws, splits, n4, out);
+      wgrad_reduce_kernel<T, O, 4><<<dim3(static_cast<unsigned>((n4 + 63) / 64)), blk, 0, st>>>(ws, splits, n4, out);
     else
-      wgrad_reduce_kernel<T, 1><<<dim3(static_cast<unsigned>((n4 + NT - 1) / NT)), blk, 0, st>>>(ws, splits, n4, out);
+      wgrad_reduce_kernel<T, O, 1>
+          <<<dim3(static_cast<unsigned>((n4 + NT - 1) / NT)), blk, 0, st>>>(ws, splits, n4, out);
   };
-  if (dtype == TSATTN_BF16) reduce(bf16{});
-  else reduce(f16{});
+  if (dtype == TSATTN_BF16) out_dtype == TSATTN_F32 ? reduce(bf16{}, 0.f) : reduce(bf16{}, bf16{});
+  else out_dtype == TSATTN_F32 ? reduce(f16{}, 0.f) : reduce(f16{}, f16{});
   return hipGetLastError();
 }
 

@@ -201,7 +201,7 @@ SIGNATURES = {
     "tsattn_linear_wgrad_workspace": (c_size_t, [c_int32, c_int32, c_int32]),
     "tsattn_linear_wgrad": (
         c_int,
-        [c_int32, c_int32, c_int32, c_int32, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p,
+        [c_int32, c_int32, c_int32, c_int32, c_int32, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p,
          c_size_t, c_void_p],
     ),
     "tsattn_cached_step_workspace": (c_size_t, [POINTER(StepDesc)]),

@@ -16,7 +16,7 @@ import math
 from .. import _lib
 from ..amp import _cast_inputs
 from ..device import current_stream, random_uniform
-from ..tensor import Tensor, _sum_to_shape, is_grad_enabled, is_torch
+from ..tensor import Tensor, _sum_to_shape, is_grad_enabled, is_torch, no_grad
 from .attention import rotary_embedding, scaled_dot_product_attention
 
 __all__ = [
@@ -55,8 +55,12 @@ def _compute(raw):
 
 
 def linear(input: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
-    """x @ W^T + b as one node (reference ``functional.py:63-90``), autocast-aware."""
-    input, weight, bias = _cast_inputs(input, weight, bias)
+    """x @ W^T + b as one node (reference ``functional.py:63-90``), autocast-aware:
+    the casts belong to the node, its gradients are rounded as the cast operands'
+    would be and returned in the dtypes of the operands given."""
+    given = tuple(t for t in (input, weight, bias) if t is not None)
+    with no_grad():
+        input, weight, bias = _cast_inputs(input, weight, bias)
     if input.ndim < 1 or weight.ndim != 2 or input.shape[-1] != weight.shape[1]:
         raise ValueError("linear expects [...,in_features] and [out_features,in_features]")
     parents = (input, weight) if bias is None else (input, weight, bias)
@@ -77,16 +81,17 @@ def linear(input: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
     def backward(g):
         flat = g.reshape(-1, weight.shape[0])
         grads = [(flat @ w).reshape(input.shape).to(input.dtype),
-                 _weight_grad(flat, x, input.device).to(weight.dtype)]
+                 _weight_grad(flat, x, input.device, weight.dtype, given[1].dtype)]
         if bias is not None:
             grads.append(flat.sum(0).to(bias.dtype))
-        return tuple(grads)
+        return tuple(d.to(t.dtype) for d, t in zip(grads, given))
 
-    return Tensor._from_op(out, parents, backward, "linear")
+    return Tensor._from_op(out, given, backward, "linear")
 
 
-def _weight_grad(g, x, dev):
-    """``g^T x`` over the tokens: one split contraction kernel
+def _weight_grad(g, x, dev, dtype, store):
+    """``g^T x`` over the tokens, rounded to ``dtype`` and given in ``store`` (that
+    or float32, into which the kernel widens the rounded sums): one split contraction kernel
     (``tsattn_linear_wgrad``) where the product is long and its output small
     enough to leave most of the chip idle otherwise -- 4096 tokens and up to
     3072 x 768 outputs (512 x 512, 8192 tokens: 53 us as a library product, 20
@@ -101,15 +106,17 @@ def _weight_grad(g, x, dev):
             or tokens * max(g.stride(0), x.stride(0)) * 2 >= 2**31
             or any(t.stride(1) != 1 or t.stride(0) % 8 or t.stride(0) < t.shape[1] or t.data_ptr() % 16
                    for t in (g, x))):
-        return g.t() @ x
+        return (g.t() @ x).to(dtype)
+    if store != torch.float32 or dtype != g.dtype:
+        store = g.dtype
     lib = _lib.load()
-    out = torch.empty((m, n), dtype=g.dtype, device=g.device)
+    out = torch.empty((m, n), dtype=store, device=g.device)
     nbytes = lib.tsattn_linear_wgrad_workspace(tokens, m, n)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=g.device)
-    _lib.check(lib.tsattn_linear_wgrad(_code(g), tokens, m, n, g.data_ptr(), g.stride(0), x.data_ptr(),
+    _lib.check(lib.tsattn_linear_wgrad(_code(g), _code(out), tokens, m, n, g.data_ptr(), g.stride(0), x.data_ptr(),
                                        x.stride(0), out.data_ptr(), ws.data_ptr(), nbytes,
                                        current_stream(dev)), "linear weight gradient")
-    return out
+    return out if dtype == g.dtype else out.to(dtype)
 
 
 def _rows_linear(x, w, bias, dev):

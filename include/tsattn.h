@@ -463,11 +463,12 @@ int tsattn_rows_swiglu(int32_t dtype, int32_t rows, int32_t k, int32_t n, const 
 /*
  * Weight gradient of a linear layer (src/tensorsmith/nn/functional.py:63-90, the
  * VJP): dw [m, n] = g^T x over `tokens` rows, g [tokens, m] and x [tokens, n]
- * with row strides in elements; fp32 sums, rounded to dtype once.  f16 or
+ * with row strides in elements; fp32 sums, rounded to dtype once and stored in
+ * out_dtype: dtype, or f32 (the rounded value widened).  f16 or
  * bf16, m, n and the strides multiples of 8, 16-byte aligned arrays (others:
  * TSATTN_ERR_UNSUPPORTED).  Deterministic.
  */
-int tsattn_linear_wgrad(int32_t dtype, int32_t tokens, int32_t m, int32_t n, const void *g, int64_t g_stride,
+int tsattn_linear_wgrad(int32_t dtype, int32_t out_dtype, int32_t tokens, int32_t m, int32_t n, const void *g, int64_t g_stride,
                         const void *x, int64_t x_stride, void *dw, void *workspace, size_t workspace_bytes,
                         void *stream);
 

@@ -42,11 +42,13 @@ def test_wgrad_matches_float64(tokens, m, n, dt):
     lib = _lib.load()
     nbytes = lib.tsattn_linear_wgrad_workspace(tokens, m, n)
     ws = torch.full((nbytes,), 255, dtype=torch.uint8, device="cuda")  # NaN bytes: every partial is written
-    out = torch.empty(m, n, dtype=dt, device="cuda")
-    _lib.check(lib.tsattn_linear_wgrad(CODE[dt], tokens, m, n, g.data_ptr(), g.stride(0), x.data_ptr(), x.stride(0),
-                                       out.data_ptr(), ws.data_ptr(), nbytes,
-                                       torch.cuda.current_stream().cuda_stream), "wgrad")
+    out, wide = (torch.empty(m, n, dtype=t, device="cuda") for t in (dt, torch.float32))
+    for to, code in ((out, CODE[dt]), (wide, _lib.F32)):
+        _lib.check(lib.tsattn_linear_wgrad(CODE[dt], code, tokens, m, n, g.data_ptr(), g.stride(0), x.data_ptr(),
+                                           x.stride(0), to.data_ptr(), ws.data_ptr(), nbytes,
+                                           torch.cuda.current_stream().cuda_stream), "wgrad")
     _close(out, g.double().t() @ x.double(), dt, tokens)
+    assert torch.equal(wide, out.float())  # the rounded sums, widened
 
 
 @pytest.mark.parametrize("rows,out_features", [((4, 1024), 264), ((3, 1365), 264), ((4096,), 100)])
