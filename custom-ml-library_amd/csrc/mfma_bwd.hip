@@ -413,10 +413,9 @@ __global__ __launch_bounds__(NT, (dkdv_wg_per_cu<DK, DV, MK, DR>())) void dkdv_k
                    "v_lshlrev_b32 %0, 4, %0"
                    : "=v"(l16));
       const uint32_t mvoff = (l16 / MROW) * ms2 + l16 % MROW;
-      const int64_t extent = ((p.Sq - 1) * p.mask.s2 + (p.Sk - 1) * p.mask.s3 + 1) * MES;
       const u32x4 mdesc = make_desc(
           static_cast<const char *>(p.mask.data) + (b * p.mask.s0 + t_hq(t) * p.mask.s1) * MES,
-          static_cast<uint32_t>(extent));
+          mask_extent<MK>(p));
 #pragma unroll
       for (int u = 0; u < MPARTS; ++u) {
         const int n = w + NW * u;
@@ -597,10 +596,9 @@ __global__ __launch_bounds__(NT, (dkdv_wg_per_cu<DK, DV, MK, DR>())) void dkdv_k
     MaskFetch mf;
     if constexpr (MK != 0 && !MSTAGE) {
       constexpr int mes = mask_bytes<MK>();
-      const int64_t extent = ((p.Sq - 1) * p.mask.s2 + (p.Sk - 1) * p.mask.s3 + 1) * mes;
       const u32x4 mdesc = make_desc(
           static_cast<const char *>(p.mask.data) + (b * p.mask.s0 + hq * p.mask.s1) * mes,
-          static_cast<uint32_t>(extent));
+          mask_extent<MK>(p));
       const int64_t off0 = (static_cast<int64_t>(q0 + 4 * h) * p.mask.s2 +
                             static_cast<int64_t>(key) * p.mask.s3) * mes;
       mf.issue<mes>(mdesc, static_cast<uint32_t>(off0), static_cast<uint32_t>(p.mask.s2 * mes));
@@ -1070,9 +1068,8 @@ __global__ __launch_bounds__(NT, 2) void dq_kernel(BwdArgs a) {
   u32x4 mdesc{};
   uint32_t mrow = 0, mstep = 0;
   if constexpr (MK != 0) {
-    const int64_t extent = ((p.Sq - 1) * p.mask.s2 + (p.Sk - 1) * p.mask.s3 + 1) * mes;
     mdesc = make_desc(static_cast<const char *>(p.mask.data) + (b * p.mask.s0 + hq * p.mask.s1) * mes,
-                      static_cast<uint32_t>(extent));
+                      mask_extent<MK>(p));
     mrow = static_cast<uint32_t>(static_cast<int64_t>(qrow) * p.mask.s2 * mes);
     mstep = static_cast<uint32_t>(p.mask.s3 * mes);
     if (qrow >= p.Sq) klim = 0;

@@ -164,6 +164,14 @@ constexpr bool mask_vec(int MK) { return MK > 3; }
 // Bytes per mask element.
 template <int MK>
 constexpr int mask_bytes() { return mask_kind(MK) == 1 ? 1 : (mask_kind(MK) == 2 ? 4 : 2); }
+// Bytes of a mask's (b, h) slice for a buffer's range.  Pieces are range-checked
+// per whole 4 bytes, so the last element's four count as inside: they are one
+// aligned word with it.
+template <int MK>
+__device__ __forceinline__ uint32_t mask_extent(const Problem &p) {
+  const int64_t n = ((p.Sq - 1) * p.mask.s2 + (p.Sk - 1) * p.mask.s3 + 1) * mask_bytes<MK>();
+  return static_cast<uint32_t>(mask_vec(MK) ? (n + 3) & ~int64_t(3) : n);
+}
 
 // Apply fetched mask elements: score i is allowed iff lo <= kc(i) < hi and
 // the mask allows it; disallowed scores become -inf.  With an additive mask

@@ -281,9 +281,8 @@ __global__ __launch_bounds__(NT, 2) void fwd_kernel(FwdArgs a) {
   u32x4 mdesc{};
   uint32_t mrow = 0, mstep = 0;
   if constexpr (MK != 0) {
-    const int64_t extent = ((p.Sq - 1) * p.mask.s2 + (p.Sk - 1) * p.mask.s3 + 1) * mes;
     mdesc = make_desc(static_cast<const char *>(p.mask.data) + (b * p.mask.s0 + hq * p.mask.s1) * mes,
-                      static_cast<uint32_t>(extent));
+                      mask_extent<MK>(p));
     mrow = static_cast<uint32_t>(static_cast<int64_t>(qrow) * p.mask.s2 * mes);
     mstep = static_cast<uint32_t>(p.mask.s3 * mes);
     if (qrow >= p.Sq) klim = 0;

