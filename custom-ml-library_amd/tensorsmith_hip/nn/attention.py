@@ -93,10 +93,11 @@ def _problem(b, hq, hkv, sq, sk, dqk, dv, dtype_code, scale, is_causal, offset):
 
 def _forward(lib, prob, rope, vq, vk, vv, vo, lse_ptr, tdev, stream) -> None:
     """The forward, with scratch for splitting the keys where the problem has
-    too few query row blocks to fill the chip."""
+    too few query row blocks to fill the chip (16-bit only; the question costs
+    a small fp32 step about 1 us of its 57)."""
     import torch
 
-    nbytes = lib.tsattn_sdpa_forward_workspace(ctypes.byref(prob))
+    nbytes = lib.tsattn_sdpa_forward_workspace(ctypes.byref(prob)) if prob.dtype in (_lib.F16, _lib.BF16) else 0
     ws = torch.empty(nbytes, dtype=torch.uint8, device=tdev) if nbytes else None
     _lib.check(lib.tsattn_sdpa_forward_split(
         ctypes.byref(prob), rope, vq, vk, vv, vo, lse_ptr,
