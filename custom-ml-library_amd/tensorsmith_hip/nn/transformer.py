@@ -81,7 +81,9 @@ def _cached_step(x: Tensor, attention, cache, is_causal: bool = True, block=None
         if (not all(_plain(m, Linear) and m.bias is None for m in mlp) or not _plain(ffn, SwiGLU)
                 or not _plain(attention, MultiHeadAttention) or not _plain(block.attention_norm, RMSNorm)
                 or not _plain(block.ffn_norm, RMSNorm)
-                or any(d.training and d.p for d in (block.residual_dropout, ffn.dropout))
+                # (a Dropout that is off passes its input on; anything else in its place runs)
+                or not all(_plain(d, Dropout) and 0 <= d.p < 1 and not (d.training and d.p)
+                           for d in (block.residual_dropout, ffn.dropout))
                 or not all(n.eps > 0 and math.isfinite(n.eps)
                            for n in (block.attention_norm, block.ffn_norm))):
             return None
