@@ -43,12 +43,21 @@ from .layers import Dropout, Embedding, Linear
 from .module import Module, Parameter
 
 random_uniform = _device.random_uniform
-_PROJECT_APPEND = KVCache._project_append
 
 
 def _plain(module, cls) -> bool:
-    """``module`` is a ``cls`` itself, its forward not replaced."""
+    """``module`` is a ``cls`` itself, its forward not replaced on the instance
+    (on the class: ``_step_methods``)."""
     return type(module) is cls and "forward" not in module.__dict__
+
+
+def _step_methods() -> tuple:
+    """The methods that a cached step in one call stands for, as they are bound
+    now.  Compared with what they were at import (``_STEP_METHODS``): where a
+    program replaced one on its class, to trace it or to change it, the layers
+    run one by one and so does the replacement."""
+    return (Module.__call__, Linear.forward, RMSNorm.forward, SwiGLU.forward, Dropout.forward,
+            MultiHeadAttention.forward, KVCache._project_append, KVCache.get)
 
 
 def _cached_step(x: Tensor, attention, cache, is_causal: bool = True, block=None):
@@ -63,7 +72,8 @@ def _cached_step(x: Tensor, attention, cache, is_causal: bool = True, block=None
 
     raw = x._data
     if (raw.dtype not in (torch.float16, torch.bfloat16) or type(cache) is not KVCache
-            or KVCache._project_append is not _PROJECT_APPEND or cache.dtype != raw.dtype
+            or _step_methods() != _STEP_METHODS or "_project_append" in vars(cache)
+            or cache.dtype != raw.dtype
             or cache.device != x.device or attention.backend == "native"):
         return None
     b, t, e = raw.shape
@@ -314,6 +324,9 @@ class TransformerDecoderBlock(Module):
         hidden = input + self.residual_dropout(
             self.attention(self.attention_norm(input), cache=cache, attn_mask=attn_mask))
         return hidden + self.ffn(self.ffn_norm(hidden))
+
+
+_STEP_METHODS = _step_methods()
 
 
 @dataclass(frozen=True)

@@ -86,3 +86,15 @@ def test_a_dropout_that_drops_is_run(stub):
     assert _step(block) is None and not stub
     block.ffn.dropout.p = 0.0
     assert _step(block) is not None
+
+
+@pytest.mark.parametrize("cls,name", [(Module, "__call__"), (nn.Linear, "forward"), (nn.RMSNorm, "forward"),
+                                      (nn.SwiGLU, "forward"), (nn.Dropout, "forward"),
+                                      (nn.MultiHeadAttention, "forward"), (nn.KVCache, "_project_append"),
+                                      (nn.KVCache, "get")], ids=lambda v: getattr(v, "__name__", v))
+def test_a_method_replaced_on_its_class_is_run(stub, cls, name):
+    block = _block()
+    original = getattr(cls, name)
+    with patch.object(cls, name, lambda self, *a, **k: original(self, *a, **k)):
+        assert _step(block) is None and not stub
+    assert _step(block) is not None
