@@ -194,3 +194,16 @@ def current_stream(dev: Device) -> int:
     import torch
 
     return torch.cuda.current_stream(dev.torch).cuda_stream
+
+
+def launch(dev: Device, function, *args) -> int:
+    """``function(*args, stream)``, a library call, on ``dev``'s current stream and
+    with ``dev`` the current device: a kernel goes to the current device whatever
+    its operands' is, and the default stream's handle (0) names no device."""
+    import torch
+
+    stream = current_stream(dev)
+    if torch.cuda.current_device() == dev.index:
+        return function(*args, stream)
+    with torch.cuda.device(dev.index):
+        return function(*args, stream)

@@ -15,7 +15,7 @@ import math
 
 from .. import _lib
 from ..amp import _cast_inputs
-from ..device import current_stream, random_uniform
+from ..device import launch, random_uniform
 from ..tensor import Tensor, _sum_to_shape, is_grad_enabled, is_torch, no_grad
 from .attention import rotary_embedding, scaled_dot_product_attention
 
@@ -113,9 +113,8 @@ def _weight_grad(g, x, dev, dtype, store):
     out = torch.empty((m, n), dtype=store, device=g.device)
     nbytes = lib.tsattn_linear_wgrad_workspace(tokens, m, n)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=g.device)
-    _lib.check(lib.tsattn_linear_wgrad(_code(g), _code(out), tokens, m, n, g.data_ptr(), g.stride(0), x.data_ptr(),
-                                       x.stride(0), out.data_ptr(), ws.data_ptr(), nbytes,
-                                       current_stream(dev)), "linear weight gradient")
+    _lib.check(launch(dev, lib.tsattn_linear_wgrad, _code(g), _code(out), tokens, m, n, g.data_ptr(), g.stride(0),
+                      x.data_ptr(), x.stride(0), out.data_ptr(), ws.data_ptr(), nbytes), "linear weight gradient")
     return out if dtype == g.dtype else out.to(dtype)
 
 
@@ -137,10 +136,9 @@ def _rows_linear(x, w, bias, dev):
                                       or bias.data_ptr() % 16))):
         return None
     out = torch.empty((rows, n), dtype=x.dtype, device=x.device)
-    _lib.check(_lib.load().tsattn_rows_linear(
-        _code(x), rows, k, n, x.data_ptr(), x.stride(0), w.data_ptr(),
-        None if bias is None else bias.data_ptr(), None, 0, out.data_ptr(), n, current_stream(dev)),
-        "few-row linear")
+    _lib.check(launch(dev, _lib.load().tsattn_rows_linear, _code(x), rows, k, n, x.data_ptr(), x.stride(0),
+                      w.data_ptr(), None if bias is None else bias.data_ptr(), None, 0, out.data_ptr(), n),
+               "few-row linear")
     return out
 
 
@@ -217,9 +215,8 @@ def _norm_kernel(input, weight, bias, eps, rms, dim, parents) -> Tensor:
     if is_grad_enabled() and any(p.requires_grad for p in parents):
         rstd = torch.empty(rows, dtype=torch.float32, device=x.device)
         mean = None if rms else torch.empty(rows, dtype=torch.float32, device=x.device)
-    _lib.check(lib.tsattn_norm_forward(code, w_code, rows, dim, rms, _ptr(x), _ptr(w), _ptr(b),
-                                       _ptr(out), _ptr(mean), _ptr(rstd), eps,
-                                       ctypes.c_void_p(current_stream(input.device))), "norm")
+    _lib.check(launch(input.device, lib.tsattn_norm_forward, code, w_code, rows, dim, rms, _ptr(x), _ptr(w),
+                      _ptr(b), _ptr(out), _ptr(mean), _ptr(rstd), eps), "norm")
 
     def backward(g):
         g = _flat(g.to(x.dtype))
@@ -228,11 +225,9 @@ def _norm_kernel(input, weight, bias, eps, rms, dim, parents) -> Tensor:
         db = None if b is None else torch.empty(b.shape, dtype=b.dtype, device=x.device)
         nbytes = lib.tsattn_norm_backward_workspace(rows, dim, rms)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-        _lib.check(lib.tsattn_norm_backward(code, w_code, rows, dim, rms, _ptr(x), _ptr(w), _ptr(g),
-                                            _ptr(mean), _ptr(rstd), _ptr(dx), _ptr(dw), _ptr(db),
-                                            _ptr(ws), nbytes,
-                                            ctypes.c_void_p(current_stream(input.device))),
-                   "norm backward")
+        _lib.check(launch(input.device, lib.tsattn_norm_backward, code, w_code, rows, dim, rms, _ptr(x),
+                          _ptr(w), _ptr(g), _ptr(mean), _ptr(rstd), _ptr(dx), _ptr(dw), _ptr(db),
+                          _ptr(ws), nbytes), "norm backward")
         return (dx, dw) if b is None else (dx, dw, db)
 
     return Tensor._from_op(out, parents, backward, "rms_norm" if rms else "layer_norm")
@@ -276,16 +271,13 @@ def _silu_mul(gate: Tensor, up: Tensor) -> Tensor:
     lib, code = _lib.load(), _code(a)
     a, b = _flat(a), _flat(b)
     out = torch.empty(a.shape, dtype=a.dtype, device=a.device)
-    _lib.check(lib.tsattn_silu_mul(code, a.numel(), _ptr(a), _ptr(b), _ptr(out),
-                                   ctypes.c_void_p(current_stream(gate.device))), "SwiGLU")
+    _lib.check(launch(gate.device, lib.tsattn_silu_mul, code, a.numel(), _ptr(a), _ptr(b), _ptr(out)), "SwiGLU")
 
     def backward(g):
         g = _flat(g.to(a.dtype))
         da, db = torch.empty_like(a), torch.empty_like(b)
-        _lib.check(lib.tsattn_silu_mul_backward(code, a.numel(), _ptr(a), _ptr(b), _ptr(g), _ptr(da),
-                                                _ptr(db),
-                                                ctypes.c_void_p(current_stream(gate.device))),
-                   "SwiGLU backward")
+        _lib.check(launch(gate.device, lib.tsattn_silu_mul_backward, code, a.numel(), _ptr(a), _ptr(b),
+                          _ptr(g), _ptr(da), _ptr(db)), "SwiGLU backward")
         return da, db
 
     return Tensor._from_op(out, (gate, up), backward, "silu_mul")

@@ -32,7 +32,7 @@ from dataclasses import dataclass
 
 from .. import _lib
 from .. import device as _device
-from ..device import current_stream
+from ..device import launch
 from ..tensor import Tensor, cat, is_grad_enabled, no_grad
 from . import functional as F
 from .attention import (BACKENDS, DECODE_MIN_KEYS, _dtype_code, _view, decode_int8_cache, rope_tables,
@@ -149,8 +149,7 @@ def _cached_step(x: Tensor, attention, cache, is_causal: bool = True, block=None
     if nbytes == 0:
         return None
     ws = torch.empty(nbytes, dtype=torch.uint8, device=raw.device)
-    _lib.check(lib.tsattn_cached_step(desc, ws.data_ptr(), nbytes, current_stream(x.device)),
-               "cached step")
+    _lib.check(launch(x.device, lib.tsattn_cached_step, desc, ws.data_ptr(), nbytes), "cached step")
     cache.length = stop
     return out
 

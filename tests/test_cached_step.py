@@ -28,7 +28,8 @@ def stub():
     with ExitStack() as stack:
         for patched in (patch.object(D.Device, "torch", torch.device("cpu")),
                         patch.object(D, "is_available", lambda value: True),
-                        patch.object(T, "current_stream", lambda dev: 0),
+                        patch.object(D, "current_stream", lambda dev: 0),
+                        patch.object(torch.cuda, "current_device", lambda: 0),
                         patch.object(_lib, "load", lambda: lib)):
             stack.enter_context(patched)
         yield calls
