@@ -36,6 +36,8 @@
 // their mean, into an empty one.  B4 H8 S777 D64, a [B,1,S,S] mask of three
 // documents a row and the causal flag, forward + backward: on the generic
 // kernels these problems ran on before 1455 us, here 180 us.
+#include <type_traits>
+
 #include "mfma_common.h"
 
 namespace tsattn {
@@ -184,6 +186,94 @@ struct F32Mask {
   }
 };
 
+// Infinities and NaN under a general mask.  A score's MFMA holds nothing of
+// another key or row, and a masked one is replaced whatever it is; the products
+// with P and dS sum over keys (rows), where 0 * inf is NaN.  As in the generic
+// kernels, P = 0 takes nothing from its key or row.  The tile loops run as if
+// all were finite; where a result is not, they run again with CAREFUL: non-finite
+// operands enter as 0, and the value rows' (V, dO) reach the rows (keys) with
+// P != 0 through add_nonfinite.  K and Q need no second step: beside one of
+// theirs that is not finite, P is 0 or the row's P and dS are not finite
+// themselves.  With the selects in the one loop D = 64 lost 5 - 10% and the
+// forward at D = 128 30 - 60%, by their registers; two walks cost 2 - 3% (B4 H8
+// S777 D64, packed documents, causal: forward 49.5 -> 51.9 us, backward 130 -> 133).
+__device__ __forceinline__ bool not_finite(float x) { return __builtin_amdgcn_classf(x, 0x207); }
+
+// acc += tile^T p, of the tile's non-finite elements and p != 0 (rare: a tile
+// with such elements; written for few registers).  A lane's 32 rows (keys) with
+// p != 0 as bits, and each channel's with +inf or NaN and with -inf or NaN.
+template <typename TL, int PDT>
+__device__ __forceinline__ void add_nonfinite(f32x16 (&acc)[PDT], const f32x16 &p, const char *tile, int c, int h) {
+  asm volatile("" : "+v"(c), "+v"(h));  // (its addresses are not to be kept across the tile loop)
+  uint32_t on = 0;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) on |= p[i] != 0.f ? 1u << (8 * (i >> 2) + (i & 3)) : 0u;
+  on <<= 4 * h;
+  on |= __shfl_xor(on, 32, 64);
+#pragma unroll
+  for (int dt = 0; dt < PDT; ++dt) {
+    uint32_t up = 0, down = 0;  // of channel 32 dt + c
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float v = TL::elem(tile, 8 * (i >> 2) + 4 * h + (i & 3), 32 * dt + c);
+      up |= __builtin_amdgcn_classf(v, 0x203) ? 1u << (8 * (i >> 2) + (i & 3)) : 0u;
+      down |= __builtin_amdgcn_classf(v, 0x007) ? 1u << (8 * (i >> 2) + (i & 3)) : 0u;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    up <<= 4 * h, down <<= 4 * h;
+    up |= __shfl_xor(up, 32, 64), down |= __shfl_xor(down, 32, 64);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int ch = 8 * (e >> 2) + 4 * h + (e & 3);  // this element's channel in the block
+      acc[dt][e] += (__shfl(up, ch, 64) & on ? INFINITY : 0.f) + (__shfl(down, ch, 64) & on ? -INFINITY : 0.f);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
+// Whether no score of the wave's 32 x 32 tile can overflow or be NaN, from its
+// operands' rows: lane (c, h) has half a row of each, `fixed` the sum of its
+// magnitudes for the one in registers (times the scale, if above 1), the other
+// in `tile`.  Then a tile whose additive mask is -inf throughout has P = 0; a
+// NaN or +inf score plus -inf would be NaN.
+template <typename TL, int HD>
+__device__ __forceinline__ bool scores_finite(float fixed, const char *tile, int c, int h) {
+  float sum = 0.f;
+#pragma unroll
+  for (int q = 0; q < HD / 4; ++q) {
+    const float4 x = TL::chunk(tile, c, h * (HD / 4) + q);
+    sum += fabsf(x.x) + fabsf(x.y) + fabsf(x.z) + fabsf(x.w);
+  }
+  return __ballot(!(sum < 1e18f && fixed < 1e18f)) == 0ull;  // |score| <= 4e36
+}
+template <int HD>
+__device__ __forceinline__ float magnitudes(const float (&x)[HD], float scale) {
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < HD; ++i) sum += fabsf(x[i]);
+  return sum * fmaxf(scale, 1.f);
+}
+
+// A lane's coordinate in a second walk over the tiles: the compiler does not see
+// that it is the first one's, so the addresses made of it are not kept in
+// registers from the first walk on.
+template <bool AGAIN>
+__device__ __forceinline__ int again_lane(int x) {
+  if constexpr (AGAIN) asm volatile("" : "+v"(x));
+  return x;
+}
+
+// whether an accumulator of the wave is not finite
+template <int N>
+__device__ __forceinline__ bool any_not_finite(const f32x16 (&acc)[N]) {
+  float t = 0.f;
+#pragma unroll
+  for (int n = 0; n < N; ++n)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) t = fmaf(acc[n][e], 0.f, t);
+  return __ballot(t != t) != 0ull;
+}
+
 struct F32Args {
   Problem p;
   View q, k, v, o, dout, dq, dk, dv;
@@ -294,7 +384,7 @@ __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
   // block n = w + NW u of the stage (split: n = u), K blocks first.  A tile
   // past the last one reads past the buffer ranges (zeros, no memory access)
   // into the spare block, so every wave issues the same parts.
-  auto issue_part = [&](int jj, int u) {
+  auto issue_part = [&](int jj, int u) __attribute__((always_inline)) {
     const int n = SPLIT ? u : w + NW * u;
     const int tile = first + STRIDE * jj;
     const bool real = tile < n_tiles;
@@ -353,8 +443,13 @@ __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
   }
 #pragma unroll
   for (int i = 0; i < HD; ++i) asm volatile("" : "+v"(qf[i]));
+  float qmag = 0.f;
+  if constexpr (ADD) qmag = magnitudes(qf, a.scale);
   if constexpr (!SPLIT) __syncthreads();
 
+  auto walk = [&](auto careful) __attribute__((always_inline)) {
+  constexpr bool CAREFUL = decltype(careful)::value;
+  const int c = again_lane<CAREFUL>(lane & 31), h = again_lane<CAREFUL>(lane >> 5);
   for (int jj = 0; jj < my_tiles; ++jj) {
     const int j = first + STRIDE * jj;
     const char *kt = ring_p + (jj & 1) * STAGE;
@@ -363,7 +458,7 @@ __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
     if constexpr (MK != 0) {
       mask.template take<true>(p, c, h);
       mask.issue_rows(p, mrs, qw, (j + STRIDE) * BN, c, h);  // (past the last tile: not used)
-      work = work && mask.any;
+      if (work && !mask.any) work = ADD && !scores_finite<TL, HD>(qmag, kt, c, h);
     }
     if (work) {
       // S^T = K Q^T, the next tile's parts spread over the steps; each
@@ -430,6 +525,7 @@ __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
       {
         constexpr int NS_ = 16 * PDT, FD = 2;
         float vf[FD + 1];
+        bool bad = false;  // V has an element that is not finite
         auto vload = [&](int t) {
           const int i = t / PDT, dt = t % PDT;
           vf[t % (FD + 1)] = TL::elem(vt, 8 * (i >> 2) + 4 * h + (i & 3), 32 * dt + c);
@@ -440,9 +536,16 @@ __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
 #pragma unroll
         for (int t = 0; t < NS_; ++t) {
           if (t + FD < NS_) vload(t + FD);
-          oacc[t % PDT] = mfma32f(vf[t % (FD + 1)], s[t / PDT], oacc[t % PDT]);
+          float v = vf[t % (FD + 1)];
+          if constexpr (CAREFUL) {
+            const bool nf = not_finite(v);
+            bad |= nf;
+            v = nf ? 0.f : v;
+          }
+          oacc[t % PDT] = mfma32f(v, s[t / PDT], oacc[t % PDT]);
           __builtin_amdgcn_sched_barrier(0);
         }
+        if (CAREFUL && __ballot(bad) != 0ull) add_nonfinite<TL>(oacc, s, vt, c, h);
       }
     } else {
 #pragma unroll
@@ -455,6 +558,23 @@ __global__ __launch_bounds__(NT, SPLIT ? 1 : 2) void fwd_f32_kernel(F32Args a) {
       wait_lgkm0();
     } else {
       __syncthreads();
+    }
+  }
+  };
+  walk(std::false_type{});
+  if constexpr (MK != 0) {
+    bool again = any_not_finite(oacc);
+    if constexpr (!SPLIT) again = __syncthreads_or(again);  // (the waves share the ring)
+    if (again) {
+#pragma unroll
+      for (int dt = 0; dt < PDT; ++dt) oacc[dt] = f32x16{};
+      m = thr = -INFINITY, l = nbase = 0.f;
+      mask.issue_rows(p, mrs, qw, first * BN, c, h);
+#pragma unroll
+      for (int u = 0; u < PARTS; ++u) issue_part(0, u);
+      wait_vm_n<0>();
+      if constexpr (!SPLIT) __syncthreads();
+      walk(std::true_type{});
     }
   }
 
@@ -645,7 +765,7 @@ __global__ __launch_bounds__(NT, 1) void dq_f32_kernel(F32Args a) {
   const char *ring_p = lds + (SPLIT ? w * 2 * STAGE : 0);
   const uint32_t spare = lds0 + RINGS * 2 * STAGE;
   // part u of local tile jj (tile first + STRIDE jj), as in the forward
-  auto issue_part = [&](int jj, int u) {
+  auto issue_part = [&](int jj, int u) __attribute__((always_inline)) {
     const int n = SPLIT ? u : w + NW * u;
     const int tile = first + STRIDE * jj;
     const bool real = tile < n_tiles;
@@ -695,8 +815,13 @@ __global__ __launch_bounds__(NT, 1) void dq_f32_kernel(F32Args a) {
   }
 #pragma unroll
   for (int i = 0; i < HD; ++i) asm volatile("" : "+v"(qf[i]), "+v"(gf[i]));
+  float qmag = 0.f;
+  if constexpr (MK >= 2) qmag = magnitudes(qf, a.scale);
   if constexpr (!SPLIT) __syncthreads();
 
+  auto walk = [&](auto careful) __attribute__((always_inline)) {
+  constexpr bool CAREFUL = decltype(careful)::value;
+  const int c = again_lane<CAREFUL>(lane & 31), h = again_lane<CAREFUL>(lane >> 5);
   for (int jj = 0; jj < my_tiles; ++jj) {
     const int j = first + STRIDE * jj;
     const char *kt = ring_p + (jj & 1) * STAGE;
@@ -705,7 +830,7 @@ __global__ __launch_bounds__(NT, 1) void dq_f32_kernel(F32Args a) {
     if constexpr (MK != 0) {
       mask.template take<true>(p, c, h);
       mask.issue_rows(p, mrs, qw, (j + STRIDE) * BN, c, h);  // (past the last tile: not used)
-      work = work && mask.any;
+      if (work && !mask.any) work = MK >= 2 && !scores_finite<TL, HD>(qmag, kt, c, h);
     }
     if (work) {
       f32x16 s = f32x16{}, dp = f32x16{};
@@ -760,6 +885,7 @@ __global__ __launch_bounds__(NT, 1) void dq_f32_kernel(F32Args a) {
         else x = (s[i] + nl) * sl;
         const float pv = ((kc_ < lm) & (((kbits >> kc_) & 1u) != 0)) ? fast_exp2(x) : 0.f;
         s[i] = pv * (dp[i] + nd);
+        if (CAREFUL && pv == 0.f) s[i] = 0.f;
       }
       // dQ^T += K^T dS^T: step i takes keys crow(i, h) (register i of dS^T)
       {
@@ -775,7 +901,9 @@ __global__ __launch_bounds__(NT, 1) void dq_f32_kernel(F32Args a) {
 #pragma unroll
         for (int t = 0; t < NS_; ++t) {
           if (t + FD < NS_) kload(t + FD);
-          acc[t % PDT] = mfma32f(kf[t % (FD + 1)], s[t / PDT], acc[t % PDT]);
+          float k = kf[t % (FD + 1)];
+          if constexpr (CAREFUL) k = not_finite(k) ? 0.f : k;
+          acc[t % PDT] = mfma32f(k, s[t / PDT], acc[t % PDT]);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -786,6 +914,22 @@ __global__ __launch_bounds__(NT, 1) void dq_f32_kernel(F32Args a) {
     wait_vm_n<0>();
     if constexpr (SPLIT) wait_lgkm0();  // (this wave's ring only)
     else __syncthreads();
+  }
+  };
+  walk(std::false_type{});
+  if constexpr (MK != 0) {  // (as in the forward)
+    bool again = any_not_finite(acc);
+    if constexpr (!SPLIT) again = __syncthreads_or(again);
+    if (again) {
+#pragma unroll
+      for (int dt = 0; dt < PDT; ++dt) acc[dt] = f32x16{};
+      mask.issue_rows(p, mrs, qw, first * BN, c, h);
+#pragma unroll
+      for (int u = 0; u < PARTS; ++u) issue_part(0, u);
+      wait_vm_n<0>();
+      if constexpr (!SPLIT) __syncthreads();
+      walk(std::true_type{});
+    }
   }
   float *orow = static_cast<float *>(const_cast<void *>(a.dq.data)) + b * a.dq.s0 + hq * a.dq.s1 +
                 static_cast<int64_t>(qrow < p.Sq ? qrow : 0) * a.dq.s2;
@@ -926,7 +1070,7 @@ __global__ __launch_bounds__(NT, 1) void dkdv_f32_kernel(F32Args a) {
   // its Q / dO blocks (split: all of them) and row values, and its part of a
   // general mask
   F32Mask<MK> mask;
-  auto issue = [&](int jj) {
+  auto issue = [&](int jj) __attribute__((always_inline)) {
     const int it = first + STRIDE * jj;
     const bool real = it < n_iter;
     const int r = real ? it / n_qt : 0, qi = real ? it - r * n_qt : 0;
@@ -972,8 +1116,13 @@ __global__ __launch_bounds__(NT, 1) void dkdv_f32_kernel(F32Args a) {
   wait_vm_n<0>();
 #pragma unroll
   for (int i = 0; i < HD; ++i) asm volatile("" : "+v"(kf[i]), "+v"(vf[i]));
+  float kmag = 0.f;
+  if constexpr (MK >= 2) kmag = magnitudes(kf, a.scale);
   if constexpr (!SPLIT) __syncthreads();
 
+  auto walk = [&](auto careful) __attribute__((always_inline)) {
+  constexpr bool CAREFUL = decltype(careful)::value;
+  const int c = again_lane<CAREFUL>(lane & 31), h = again_lane<CAREFUL>(lane >> 5);
   for (int jj = 0; jj < my_iter; ++jj) {
     const int it = first + STRIDE * jj;
     const char *qt = ring_p + (jj & 1) * STAGE;
@@ -984,7 +1133,7 @@ __global__ __launch_bounds__(NT, 1) void dkdv_f32_kernel(F32Args a) {
     bool work = true;
     if constexpr (MK != 0) {
       mask.template take<false>(p, c, h);
-      work = mask.any;
+      work = mask.any || (MK >= 2 && !scores_finite<TL, HD>(kmag, qt, c, h));
     }
     issue(jj + 1);
     if (work) {
@@ -1027,11 +1176,13 @@ __global__ __launch_bounds__(NT, 1) void dkdv_f32_kernel(F32Args a) {
       const float pv = ok ? fast_exp2(x) : 0.f;
       s[i] = pv;
       dp[i] = pv * (dp[i] + rvl[BN + rr]);
+      if (CAREFUL && pv == 0.f) dp[i] = 0.f;
     }
     // dV^T += dO^T P, dK^T += Q^T dS: step i takes rows crow(i, h)
     {
       constexpr int NS_ = 16 * PDT, FD = 2;
       float gfr[FD + 1], qfr[FD + 1];
+      bool bad = false;  // dO has an element that is not finite
       auto load = [&](int t) {
         const int i = t / PDT, dt = t % PDT, rr = 8 * (i >> 2) + 4 * h + (i & 3);
         gfr[t % (FD + 1)] = TL::elem(gt, rr, 32 * dt + c);
@@ -1043,15 +1194,37 @@ __global__ __launch_bounds__(NT, 1) void dkdv_f32_kernel(F32Args a) {
 #pragma unroll
       for (int t = 0; t < NS_; ++t) {
         if (t + FD < NS_) load(t + FD);
-        dva[t % PDT] = mfma32f(gfr[t % (FD + 1)], s[t / PDT], dva[t % PDT]);
-        dka[t % PDT] = mfma32f(qfr[t % (FD + 1)], dp[t / PDT], dka[t % PDT]);
+        float g = gfr[t % (FD + 1)], q = qfr[t % (FD + 1)];
+        if constexpr (CAREFUL) {
+          const bool nf = not_finite(g);
+          bad |= nf;
+          g = nf ? 0.f : g;
+          q = not_finite(q) ? 0.f : q;
+        }
+        dva[t % PDT] = mfma32f(g, s[t / PDT], dva[t % PDT]);
+        dka[t % PDT] = mfma32f(q, dp[t / PDT], dka[t % PDT]);
         __builtin_amdgcn_sched_barrier(0);
       }
+      if (CAREFUL && __ballot(bad) != 0ull) add_nonfinite<TL>(dva, s, gt, c, h);
     }
     }  // work
     wait_vm_n<0>();
     if constexpr (SPLIT) wait_lgkm0();  // (this wave's ring only)
     else __syncthreads();
+  }
+  };
+  walk(std::false_type{});
+  if constexpr (MK != 0) {  // (as in the forward)
+    bool again = any_not_finite(dka) || any_not_finite(dva);
+    if constexpr (!SPLIT) again = __syncthreads_or(again);
+    if (again) {
+#pragma unroll
+      for (int dt = 0; dt < PDT; ++dt) dka[dt] = dva[dt] = f32x16{};
+      issue(0);
+      wait_vm_n<0>();
+      if constexpr (!SPLIT) __syncthreads();
+      walk(std::true_type{});
+    }
   }
   const int krow_i = key < p.Sk ? key : 0;
   float *krow = static_cast<float *>(const_cast<void *>(a.dk.data)) + b * a.dk.s0 + hk * a.dk.s1 +

@@ -104,3 +104,92 @@ def test_f32_general_masks(case):
                      backend="streaming", enable_gqa=hkv != hq)
         for x, y, n in zip(got, (ref.out_cast, *ref.backward(inp.do)), names):
             np.testing.assert_allclose(x, y, **TOL, err_msg=n)
+
+
+NONFINITE = [
+    # (B, Hq, Hkv, S, D, mask): few row blocks (the split form) and enough of them (the whole form)
+    (1, 2, 2, 100, 64, "bool"), (1, 2, 1, 131, 32, "add"), (1, 2, 2, 135, 128, "bool"), (1, 2, 2, 135, 128, "add"),
+    (16, 16, 16, 97, 64, "bool"), (16, 16, 8, 129, 32, "add"), (16, 16, 16, 129, 64, "add"),
+]
+
+
+@pytest.mark.parametrize("case", NONFINITE, ids=lambda c: "x".join(map(str, c)))
+def test_masked_infinities_and_nan_stay_out(case):
+    """Infinities and NaN in K and V of masked keys, in Q and dO of rows that see
+    nothing, and in V and dO where they are seen: finite and non-finite where the
+    generic kernels are, which multiply with P != 0 only."""
+    b, hq, hkv, s, d, kind = case
+    print("f32 masks, non-finite operands", case, flush=True)
+    rng = np.random.default_rng(s + d)
+    inp = attention_inputs(b, hq, s, d, DT, heads_kv=hkv, seed=31)
+    q, k, v, g = (x.copy() for x in (inp.q, inp.k, inp.v, inp.do))
+    inf, nan = np.inf, np.nan
+    seen = rng.random((b, 1, s, s)) > 0.3
+    seen[..., 40:72, 32:64] = False     # a whole tile masked, and one in part
+    seen[:, :, :, [3, 45, 70]] = False  # keys nobody sees, with what a cache's unused rows can hold
+    k[:, :, 3], k[:, :, 45, 1], k[:, :, 70, 0] = nan, inf, -inf
+    v[:, :, 3], v[:, :, 45, 5], v[:, :, 70, 7] = nan, inf, -inf
+    seen[:, :, :, [10, 33]] = False     # keys some rows see, whose infinities and NaN these rows get
+    seen[:, :, 7, 10] = seen[:, :, 80, 10] = seen[:, :, 20, 33] = seen[:, :, 80, 33] = True
+    v[:, :, 10, [0, 9, 31]] = [inf, -inf, nan]
+    v[:, :, 33, [0, 9, 30]] = [inf, inf, -inf]
+    seen[:, :, [12, 50]] = False        # rows that see nothing
+    q[:, :, 12], q[:, :, 50, 2], g[:, :, 12, 4], g[:, :, 50] = nan, inf, inf, nan
+    g[:, :, 66, 6] = inf                # a row that does
+    mask = torch.from_numpy(seen).cuda()
+    if kind == "add":
+        mask = torch.zeros(mask.shape, device="cuda").masked_fill_(~mask, -inf)
+        k[:, :, [3, 45, 70]] = inp.k[:, :, [3, 45, 70]]  # (NaN + -inf is NaN: the next test)
+        q[:, :, [12, 50]] = inp.q[:, :, [12, 50]]
+    t = [abi.dev_tensor(x, DT) for x in (q, k, v, g)]
+
+    def run():
+        out, lse, path = abi.forward(*t[:3], mask=mask)
+        return path, [abi.host(x) for x in (out, *abi.backward(*t[:3], out, t[3], lse, mask=mask)[:3], lse)]
+
+    path, got = run()
+    assert path == _lib.PATH_MFMA
+    with abi.generic_only():
+        path, want = run()
+    assert path == _lib.PATH_GENERIC
+    assert np.isinf(want[0]).any() and np.isnan(want[0]).any() and np.isfinite(want[0]).mean() > 0.5
+    for x, y, n in zip(got, want, ("out", "dq", "dk", "dv", "lse")):
+        fine = np.isfinite(y)
+        np.testing.assert_array_equal(np.isfinite(x), fine, err_msg=n)
+        np.testing.assert_allclose(x[fine], y[fine], **TOL, err_msg=n)
+    for n, i in (("out", 0), ("dv", 3)):  # and the same infinities
+        np.testing.assert_array_equal(np.nan_to_num(got[i][~np.isfinite(want[i])], posinf=1, neginf=-1),
+                                      np.nan_to_num(want[i][~np.isfinite(want[i])], posinf=1, neginf=-1), err_msg=n)
+
+
+@pytest.mark.parametrize("what", ["K", "Q", "overflow"])
+@pytest.mark.parametrize("b,d", [(1, 64), (16, 64), (16, 128)])
+def test_a_tile_of_minus_infinity_is_skipped_only_where_that_is_exact(b, d, what):
+    """-inf added to a score that is NaN or overflows is NaN, also where it is -inf
+    for the whole tile."""
+    print("f32 masks, -inf tiles", b, d, what, flush=True)
+    h, s = 16, 130
+    inp = attention_inputs(b, h, s, d, DT, seed=37)
+    q, k, v, g = (x.copy() for x in (inp.q, inp.k, inp.v, inp.do))
+    if what == "K":
+        k[:, 0, 40, 3] = np.nan
+    elif what == "Q":
+        q[:, 0, 33, 3] = np.inf
+    else:
+        q[:, 0, 5], k[:, 0, 40] = 1e20, 1e20
+    mask = torch.zeros(1, 1, s, s, device="cuda")
+    mask[..., 32:64] = -np.inf
+    t = [abi.dev_tensor(x, DT) for x in (q, k, v, g)]
+
+    def run():
+        out, lse, path = abi.forward(*t[:3], mask=mask)
+        return [abi.host(x) for x in (out, *abi.backward(*t[:3], out, t[3], lse, mask=mask)[:3])]
+
+    got = run()
+    with abi.generic_only():
+        want = run()
+    assert np.isnan(want[0][:, 0]).any() and np.isfinite(want[0][:, 1:]).all()
+    for x, y, n in zip(got, want, ("out", "dq", "dk", "dv")):
+        np.testing.assert_array_equal(np.isfinite(x), np.isfinite(y), err_msg=n)
+        # (the head's rows are NaN, and their P without a sum to divide by: the others')
+        np.testing.assert_allclose(x[:, 1:], y[:, 1:], **TOL, err_msg=n)
