@@ -7,8 +7,8 @@
 // cross-lane sum a lane, so from a few rows on the kernel is bound by them and
 // not by HBM (4 rows, B64 Hkv8 D128 over 1025 f16 keys: 90 us for 268 MB, 3.0
 // TB/s; over int8 codes 48 us for 66 MB).  Here a 32-key tile of D = 128 takes
-// 8 MFMAs (16x16x32) for the scores and 16 or 24 for the values whatever the
-// rows (up to 16, of which 2 .. 8 are used): 400 to 500 cycles for 16 KB, a
+// 8 MFMAs (16x16x32) for the scores and 24 for the values whatever the
+// rows (up to 16, of which 2 .. 8 are used): about 500 cycles for 16 KB, a
 // fifth of its share of HBM.
 //
 // Measured, vector kernel -> this one: that f16 case 90 -> 48 us (5.6 TB/s), the
@@ -18,9 +18,11 @@
 //
 // Precision: q k products are exact in the MFMA and sum in fp32.  The
 // probabilities are fp32 and stay so: each enters the value product as a sum
-// of two f16 or three bf16 numbers (22 or 24 bits), one MFMA each over the
-// same value fragment.  f16 parts are taken of P 2^14, so that the second
-// part of all but vanishing probabilities is a normal number; the factor cancels in acc / l.
+// of three f16 or bf16 numbers, one MFMA each over the same value fragment.
+// The first two are truncated, so the three hold all 24 bits.  f16 parts are
+// taken of P 2^14 (the factor cancels in acc / l): below P = 2^-15, where the
+// last bits pass f16's smallest number, they are rounded at 2^-39 of the row's
+// largest P.
 //
 // Every wave works alone on the tiles w, w + NWV, ... of the split through an LDS
 // ring of its own (no barrier until the merge).  16-bit caches: K and V tiles
@@ -66,24 +68,25 @@ constexpr int dm_waves() {
   return Q8 ? (D == 256 ? 2 : 4) : (D == 64 ? 4 : (D == 128 ? 2 : 1));
 }
 
-// x = hi + lo (+ lo2), packed pairs of PT.
+// x = hi + mid + lo, packed pairs of PT: hi and mid truncated, lo what is left.
 template <typename PT>
 struct Parts {
-  static constexpr int N = std::is_same_v<PT, bf16> ? 3 : 2;
+  static constexpr int N = 3;
   __device__ __forceinline__ static void split(float a, float b, uint32_t (&out)[N]) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      out[i] = pack2<PT>(a, b);
-      if (i + 1 < N) {
-        if constexpr (std::is_same_v<PT, bf16>) {
-          a -= __builtin_bit_cast(float, out[i] << 16);
-          b -= __builtin_bit_cast(float, out[i] & 0xFFFF0000u);
-        } else {
-          a -= static_cast<float>(__builtin_bit_cast(f16, static_cast<uint16_t>(out[i])));
-          b -= static_cast<float>(__builtin_bit_cast(f16, static_cast<uint16_t>(out[i] >> 16)));
-        }
+    for (int i = 0; i < N - 1; ++i) {
+      if constexpr (std::is_same_v<PT, bf16>) {
+        const uint32_t x = __builtin_bit_cast(uint32_t, a), y = __builtin_bit_cast(uint32_t, b);
+        out[i] = __builtin_amdgcn_perm(y, x, 0x07060302u);
+        a -= __builtin_bit_cast(float, x & 0xFFFF0000u);
+        b -= __builtin_bit_cast(float, y & 0xFFFF0000u);
+      } else {
+        out[i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
+        a -= static_cast<float>(__builtin_bit_cast(f16, static_cast<uint16_t>(out[i])));
+        b -= static_cast<float>(__builtin_bit_cast(f16, static_cast<uint16_t>(out[i] >> 16)));
       }
     }
+    out[N - 1] = pack2<PT>(a, b);
   }
 };
 

@@ -6,12 +6,13 @@ after a 32-key tile and a wave's second tile, splits shorter than one tile per
 wave, every row count the routing sends here, caches whose rows are not
 contiguous ([B,S,H,D] memory), general and key-padding masks, an empty row.
 The bound is the rounding of the result to its dtype: the probabilities enter
-the value product with 22 (f16) or 24 (bf16) bits and the sums are fp32, so
-2e-6 of the row's largest value on top of half an ulp.
+the value product with all their bits and the sums are fp32, so 4e-6 of the row's
+largest value (sums over up to 700 keys) on top of half an ulp.
 """
 
 from __future__ import annotations
 
+import ctypes
 import math
 
 import pytest
@@ -112,3 +113,28 @@ def test_int8_decode_rows_match_float64(n, rep, d, split, dt):
     assert path == _lib.PATH_DECODE
     k, v = ((c.double() * s.double())[:, :, :n] for c, s in ((k8, ks), (v8, vs)))
     _check(out, _reference(q, k, v, n - 1, None), dt)
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d", [64, 128])
+def test_probabilities_enter_with_all_their_bits(d, dt):
+    """Over values that are one-hot a split's partial rows are its probabilities:
+    half of them are odd in their last of 24 bits."""
+    b, hkv, rep, n = 4, 2, 4, d
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    q, k = (torch.randn(b, h, s, d, generator=gen, device="cuda").to(dt) for h, s in ((hkv * rep, 1), (hkv, n)))
+    v = torch.eye(n, dtype=dt, device="cuda").expand(b, hkv, n, d).contiguous()
+    p = abi.problem(q, k, v)
+    lib, out = _lib.load(), torch.empty_like(q)
+    nbytes = lib.tsattn_decode_workspace(ctypes.byref(p), n)
+    ws = torch.zeros(nbytes // 4, device="cuda")
+    _lib.check(lib.tsattn_decode_forward(ctypes.byref(p), abi.view(q), abi.view(k), abi.view(v), abi.view(out), n,
+                                         ws.data_ptr(), nbytes, abi.stream()), "decode")
+    part = ws[:b * hkv * rep * (d + 2)].view(b, hkv, rep, d + 2)  # one split: acc, max, sum
+    bits = part[..., :d].contiguous().view(torch.int32)
+    seen = part[..., :d] > part[..., :d].amax(-1, keepdim=True) * 2.0**-15
+    assert seen.float().mean() > 0.9
+    odd = (bits[seen] & 1).float().mean().item()  # of 2048 and more: 0.5 +- 0.011
+    assert 0.45 < odd < 0.55, odd
+    total = part[..., :d].double().sum(-1)  # and their sum is the denominator, within its fp32 sums
+    assert ((part[..., d + 1].double() - total).abs() / total).max().item() <= 1e-6
