@@ -72,6 +72,22 @@ constexpr int dm_waves() {
 template <typename PT>
 struct Parts {
   static constexpr int N = 3;
+  // The parts over values that may be infinite: where x != 0 none is 0 (0 * inf
+  // would be NaN: f16's smallest number is 2^-38 of the row's largest P, bf16's
+  // normal one nothing), and beside an infinite hi (int8 caches' scales are in x)
+  // the others are finite.
+  __device__ __forceinline__ static void fill(float a, float b, uint32_t (&out)[N]) {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    constexpr uint16_t kTiny = std::is_same_v<PT, bf16> ? 0x0080 : 0x0001;
+    const u16x2 least = {a != 0.f ? kTiny : uint16_t(0), b != 0.f ? kTiny : uint16_t(0)};
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      u16x2 x = __builtin_bit_cast(u16x2, out[i]);
+      if (i > 0 && __builtin_isinf(a)) x[0] = 0;
+      if (i > 0 && __builtin_isinf(b)) x[1] = 0;
+      out[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(x, least));
+    }
+  }
   __device__ __forceinline__ static void split(float a, float b, uint32_t (&out)[N]) {
 #pragma unroll
     for (int i = 0; i < N - 1; ++i) {
@@ -186,22 +202,20 @@ __global__ __launch_bounds__((64 * dm_waves<D, Q8>()), (Q8 && D < 256 ? 2 : 1)) 
 #pragma unroll
   for (int e = 0; e < 2; ++e)
     voff_l[e] = ((4 * g + (c >> 2)) * 4 + ((2 * e + ((c & 3) >> 1)) ^ g)) * 16 + (c & 1) * 8;
-  auto krows = [&](const char *tile, int kb, int ks) { return ld16(tile + (kb * QG + ks) * 1024 + koff_l); };
-  auto vcols = [&](const char *tile, int dt) {
+  auto krows = [&](const char *tile, int kb, int ks) __attribute__((always_inline)) { return ld16(tile + (kb * QG + ks) * 1024 + koff_l); };
+  auto vcols = [&](const char *tile, int dt) __attribute__((always_inline)) {
     const char *blk = tile + (dt >> 1) * 1024 + voff_l[dt & 1];
     const u32x2 x = ds_read_tr<PT>(reinterpret_cast<const PT *>(blk));
     const u32x2 y = ds_read_tr<PT>(reinterpret_cast<const PT *>(blk + QG * 1024));
     return u32x4{x[0], x[1], y[0], y[1]};
   };
   f32x4 oacc[PDT];
-#pragma unroll
-  for (int dt = 0; dt < PDT; ++dt) oacc[dt] = f32x4{};
   // f16 parts are of P 2^14: the state's maximum is kept that much lower
   constexpr float kShift = std::is_same_v<PT, f16> ? 14.f : 0.f;
-  float m = -INFINITY, l = 0.f;
+  float m, l;
 
   // Scores of the K tile at kt: element i is key 16 (i / 4) + 4 g + i % 4
-  auto scores = [&](const char *kt, float (&x)[8]) {
+  auto scores = [&](const char *kt, float (&x)[8]) __attribute__((always_inline)) {
     f32x4 s[2] = {f32x4{}, f32x4{}};
     u32x4 kf[2][2];
 #pragma unroll
@@ -219,9 +233,9 @@ __global__ __launch_bounds__((64 * dm_waves<D, Q8>()), (Q8 && D < 256 ? 2 : 1)) 
   };
   // Scores x (log2 units) of tile j -> the probabilities' parts; the running
   // maximum is raised (and l, acc rescaled) as the reference's recurrence does.
-  // vsc: the tile's value scales (int8 caches).
+  // vsc: the tile's value scales (int8 caches).  filled: with Parts::fill.
   u32x4 pb[NP];
-  auto softmax = [&](float (&x)[8], int j, const float *vsc) {
+  auto softmax = [&](float (&x)[8], int j, const float *vsc, auto filled) __attribute__((always_inline)) {
     const int kv0 = j * BN;
     if (j >= edge || masked) {
       const int lim = klim - kv0 - 4 * g;
@@ -262,12 +276,13 @@ __global__ __launch_bounds__((64 * dm_waves<D, Q8>()), (Q8 && D < 256 ? 2 : 1)) 
       }
       uint32_t part[NP];
       Parts<PT>::split(p0, p1, part);
+      if constexpr (decltype(filled)::value) Parts<PT>::fill(p0, p1, part);
 #pragma unroll
       for (int n = 0; n < NP; ++n) pb[n][i >> 1] = part[n];
     }
   };
   // O^T += V^T P^T, every value fragment read once for the NP parts
-  auto values = [&](const char *vt) {
+  auto values = [&](const char *vt) __attribute__((always_inline)) {
     u32x4 vf[3];
     vf[0] = vcols(vt, 0);
     vf[1] = vcols(vt, 1);
@@ -279,6 +294,11 @@ __global__ __launch_bounds__((64 * dm_waves<D, Q8>()), (Q8 && D < 256 ? 2 : 1)) 
     }
   };
 
+  // The wave's walk over its tiles.
+  auto walk = [&](auto filled) __attribute__((always_inline)) {
+#pragma unroll
+  for (int dt = 0; dt < PDT; ++dt) oacc[dt] = f32x4{};
+  m = -INFINITY, l = 0.f;
   if constexpr (!Q8) {
     const u32x4 kdesc = make_desc(kbase, static_cast<uint32_t>(keys) * ks_b);
     const u32x4 vdesc = make_desc(vbase, static_cast<uint32_t>(keys) * vs_b);
@@ -286,7 +306,7 @@ __global__ __launch_bounds__((64 * dm_waves<D, Q8>()), (Q8 && D < 256 ? 2 : 1)) 
     const uint32_t koff = (lane >> 2) * ks_b + chunk * 16, voff = (lane >> 2) * vs_b + chunk * 16;
     // local tile t (tile w + NWV t of the split) into stage t & 1; tiles past
     // the last read past the buffer range (zeros, no memory access)
-    auto issue = [&](u32x4 desc, uint32_t off, uint32_t stride, int t, uint32_t half) {
+    auto issue = [&](u32x4 desc, uint32_t off, uint32_t stride, int t, uint32_t half) __attribute__((always_inline)) {
       const uint32_t st = lds0 + static_cast<uint32_t>(t & 1) * 2 * TILE + half;
       const uint32_t row = t < mine ? static_cast<uint32_t>((w + NWV * t) * BN) * stride : 0x80000000u;
 #pragma unroll
@@ -306,7 +326,7 @@ __global__ __launch_bounds__((64 * dm_waves<D, Q8>()), (Q8 && D < 256 ? 2 : 1)) 
       issue(vdesc, voff, vs_b, t + 1, TILE);  // (that stage's V was read for tile t - 1)
 #pragma unroll
       for (int i = 0; i < 8; ++i) x[i] *= a.sl;
-      softmax(x, w + NWV * t, nullptr);
+      softmax(x, w + NWV * t, nullptr, filled);
       __builtin_amdgcn_sched_barrier(0);
       wait_vm_n<2 * BLK>();  // V of tile t; K and V of t + 1 in flight
       __builtin_amdgcn_sched_barrier(0);
@@ -332,7 +352,7 @@ __global__ __launch_bounds__((64 * dm_waves<D, Q8>()), (Q8 && D < 256 ? 2 : 1)) 
       u32x2 k[NL], v[NL];
       float sc;
     };
-    auto load = [&](int t, Codes &x) {
+    auto load = [&](int t, Codes &x) __attribute__((always_inline)) {
       const int key0 = (w + NWV * t) * BN;
       const bool real = t < mine;
 #pragma unroll
@@ -345,7 +365,7 @@ __global__ __launch_bounds__((64 * dm_waves<D, Q8>()), (Q8 && D < 256 ? 2 : 1)) 
       const int key = min(key0 + (lane & 31), keys - 1);  // (past the split: its last key, masked)
       x.sc = sp[static_cast<int64_t>(k_begin + key) * sv.s2];
     };
-    auto compute = [&](int t, Codes &cd) {
+    auto compute = [&](int t, Codes &cd) __attribute__((always_inline)) {
       char *kt = mylds, *vt = mylds + TILE;
 #pragma unroll
       for (int u = 0; u < NL; ++u) {
@@ -370,7 +390,7 @@ __global__ __launch_bounds__((64 * dm_waves<D, Q8>()), (Q8 && D < 256 ? 2 : 1)) 
           vsc[4 * e + i] = v4[i];
         }
       }
-      softmax(x, w + NWV * t, vsc);
+      softmax(x, w + NWV * t, vsc, filled);
       values(vt);
       wait_lgkm0();  // the tile read before the next one overwrites it
       __builtin_amdgcn_sched_barrier(0);
@@ -385,6 +405,16 @@ __global__ __launch_bounds__((64 * dm_waves<D, Q8>()), (Q8 && D < 256 ? 2 : 1)) 
       }
     }
   }
+  };
+  walk(std::false_type{});
+  // sums that are not finite: again with filled parts (rare; its own code, so
+  // that the first walk keeps its registers)
+  float bad = 0.f;
+#pragma unroll
+  for (int dt = 0; dt < PDT; ++dt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bad = fmaf(oacc[dt][i], 0.f, bad);
+  if (__ballot(bad != bad) != 0ull) walk(std::true_type{});
 
   // Merge the waves: [wave][row][D | m | l] in LDS, then every thread sums its
   // share of the outputs over the waves.

@@ -138,3 +138,34 @@ def test_probabilities_enter_with_all_their_bits(d, dt):
     assert 0.45 < odd < 0.55, odd
     total = part[..., :d].double().sum(-1)  # and their sum is the denominator, within its fp32 sums
     assert ((part[..., d + 1].double() - total).abs() / total).max().item() <= 1e-6
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d,n,int8", [(64, 200, False), (128, 700, False), (256, 90, False), (64, 200, True),
+                                      (128, 700, True)])
+def test_infinite_values_stay_infinite(d, n, int8, dt):
+    """p inf is inf, whatever the parts p is split in; the other channels, splits
+    and heads are as they were."""
+    print("decode, infinite values", d, n, int8, dt, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    b, hkv, rep, inf = 2, 2, 4, math.inf
+    q = torch.randn(b, hkv * rep, 1, d, generator=gen, device="cuda").to(dt) * 0.5
+    if int8:
+        k, v = (torch.randint(-127, 128, (b, hkv, n, d), generator=gen, device="cuda", dtype=torch.int8)
+                for _ in range(2))
+        ks, vs = (torch.full((b, hkv, n, 1), 0.02, device="cuda") for _ in range(2))
+        v[:, 0, 7, 3], vs[:, 0, 7] = 0, inf  # (that channel: inf * 0)
+        out, _ = abi.decode_int8(q, k, v, ks, vs, n, causal=True, offset=n - 1)
+        k, v = k.double() * ks.double(), v.double() * vs.double()
+    else:
+        k, v = (torch.randn(b, hkv, n, d, generator=gen, device="cuda").to(dt) for _ in range(2))
+        v[:, 0, 7, 3], v[:, 0, 75, 4], v[:, 0, 60, 5] = inf, -inf, math.nan
+        v[:, 0, 20, 6], v[:, 0, 21, 6] = inf, -inf
+        out = abi.decode(q, k, v, causal=True, offset=n - 1)
+    want = _reference(q, k, v, n - 1, None)
+    assert torch.isinf(want).any() and torch.isnan(want).any() and torch.isfinite(want[:, rep:]).all()
+    fine = torch.isfinite(want)
+    assert torch.equal(torch.nan_to_num(out[~fine].double(), posinf=1, neginf=-1),
+                       torch.nan_to_num(want[~fine], posinf=1, neginf=-1))
+    for x, y in ((out.masked_fill(~fine, 0), want.masked_fill(~fine, 0)), (out[:, rep:], want[:, rep:])):
+        _check(x, y, dt)
