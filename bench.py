@@ -65,7 +65,7 @@ LONG_B, LONG_H, LONG_S = 16, 16, 8192
 LM_LAYERS, LM_DIM, LM_HEADS, LM_FFN, LM_VOCAB, LM_B, LM_S = 6, 512, 8, 2048, 32000, 8, 1024
 ATTN_KERNELS = ("fwd_mfma", "bwd_dkdv_mfma", "bwd_dq_ds", "bwd_dq_mfma", "bwd_rows", "generic_fwd",
                 "generic_bwd_delta", "generic_bwd_dq", "generic_bwd_dkdv", "key_mask_lengths",
-                "decode_split", "decode_merge", "rope")
+                "decode_split", "decode_mfma", "decode_merge", "rope")
 
 
 def causal_fwd_flops(b, h, s, d):

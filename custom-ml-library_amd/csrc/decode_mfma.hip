@@ -65,7 +65,8 @@ __device__ __forceinline__ float quad_row_max(float x) {
 // prologue and merge run under the other's stream.
 template <int D, bool Q8>
 constexpr int dm_waves() {
-  return Q8 ? (D == 256 ? 2 : 4) : (D == 64 ? 4 : (D == 128 ? 2 : 1));
+  static_assert(!Q8 || D < 256, "int8 caches of 256 channels are the vector kernel's");
+  return Q8 || D == 64 ? 4 : (D == 128 ? 2 : 1);
 }
 
 // x = hi + mid + lo, packed pairs of PT: hi and mid truncated, lo what is left.
@@ -121,7 +122,7 @@ __device__ __forceinline__ u32x4 codes_to(u32x2 c) {
 
 // MK: the problem has a mask (its element reads cost registers and code).
 template <typename T, int D, bool Q8, bool MK>
-__global__ __launch_bounds__((64 * dm_waves<D, Q8>()), (Q8 && D < 256 ? 2 : 1)) void decode_mfma_kernel(DecArgs a) {
+__global__ __launch_bounds__((64 * dm_waves<D, Q8>()), (Q8 ? 2 : 1)) void decode_mfma_kernel(DecArgs a) {
   using KT = std::conditional_t<Q8, int8_t, T>;   // cache element type
   using PT = std::conditional_t<Q8, bf16, T>;     // value tiles and probability parts
   constexpr int NWV = dm_waves<D, Q8>();
@@ -457,7 +458,7 @@ __global__ __launch_bounds__((64 * dm_waves<D, Q8>()), (Q8 && D < 256 ? 2 : 1)) 
 template <typename T, bool Q8>
 void launch_t(const DecArgs &a, hipStream_t st) {
   const dim3 g(a.max_splits, a.p.Hkv, a.p.B);
-  Probe pr_(Q8 ? "decode_split_int8" : "decode_split", st);
+  Probe pr_(Q8 ? "decode_mfma_int8" : "decode_mfma", st);
   auto run = [&](auto d, auto mk) {
     constexpr int D = decltype(d)::value;
     decode_mfma_kernel<T, D, Q8, decltype(mk)::value><<<g, dim3(64 * dm_waves<D, Q8>()), 0, st>>>(a);

@@ -62,6 +62,15 @@ def _check(got, want, dtype):
     assert (err / scale).max().item() <= 4e-6, (err / scale).max().item()
 
 
+def _probed(run):
+    _lib.profile_reset()
+    _lib.profile_enable(True)
+    out = run()
+    torch.cuda.synchronize()
+    _lib.profile_enable(False)
+    return out, _lib.profile_read()
+
+
 def _caches(gen, b, h, n, d, layout):
     out = []
     for _ in range(2):
@@ -90,8 +99,8 @@ def test_decode_rows_match_float64(case):
         mask = torch.randn(b, 1, sq, n, generator=gen, device="cuda")
         mask[..., 32:96] = -math.inf
         kw["mask"] = mask
-    got = abi.decode(q, k, v, split_len=split, **kw)
-    assert _lib.last_kernel_path() == _lib.PATH_DECODE
+    got, probes = _probed(lambda: abi.decode(q, k, v, split_len=split, **kw))
+    assert "decode_mfma" in probes and "decode_split" not in probes
     _check(got, _reference(q, k, v, n - sq, mask), dt)
 
 
@@ -109,8 +118,11 @@ def test_int8_decode_rows_match_float64(n, rep, d, split, dt):
               for _ in range(2))
     ks, vs = (torch.rand(b, hkv, n + 5, 1, generator=gen, device="cuda") * 0.02 + 1e-4 for _ in range(2))
     vs[:, :, 7] = 30.0
-    out, path = abi.decode_int8(q, k8, v8, ks, vs, n, split_len=split, causal=True, offset=n - 1)
+    (out, path), probes = _probed(
+        lambda: abi.decode_int8(q, k8, v8, ks, vs, n, split_len=split, causal=True, offset=n - 1))
     assert path == _lib.PATH_DECODE
+    # 256 channels of codes are the vector kernel's
+    assert ("decode_mfma_int8" in probes) == (d < 256) and ("decode_split_int8" in probes) == (d == 256)
     k, v = ((c.double() * s.double())[:, :, :n] for c, s in ((k8, ks), (v8, vs)))
     _check(out, _reference(q, k, v, n - 1, None), dt)
 
