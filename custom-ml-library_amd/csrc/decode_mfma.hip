@@ -12,9 +12,8 @@
 // fifth of its share of HBM.
 //
 // Measured, vector kernel -> this one: that f16 case 90 -> 48 us (5.6 TB/s), the
-// int8 one 48 -> 23 us (2.9 TB/s); 2 rows, B16 Hkv16 D128 over 4000 bf16 keys,
-// at the card's copy rate: 98 us (5.3 TB/s).  One row stays on the vector
-// kernel, which reaches 6.5 TB/s there.
+// int8 one 48 -> 23 us (2.9 TB/s).  One row, and two over large caches
+// (decode_mfma_applies), stay on the vector kernel, which reaches 6.5 TB/s there.
 //
 // Precision: q k products are exact in the MFMA and sum in fp32.  The
 // probabilities are fp32 and stay so: each enters the value product as a sum
@@ -478,6 +477,20 @@ bool decode_mfma_applies(const DecArgs &a, int dtype, bool q8) {
   if (dtype != TSATTN_F16 && dtype != TSATTN_BF16) return false;
   if (a.rows < 2 || a.rows > 8 || !(a.sl > 0.f) || !isfinite(a.sl)) return false;
   if (q8 && a.p.Dqk == 256) return false;  // (its codes, accumulators and parts exceed the registers)
+  if (a.rows == 2) {
+    // Two rows are few enough for the vector kernel to reach HBM's rate, and
+    // then it is the faster one (16-bit, 64 sequences of 8 KV heads, 4000 keys: D64
+    // 85 us, here 93; D128 173 and 186): it takes what the last-level cache does
+    // not hold, 256 MiB (int8 at D128: half of that; 2000 keys 66 and 76 us), all of
+    // D256 (4 sequences, 1000 keys: 13.2 and 14.6), and at D128 many heads of few
+    // keys, which its shorter splits spread better (16 sequences, 1000 keys: 17.6
+    // and 19.3).  The rest is faster here (D64, 16 x 8 heads, 4000 keys: 42 and 27;
+    // int8 43 and 25; D128, 8 heads, 16000 keys: 31 and 21).
+    const Problem &p = a.p;
+    const int64_t heads = static_cast<int64_t>(p.B) * p.Hkv, mib = heads * p.Sk * p.Dqk * 2 * (q8 ? 1 : 2) >> 20;
+    if (p.Dqk == 256 || mib >= (q8 && p.Dqk == 128 ? 128 : 256)) return false;
+    if (p.Dqk == 128 && !q8 && heads >= 128 && p.Sk < 4000) return false;
+  }
   // a split's rows are addressed with 32-bit offsets from its first key
   const int64_t es = q8 ? 1 : 2, most = static_cast<int64_t>(a.split_len) + 64;
   return a.k.s2 > 0 && a.v.s2 > 0 && most * a.k.s2 * es < (int64_t(1) << 31) &&

@@ -181,3 +181,30 @@ def test_infinite_values_stay_infinite(d, n, int8, dt):
                        torch.nan_to_num(want[~fine], posinf=1, neginf=-1))
     for x, y in ((out.masked_fill(~fine, 0), want.masked_fill(~fine, 0)), (out[:, rep:], want[:, rep:])):
         _check(x, y, dt)
+
+
+@pytest.mark.parametrize("b,hkv,d,n,int8,kernel", [
+    (2, 2, 64, 200, False, "decode_mfma"), (2, 2, 128, 200, False, "decode_mfma"),
+    (2, 2, 128, 200, True, "decode_mfma_int8"), (1, 2, 256, 150, False, "decode_split"),
+    (16, 8, 128, 200, False, "decode_split"), (16, 8, 128, 4000, False, "decode_mfma"),
+    (16, 8, 64, 8300, False, "decode_split"), (16, 8, 128, 4200, True, "decode_split_int8")])
+def test_two_rows_take_the_faster_kernel(b, hkv, d, n, int8, kernel):
+    """Two rows a KV head on both sides of the rule, and one row on the vector kernel."""
+    print("decode, two rows", b, hkv, d, n, int8, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    q = torch.randn(b, 2 * hkv, 1, d, generator=gen, device="cuda").half()
+    if int8:
+        k, v = (torch.randint(-127, 128, (b, hkv, n, d), generator=gen, device="cuda", dtype=torch.int8) for _ in range(2))
+        ks, vs = (torch.rand(b, hkv, n, 1, generator=gen, device="cuda") * 0.02 + 1e-4 for _ in range(2))
+        run = lambda q: abi.decode_int8(q, k, v, ks, vs, n, causal=True, offset=n - 1)[0]
+    else:
+        k, v = (torch.randn(b, hkv, n, d, generator=gen, device="cuda").half() for _ in range(2))
+        run = lambda q: abi.decode(q, k, v, causal=True, offset=n - 1)
+    got, probes = _probed(lambda: run(q))
+    assert kernel in probes, sorted(probes)
+    one, probes = _probed(lambda: run(q[:, :hkv]))
+    assert "decode_split_int8" in probes if int8 else "decode_split" in probes
+    last = slice(b - 1, b)  # (one sequence against float64)
+    kd, vd = (k[last].double() * ks[last].double(), v[last].double() * vs[last].double()) if int8 else (k[last], v[last])
+    _check(got[last], _reference(q[last], kd, vd, n - 1, None), q.dtype)
+    _check(one[last], _reference(q[last, :hkv], kd, vd, n - 1, None), q.dtype)
