@@ -169,12 +169,16 @@ __global__ __launch_bounds__(NT) void wgrad_reduce_kernel(const float *part, int
   }
 }
 
-// One workgroup a CU (256): at two a CU the partial tiles' traffic doubles and
-// costs more than the second workgroup hides (8192 tokens, 512 x 512: 20 us
-// against 25; 768 x 768: 24 against 35).
+// About one workgroup a CU (256): at two a CU the partial tiles' traffic doubles
+// and costs more than the second workgroup hides (8192 tokens, 512 x 512: 20 us
+// against 25).  A number that divides the eight XCDs keeps each token range in
+// the L2s of the same XCDs; three, or five to seven, has every L2 read them all
+// (16384 tokens: 1024 x 1408, 3 splits 120 us, 4 58, the library's product 114; 768
+// x 1280, 5 splits 82, 8 41, the library 100).  Tiles past half of the CUs take 4 too
+// (1536 x 1536, 65536 tokens: 2 splits 528 us, 4 479).
 int wgrad_splits(int tokens, int M, int N) {
   const int64_t tiles = static_cast<int64_t>((M + BM - 1) / BM) * ((N + BM - 1) / BM);
-  int64_t s = (256 + tiles - 1) / tiles;
+  int64_t s = tiles >= 64 ? 4 : (tiles > 32 ? 8 : (256 + tiles - 1) / tiles);
   const int64_t most = (tokens + 4 * BT - 1) / (4 * BT);  // at least four stages a split
   if (s > most) s = most;
   if (s < 1) s = 1;

@@ -89,20 +89,29 @@ def linear(input: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
     return Tensor._from_op(out, given, backward, "linear")
 
 
+def _wgrad_pays(tokens: int, m: int, n: int) -> bool:
+    """Whether the split contraction is the faster one: a long product of an output
+    small enough to leave most of the chip idle otherwise.  Library and kernel, us:
+    512 x 512 over 8192 tokens 52 and 20, 1400 x 1400 67 and 47; 3072 x 768 over 4096
+    41 and 38, 4096 x 1024 48 and 51; at 2048 tokens both take about 19.  Outputs of
+    more than half as many 128 x 128 tiles as CUs lose their lead over many tokens
+    (1536 x 1536: 65536 tokens 543 and 485, 131072 852 and 1034), thin ones of many
+    tiles are mostly padding (16 x 16384 over 4096: 22 and 26)."""
+    tiles = -(-m // 128) * -(-n // 128)
+    return (tokens >= 4096 and tiles <= (144 if tokens < 65536 else 128)
+            and (tiles <= 64 or min(m, n) >= 128))
+
+
 def _weight_grad(g, x, dev, dtype, store):
     """``g^T x`` over the tokens, rounded to ``dtype`` and given in ``store`` (that
-    or float32, into which the kernel widens the rounded sums): one split contraction kernel
-    (``tsattn_linear_wgrad``) where the product is long and its output small
-    enough to leave most of the chip idle otherwise -- 4096 tokens and up to
-    3072 x 768 outputs (512 x 512, 8192 tokens: 53 us as a library product, 20
-    here; 3072 x 768, 4096 tokens: 45 and 43; 4096 x 1024: 48 and 51; at 2048
-    tokens both take about 19 us)."""
+    or float32, into which the kernel widens the rounded sums): one split contraction
+    kernel (``tsattn_linear_wgrad``) where that pays, else the library's product."""
     import torch
 
     tokens, m = g.shape
     n = x.shape[1]
-    if (g.dtype not in (torch.float16, torch.bfloat16) or x.dtype != g.dtype or tokens < 4096
-            or -(-m // 128) * -(-n // 128) > 144 or m % 8 or n % 8 or m == 0 or n == 0
+    if (g.dtype not in (torch.float16, torch.bfloat16) or x.dtype != g.dtype or not _wgrad_pays(tokens, m, n)
+            or m % 8 or n % 8 or m == 0 or n == 0
             or tokens * max(g.stride(0), x.stride(0)) * 2 >= 2**31
             or any(t.stride(1) != 1 or t.stride(0) % 8 or t.stride(0) < t.shape[1] or t.data_ptr() % 16
                    for t in (g, x))):

@@ -1,8 +1,8 @@
 """The split weight-gradient kernel against float64.
 
 Edges: fewer tokens than one stage, a split that ends inside a stage, more
-splits than one reducing pass, outputs one piece past a tile and smaller than
-one, strided operands; and F.linear's VJP on both sides of the rule.  Bound:
+splits than one reducing pass, eight and four splits of many tiles, outputs one
+piece past a tile and smaller than one, strided operands; and F.linear's VJP on both sides of the rule.  Bound:
 one rounding to the dtype and the fp32 sums.
 """
 
@@ -33,7 +33,7 @@ def _close(got, want, dtype, tokens):
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("tokens,m,n", [(1, 8, 8), (33, 136, 120), (161, 128, 264), (1000, 256, 128),
-                                        (4097, 512, 72), (9000, 64, 136)])
+                                        (4097, 512, 72), (9000, 64, 136), (1300, 776, 904), (600, 1160, 1032)])
 def test_wgrad_matches_float64(tokens, m, n, dt):
     print("wgrad", tokens, m, n, dt, flush=True)
     gen = torch.Generator(device="cuda").manual_seed(tokens)

@@ -1,0 +1,21 @@
+"""Which sizes the layer kernels take, on both sides of each rule's lines: sizes
+where the library's product or the chain of array operations measured faster are
+not theirs."""
+
+from __future__ import annotations
+
+import pytest
+
+pytest.importorskip("torch")
+
+from tensorsmith_hip.nn import functional as F  # noqa: E402
+
+
+@pytest.mark.parametrize("tokens,m,n,pays", [
+    (4095, 512, 512, False), (4096, 512, 512, True), (131072, 1024, 2048, True),
+    (8192, 1400, 1400, True), (4096, 3072, 768, True), (65535, 1536, 1536, True), (65536, 1536, 1536, False),
+    (4096, 4096, 1024, False), (32768, 18432, 16, False), (4096, 16, 16384, False), (4096, 16, 8192, True),
+    (4096, 128, 16384, True)])
+def test_weight_gradients(tokens, m, n, pays):
+    assert F._wgrad_pays(tokens, m, n) == pays
+    assert F._wgrad_pays(tokens, n, m) == pays
