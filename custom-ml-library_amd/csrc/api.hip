@@ -898,10 +898,12 @@ int tsattn_linear_wgrad(int32_t dtype, int32_t out_dtype, int32_t tokens, int32_
   const uintptr_t al = reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(x) |
                        reinterpret_cast<uintptr_t>(dw) | reinterpret_cast<uintptr_t>(workspace);
   if (m % 8 || n % 8 || g_stride % 8 || x_stride % 8 || g_stride < m || x_stride < n || al % 16 ||
-      static_cast<int64_t>(tokens) * (g_stride > x_stride ? g_stride : x_stride) * 2 >= (int64_t(1) << 31) ||
+      // (the last stage's lanes form 32-bit offsets of up to 31 rows past the last token)
+      (static_cast<int64_t>(tokens) + 32) * (g_stride > x_stride ? g_stride : x_stride) * 2 >= (int64_t(1) << 31) ||
       static_cast<int64_t>(m) * n >= (int64_t(1) << 31))
     return fail(TSATTN_ERR_UNSUPPORTED,
-                "the weight gradient takes m and n %% 8 == 0, 16-byte aligned rows and operands below 2^31 bytes");
+                "the weight gradient takes m and n %% 8 == 0, 16-byte aligned rows and tokens + 32 rows below 2^31 "
+                "bytes");
   const size_t need = tsattn::wgrad_workspace_bytes(tokens, m, n);
   if (!workspace || workspace_bytes < need)
     return fail(TSATTN_ERR_INVALID, "weight gradient workspace too small: %zu < %zu bytes", workspace_bytes, need);

@@ -112,7 +112,7 @@ def _weight_grad(g, x, dev, dtype, store):
     n = x.shape[1]
     if (g.dtype not in (torch.float16, torch.bfloat16) or x.dtype != g.dtype or not _wgrad_pays(tokens, m, n)
             or m % 8 or n % 8 or m == 0 or n == 0
-            or tokens * max(g.stride(0), x.stride(0)) * 2 >= 2**31
+            or (tokens + 32) * max(g.stride(0), x.stride(0)) * 2 >= 2**31
             or any(t.stride(1) != 1 or t.stride(0) % 8 or t.stride(0) < t.shape[1] or t.data_ptr() % 16
                    for t in (g, x))):
         return (g.t() @ x).to(dtype)

@@ -465,7 +465,8 @@ int tsattn_rows_swiglu(int32_t dtype, int32_t rows, int32_t k, int32_t n, const 
  * VJP): dw [m, n] = g^T x over `tokens` rows, g [tokens, m] and x [tokens, n]
  * with row strides in elements; fp32 sums, rounded to dtype once and stored in
  * out_dtype: dtype, or f32 (the rounded value widened).  f16 or
- * bf16, m, n and the strides multiples of 8, 16-byte aligned arrays (others:
+ * bf16, m, n and the strides multiples of 8, 16-byte aligned arrays, tokens + 32
+ * rows of either operand below 2^31 bytes, m n below 2^31 (others:
  * TSATTN_ERR_UNSUPPORTED).  Deterministic.
  */
 int tsattn_linear_wgrad(int32_t dtype, int32_t out_dtype, int32_t tokens, int32_t m, int32_t n, const void *g, int64_t g_stride,

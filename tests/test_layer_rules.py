@@ -8,6 +8,7 @@ import pytest
 
 pytest.importorskip("torch")
 
+from tensorsmith_hip import _lib  # noqa: E402
 from tensorsmith_hip.nn import functional as F  # noqa: E402
 
 
@@ -19,3 +20,13 @@ from tensorsmith_hip.nn import functional as F  # noqa: E402
 def test_weight_gradients(tokens, m, n, pays):
     assert F._wgrad_pays(tokens, m, n) == pays
     assert F._wgrad_pays(tokens, n, m) == pays
+
+
+@pytest.mark.parametrize("tokens,stride", [(1, 2**29), (1, 2**25), (4096, 2**18 - 8)])
+def test_weight_gradients_refuse_rows_past_their_offsets(tokens, stride):
+    """Rows past the last token are addressed and read as zeros: with their 32-bit
+    offsets wrapped they would be token 0 again.  (Refused before any launch.)"""
+    lib, at = _lib.load(), 1 << 20
+    rc = lib.tsattn_linear_wgrad(_lib.F16, _lib.F16, tokens, 64, 64, at, stride, at, stride, at, at,
+                                 lib.tsattn_linear_wgrad_workspace(tokens, 64, 64), None)
+    assert rc == _lib.ERR_UNSUPPORTED
