@@ -127,19 +127,31 @@ def _weight_grad(g, x, dev, dtype, store):
     return out if dtype == g.dtype else out.to(dtype)
 
 
+def _rows_pays(rows: int, k: int, n: int) -> bool:
+    """Whether a few rows' product is the faster call on its own kernel: as long as
+    the library's, bound by some 19 us of host time, does not end in the GPU's
+    (K 4096, N 4096: 10 us here).  The kernel reads large weights at 4.5 TB/s, the
+    library a little faster (N 28672, K 4096, 1 row: 37 us here, 35 there; over 16
+    rows N 11008: 20 and 19; over 32 rows each weight is read by two row blocks:
+    N 16384, 64 rows: 51 and 32).  And a long contraction of few outputs is one
+    workgroup's serial chain (N 256: K 8192 12 and 19 us, 16384 21 and 19, 65536 72
+    and 43)."""
+    if rows > 32 and n > 8192:
+        return False
+    return n * k * 2 <= (96 if rows <= 16 else 64) << 20 and (k <= 8192 or n >= 4096)
+
+
 def _rows_linear(x, w, bias, dev):
     """``x W^T (+ bias)`` of a few 16-bit rows in one kernel
-    (``tsattn_rows_linear``), or None outside it.  Over 32 rows each weight is
-    read by two row blocks, and wide layers are the library's (K 4096, 64 rows:
-    N 4096 13 us here and 12 there, N 16384 51 and 32).  The kernel's offsets are
+    (``tsattn_rows_linear``), or None outside it.  The kernel's offsets are
     32-bit: rows picked out of a tensor of 2^31 bytes and more are the library's."""
     import torch
 
     rows, k = x.shape
     n = w.shape[0]
     if (x.dtype not in (torch.float16, torch.bfloat16) or w.dtype != x.dtype or not 0 < rows <= 64
-            or (rows > 32 and n > 8192) or k % 8 or n % 4 or k == 0 or n == 0 or x.stride(1) != 1
-            or x.stride(0) % 8 or (rows * x.stride(0) + k) * 2 >= 2**31 or k >= 2**25
+            or not _rows_pays(rows, k, n) or k % 8 or n % 4 or k == 0 or n == 0 or x.stride(1) != 1
+            or x.stride(0) % 8 or (rows * x.stride(0) + k) * 2 >= 2**31
             or not w.is_contiguous() or x.data_ptr() % 16 or w.data_ptr() % 16
             or (bias is not None and (bias.dtype != x.dtype or not bias.is_contiguous()
                                       or bias.data_ptr() % 16))):

@@ -30,3 +30,11 @@ def test_weight_gradients_refuse_rows_past_their_offsets(tokens, stride):
     rc = lib.tsattn_linear_wgrad(_lib.F16, _lib.F16, tokens, 64, 64, at, stride, at, stride, at, at,
                                  lib.tsattn_linear_wgrad_workspace(tokens, 64, 64), None)
     assert rc == _lib.ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("rows,k,n,pays", [
+    (1, 512, 32000, True), (16, 4096, 11008, True), (17, 4096, 11008, False), (32, 4096, 8192, True),
+    (1, 4096, 14336, False), (33, 4096, 8192, True), (33, 512, 8196, False), (1, 8192, 4, True),
+    (1, 8200, 4, False), (4, 1048576, 4, False), (1, 12288, 4096, True), (64, 8192, 5120, False)])
+def test_few_rows(rows, k, n, pays):
+    assert F._rows_pays(rows, k, n) == pays
