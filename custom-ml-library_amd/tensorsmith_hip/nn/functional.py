@@ -180,6 +180,14 @@ def gelu(input: Tensor) -> Tensor:
     return Tensor._from_op(out, (input,), backward, "bias_gelu")
 
 
+def _norm_pays(rows: int, dim: int) -> bool:
+    """Whether the norm kernel, a wave a row, is the faster one: many rows shorter
+    than a wave's lanes leave it idle (f32, 2^20 rows of 8, forward and VJP: 742 us
+    here, 209 as a chain of array operations; of 64: 1032 and 1646; 2^16 rows of 8: 65 and
+    109)."""
+    return dim >= 64 or rows <= 2**16
+
+
 def _norm(input: Tensor, weight: Tensor, bias: Tensor | None, eps: float, rms: bool) -> Tensor:
     """Layer / RMS norm over the trailing ``weight.ndim`` dims (reference
     ``primitives.py:67-136``): half inputs compute in float32, the VJP uses
@@ -196,7 +204,8 @@ def _norm(input: Tensor, weight: Tensor, bias: Tensor | None, eps: float, rms: b
     _require_hip(input, "rms_norm" if rms else "layer_norm")
     dim = math.prod(weight.shape)
     if (_code(input._data) >= 0 and _code(weight._data) >= 0 and 0 < dim <= 8192 and dim % 8 == 0
-            and input.size > 0 and (bias is None or bias.dtype == weight.dtype)):
+            and input.size > 0 and (bias is None or bias.dtype == weight.dtype)
+            and _norm_pays(input.size // dim, dim)):
         return _norm_kernel(input, weight, bias, eps, rms, dim, parents)
     axes = tuple(range(input.ndim - weight.ndim, input.ndim))
     x = _compute(input._data)

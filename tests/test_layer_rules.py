@@ -38,3 +38,9 @@ def test_weight_gradients_refuse_rows_past_their_offsets(tokens, stride):
     (1, 8200, 4, False), (4, 1048576, 4, False), (1, 12288, 4096, True), (64, 8192, 5120, False)])
 def test_few_rows(rows, k, n, pays):
     assert F._rows_pays(rows, k, n) == pays
+
+
+@pytest.mark.parametrize("rows,dim,pays", [(1, 8, True), (2**16, 8, True), (2**16 + 1, 8, False),
+                                           (2**16 + 1, 56, False), (2**20, 64, True), (2**20, 8192, True)])
+def test_norms(rows, dim, pays):
+    assert F._norm_pays(rows, dim) == pays
