@@ -696,10 +696,15 @@ bool mfma_supported(const Problem &p, int dtype) {
 
 // Key splits of a forward: as many as fill the two workgroups a CU runs (512; so
 // none above 256 row blocks), each of 11 key tiles (352 keys) or more of an
-// average row.  Unsplit / split, bf16 D128 B1 causal: 32 heads, 16 rows over 8192
-// keys 137 / 25 us, 256 rows 149 / 51; 8 heads of 4096 x 4096 80 / 61; 16 heads
-// of 2048 x 2048 44 / 41; and with shorter parts the merge costs more than the
-// split gains: 32 heads of 1024 x 1024 (8 tiles a part) 27 / 32 us.
+// average row, where that pays.  It takes the longest row block down from all its
+// keys to its part of them, or to what the whole chip has to do (two workgroups a CU
+// run 1.25 times as fast as one); it costs a merge kernel and two passes over
+// the partial rows, the time of 8 key tiles and one more for every 1024 rows (24
+// at most).  Unsplit / split, bf16 D128: causal, 32 heads, 16 rows over 8192 keys 137
+// / 25 us, 256 rows 149 / 51; 8 heads of 4096 x 4096 76 / 57; 16 heads of 2048 x 2048
+// 44 / 41.  Not causal, 1024 rows: 32 heads over 1024 keys 25 / 34 us, over 2048 43 /
+// 47, over 4096 80 / 74; 16 heads over 1024 23 / 26, over 2048 40 / 34; 8 heads over 1024
+// 22.6 / 21.8.
 int mfma_forward_splits(const Problem &p) {
   if (p.drop.on || mfma_mask_mode(p) != 0) return 1;
   const int64_t total = static_cast<int64_t>((p.Sq + BM - 1) / BM) * p.Hq * p.B;
@@ -708,7 +713,12 @@ int mfma_forward_splits(const Problem &p) {
   const int64_t most = keys / (11 * BN);
   int64_t s = 512 / total;
   if (s > most) s = most;
-  return s < 2 ? 1 : static_cast<int>(s);
+  if (s < 2) return 1;
+  const int64_t longest = p.causal && p.Sq + p.offset < p.Sk ? p.Sq + p.offset : p.Sk;
+  const int64_t part = longest / s, chip = total * keys / 320;
+  const int64_t rows = static_cast<int64_t>(p.B) * p.Hq * p.Sq;
+  const int64_t cost = BN * (rows < 16 * 1024 ? 8 + rows / 1024 : 24);
+  return longest - (part > chip ? part : chip) < cost ? 1 : static_cast<int>(s);
 }
 
 size_t mfma_forward_workspace(const Problem &p) {

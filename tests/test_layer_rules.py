@@ -1,8 +1,10 @@
-"""Which sizes the layer kernels take, on both sides of each rule's lines: sizes
-where the library's product or the chain of array operations measured faster are
-not theirs."""
+"""Which sizes the layer kernels and the split forward take, on both sides of each
+rule's lines: sizes where the library's product, the chain of array operations or
+the unsplit forward measured faster are not theirs."""
 
 from __future__ import annotations
+
+import ctypes
 
 import pytest
 
@@ -44,3 +46,17 @@ def test_few_rows(rows, k, n, pays):
                                            (2**16 + 1, 56, False), (2**20, 64, True), (2**20, 8192, True)])
 def test_norms(rows, dim, pays):
     assert F._norm_pays(rows, dim) == pays
+
+
+@pytest.mark.parametrize("b,h,sq,sk,causal,parts", [
+    (1, 32, 16, 8192, True, 16), (1, 32, 500, 8192, True, 4), (1, 8, 16, 704, False, 2), (1, 8, 1024, 1024, False, 2),
+    (1, 16, 1024, 1024, False, 1), (1, 32, 1024, 1024, False, 1), (1, 32, 1024, 2048, False, 1),
+    (1, 32, 1024, 4096, False, 2), (1, 16, 1024, 2048, False, 4), (1, 16, 2048, 2048, True, 2),
+    (1, 8, 4096, 4096, True, 2), (4, 32, 128, 800, False, 1), (4, 32, 128, 3000, False, 4), (1, 33, 1024, 8192, False, 1)])
+def test_split_forwards(b, h, sq, sk, causal, parts):
+    p = _lib.Problem()
+    p.dtype, p.batch, p.heads_q, p.heads_kv = _lib.BF16, b, h, h
+    p.len_q, p.len_kv, p.dim_qk, p.dim_v, p.scale = sq, sk, 128, 128, 0.1
+    p.is_causal, p.causal_offset, p.mask_kind = int(causal), sk - sq, _lib.MASK_NONE
+    want = parts * b * h * sq * 130 * 4 if parts > 1 else 0
+    assert _lib.load().tsattn_sdpa_forward_workspace(ctypes.byref(p)) == want
