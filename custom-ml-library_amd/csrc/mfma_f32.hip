@@ -1368,10 +1368,6 @@ bool mfma_f32_supported(const Problem &p, int dtype) {
   if (!(p.scale > 0.0) || p.drop.on || p.rope.R > 0) return false;
   // masks: any boolean one, or an additive one in f32 / f16 / bf16, read with
   // 32-bit offsets (f64 masks keep their precision on the generic kernels).
-  // Additive masks over fewer than 128 query rows (one workgroup's) stay on
-  // the generic kernels, where such problems are checked to run: not for
-  // speed (B1 H2 S96 D64 forward + backward 137 us there, 45 us here).
-  if (p.mask.kind == TSATTN_MASK_ADDITIVE && p.Sq < BM) return false;
   return mfma_mask_ok(p);
 }
 

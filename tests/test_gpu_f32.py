@@ -150,13 +150,13 @@ def test_f32_mfma_agrees_with_generic():
 
 
 def test_f32_outside_the_mfma_kernels_runs_generic():
-    """Head dim 48, a float mask or unequal value dim leave the fp32 MFMA
-    kernels; they still meet the bound on the generic ones."""
+    """Head dim 48, a float64 mask (kept in its precision) or unequal value dim
+    leave the fp32 MFMA kernels; they still meet the bound on the generic ones."""
     rng = np.random.default_rng(2)
-    for name, d, dv_, fmask in (("d48", 48, 48, False), ("float mask", 64, 64, True),
+    for name, d, dv_, fmask in (("d48", 48, 48, False), ("float64 mask", 64, 64, True),
                                 ("dv differs", 64, 32, False)):
         inp = attention_inputs(1, 2, 96, d, DT, dim_v=dv_, seed=3)
-        mask = (rng.standard_normal((96, 96)) * 1.5).astype(np.float32) if fmask else None
+        mask = rng.standard_normal((96, 96)) * 1.5 if fmask else None
         ref = A.sdpa(inp.q, inp.k, inp.v, mask, True, dtype=DT, backend="streaming")
         q, k, v, g = (abi.dev_tensor(x, DT) for x in (inp.q, inp.k, inp.v, inp.do))
         m = None if mask is None else torch.from_numpy(mask).cuda()

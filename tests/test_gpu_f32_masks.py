@@ -42,6 +42,10 @@ CASES = [
     (2, 8, 4, 513, 530, 32, False, 0, "add-bf16"),
     (2, 8, 8, 600, 600, 128, True, 0, "add-f16"),
     (2, 8, 8, 640, 640, 64, False, 0, "add-lowest"),
+    (1, 2, 2, 1, 200, 64, True, 199, "add-f32"),       # fewer rows than a workgroup's
+    (2, 3, 3, 33, 97, 32, False, 0, "add-bf16"),
+    (1, 2, 1, 96, 96, 64, True, 0, "add-f32"),
+    (2, 2, 2, 127, 127, 128, True, 0, "add-f16"),
 ]
 
 
@@ -55,7 +59,7 @@ def _mask(kind, b, h, sq, sk, rng):
     elif kind.startswith("add"):
         m = (rng.standard_normal((b, 1, sq, sk)) * 1.5).astype(np.float32)
         m[rng.random(m.shape) < 0.2] = -np.inf
-        m[..., 7, :] = -np.inf  # a row that sees nothing
+        m[..., 7:8, :] = -np.inf  # a row that sees nothing
         m[..., 40:72, 64:] = -np.inf
         if kind == "add-lowest":  # the type's lowest value on a whole row: its softmax is uniform
             m[..., 11, :] = np.finfo(np.float32).min
