@@ -5,7 +5,8 @@ Boolean and additive masks of any broadcast strides are read one tile ahead of
 the products, and a tile the mask forbids whole is skipped.  The cases sit
 where that can go wrong: ragged ends in both directions, one row or key more
 than a tile, strides that are not the key order, whole tiles and whole rows
-masked, grouped heads, and both forms (split and whole) of the kernels.  Bounds
+masked, grouped heads, and both forms (split and whole) of every mask's kernels,
+which their probes name.  Bounds
 as for the unmasked fp32 kernels: every product and sum is fp32.
 """
 
@@ -46,6 +47,11 @@ CASES = [
     (2, 3, 3, 33, 97, 32, False, 0, "add-bf16"),
     (1, 2, 1, 96, 96, 64, True, 0, "add-f32"),
     (2, 2, 2, 127, 127, 128, True, 0, "add-f16"),
+    # enough row blocks for the whole form (the key blocks of grouped heads: the split one)
+    (4, 32, 32, 257, 257, 64, True, 0, "add-f32"),
+    (4, 16, 16, 513, 513, 128, True, 0, "add-f32"),
+    (4, 32, 8, 300, 290, 32, False, 0, "add-bf16"),
+    (8, 16, 16, 300, 300, 64, False, 0, "add-lowest"),
 ]
 
 
@@ -85,10 +91,18 @@ def test_f32_general_masks(case):
     inp = attention_inputs(b, hq, sq, d, DT, heads_kv=hkv, seq_k=sk, seed=29)
     q, k, v, g = (abi.dev_tensor(x, DT) for x in (inp.q, inp.k, inp.v, inp.do))
     kw = dict(causal=causal, offset=off, mask=tm)
+    _lib.profile_reset()
+    _lib.profile_enable(True)
     out, lse, path = abi.forward(q, k, v, **kw)
     grads = abi.backward(q, k, v, out, g, lse, **kw)
     torch.cuda.synchronize()
+    _lib.profile_enable(False)
+    probes = _lib.profile_read()
     assert path == _lib.PATH_MFMA and grads[3] == _lib.PATH_MFMA
+    for name, blocks in (("fwd_mfma_f32_masked", -(-sq // 128) * hq * b), ("bwd_dq_mfma_f32_masked", -(-sq // 128) * hq * b),
+                         ("bwd_dkdv_mfma_f32_masked", -(-sk // 128) * hkv * b)):
+        split = d <= 64 and blocks < torch.cuda.get_device_properties(0).multi_processor_count
+        assert name + ("_split" if split else "") in probes, (name, split, sorted(probes))
     with abi.generic_only():
         out_g, lse_g, path = abi.forward(q, k, v, **kw)
         grads_g = abi.backward(q, k, v, out_g, g, lse_g, **kw)
