@@ -93,11 +93,16 @@ def _problem(b, hq, hkv, sq, sk, dqk, dv, dtype_code, scale, is_causal, offset):
 
 def _forward(lib, prob, rope, vq, vk, vv, vo, lse_ptr, tdev, stream) -> None:
     """The forward, with scratch for splitting the keys where the problem has
-    too few query row blocks to fill the chip (16-bit only; the question costs
-    a small fp32 step about 1 us of its 57)."""
+    too few query row blocks to fill the chip.  The library is asked (about 1 us
+    of host time) only for what it can split: 16-bit problems without dropout or
+    a general mask, of at most 256 blocks of 128 rows."""
     import torch
 
-    nbytes = lib.tsattn_sdpa_forward_workspace(ctypes.byref(prob)) if prob.dtype in (_lib.F16, _lib.BF16) else 0
+    nbytes = 0
+    if (prob.dtype in (_lib.F16, _lib.BF16) and not prob.dropout_p
+            and (prob.mask_kind == _lib.MASK_NONE or prob.kv_len)
+            and -(-prob.len_q // 128) * prob.heads_q * prob.batch <= 256):
+        nbytes = lib.tsattn_sdpa_forward_workspace(ctypes.byref(prob))
     ws = torch.empty(nbytes, dtype=torch.uint8, device=tdev) if nbytes else None
     _lib.check(lib.tsattn_sdpa_forward_split(
         ctypes.byref(prob), rope, vq, vk, vv, vo, lse_ptr,

@@ -1,0 +1,94 @@
+"""Launches and scratch as the host code asks for them: device tensors stand in as
+CPU ones, the library as a stub that notes each call, the current device and the
+stream."""
+
+from __future__ import annotations
+
+import importlib
+from contextlib import ExitStack, contextmanager
+from unittest.mock import patch
+
+import pytest
+
+torch = pytest.importorskip("torch")
+
+import tensorsmith_hip as ts  # noqa: E402
+from tensorsmith_hip import _lib, nn  # noqa: E402
+from tensorsmith_hip.nn import functional as F  # noqa: E402
+
+A = importlib.import_module("tensorsmith_hip.nn.attention")
+D = importlib.import_module("tensorsmith_hip.device")
+
+
+class Stub:
+    """Every entry point; the queries give 256 bytes, the launches succeed."""
+
+    def __init__(self):
+        self.current, self.calls, self.asked = 0, [], []
+
+    def __getattr__(self, name):
+        if name.endswith("_workspace"):
+            return lambda *a: self.asked.append(name) or 256
+        return lambda *a: self.calls.append((name, self.current, a[-1])) or 0
+
+    @contextmanager
+    def device(self, index):
+        before, self.current = self.current, index
+        yield
+        self.current = before
+
+
+@pytest.fixture
+def lib():
+    lib = Stub()
+    with ExitStack() as stack:
+        for patched in (patch.object(D.Device, "torch", torch.device("cpu")),
+                        patch.object(D, "is_available", lambda value: True),
+                        patch.object(D, "current_stream", lambda dev: 0x100 + dev.index),
+                        patch.object(A, "current_stream", lambda dev: 0x100 + dev.index),
+                        patch.object(torch.cuda, "current_device", lambda: lib.current),
+                        patch.object(torch.cuda, "device", lib.device),
+                        patch.object(_lib, "load", lambda: lib)):
+            stack.enter_context(patched)
+        yield lib
+
+
+@pytest.mark.parametrize("index", [0, 1])
+def test_layers_launch_on_their_tensors_device(lib, index):
+    dev = f"hip:{index}"
+    draw = lambda *s: ts.Tensor(torch.randn(s).half(), device=dev, requires_grad=True)
+    w, gate, up = draw(64), draw(4, 64), draw(4, 64)
+    F.rms_norm(draw(4, 64), w).backward(draw(4, 64))
+    F.layer_norm(draw(4, 64), w, draw(64)).backward(draw(4, 64))
+    F._silu_mul(gate, up).backward(draw(4, 64))
+    F.linear(draw(4, 64), draw(64, 64))
+    F.linear(draw(4096, 64), draw(64, 64)).backward(draw(4096, 64))
+    block = nn.TransformerDecoderBlock(256, 4, 512, device=dev).eval()
+    block.to(dtype="float16")
+    cache = block.attention.new_cache(1, 256, dtype="float16")
+    cache.length = 200
+    with ts.no_grad():
+        block(draw(1, 1, 256), cache=cache)
+    names = {name for name, _, _ in lib.calls}
+    assert names == {"tsattn_norm_forward", "tsattn_norm_backward", "tsattn_silu_mul", "tsattn_silu_mul_backward",
+                     "tsattn_rows_linear", "tsattn_linear_wgrad", "tsattn_cached_step"}
+    for name, current, stream in lib.calls:
+        assert (current, getattr(stream, "value", stream)) == (index, 0x100 + index), name
+    assert lib.current == 0
+
+
+def _attend(dtype=torch.float16, heads=2, s=200, mask=None, dropout=0.0):
+    q, k, v = (ts.Tensor(torch.randn(1, heads, s, 64).to(dtype), device="hip") for _ in range(3))
+    mask = None if mask is None else ts.Tensor(mask, device="hip")
+    return nn.scaled_dot_product_attention(q, k, v, mask, dropout, dropout == 0.0)
+
+
+def test_split_scratch_is_asked_for_where_a_forward_can_split(lib):
+    _attend()
+    _attend(mask=torch.ones(1, 1, 1, 200, dtype=torch.bool))  # key padding
+    assert lib.asked.count("tsattn_sdpa_forward_workspace") == 2
+    for kw in (dict(dtype=torch.float32), dict(dropout=0.5), dict(mask=torch.ones(200, 200, dtype=torch.bool)),
+               dict(mask=torch.ones(200, 200)), dict(heads=129)):
+        _attend(**kw)
+    assert lib.asked.count("tsattn_sdpa_forward_workspace") == 2
+    assert [name for name, _, _ in lib.calls].count("tsattn_sdpa_forward_split") == 7
