@@ -103,7 +103,12 @@ def _forward(lib, prob, rope, vq, vk, vv, vo, lse_ptr, tdev, stream) -> None:
             and (prob.mask_kind == _lib.MASK_NONE or prob.kv_len)
             and -(-prob.len_q // 128) * prob.heads_q * prob.batch <= 256):
         nbytes = lib.tsattn_sdpa_forward_workspace(ctypes.byref(prob))
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=tdev) if nbytes else None
+    ws = None
+    if nbytes:
+        try:
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=tdev)
+        except torch.OutOfMemoryError:  # no room for the parts: unsplit
+            nbytes = 0
     _lib.check(lib.tsattn_sdpa_forward_split(
         ctypes.byref(prob), rope, vq, vk, vv, vo, lse_ptr,
         None if ws is None else ctypes.c_void_p(ws.data_ptr()), nbytes, stream), "attention forward")

@@ -121,7 +121,10 @@ def _weight_grad(g, x, dev, dtype, store):
     lib = _lib.load()
     out = torch.empty((m, n), dtype=store, device=g.device)
     nbytes = lib.tsattn_linear_wgrad_workspace(tokens, m, n)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=g.device)
+    try:
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=g.device)
+    except torch.OutOfMemoryError:  # no room for the partial sums
+        return (g.t() @ x).to(dtype)
     _lib.check(launch(dev, lib.tsattn_linear_wgrad, _code(g), _code(out), tokens, m, n, g.data_ptr(), g.stride(0),
                       x.data_ptr(), x.stride(0), out.data_ptr(), ws.data_ptr(), nbytes), "linear weight gradient")
     return out if dtype == g.dtype else out.to(dtype)

@@ -24,12 +24,12 @@ class Stub:
     """Every entry point; the queries give 256 bytes, the launches succeed."""
 
     def __init__(self):
-        self.current, self.calls, self.asked = 0, [], []
+        self.current, self.calls, self.asked, self.args = 0, [], [], {}
 
     def __getattr__(self, name):
         if name.endswith("_workspace"):
             return lambda *a: self.asked.append(name) or 256
-        return lambda *a: self.calls.append((name, self.current, a[-1])) or 0
+        return lambda *a: self.args.update({name: a}) or self.calls.append((name, self.current, a[-1])) or 0
 
     @contextmanager
     def device(self, index):
@@ -92,3 +92,24 @@ def test_split_scratch_is_asked_for_where_a_forward_can_split(lib):
         _attend(**kw)
     assert lib.asked.count("tsattn_sdpa_forward_workspace") == 2
     assert [name for name, _, _ in lib.calls].count("tsattn_sdpa_forward_split") == 7
+
+
+def test_without_room_for_scratch_the_unsplit_paths_run(lib):
+    """Split forwards and weight gradients take scratch that the paths before them
+    did not: memory that has no room for it still runs those."""
+    empty = torch.empty
+
+    def full(*a, **kw):
+        if kw.get("dtype") == torch.uint8:
+            raise torch.OutOfMemoryError
+        return empty(*a, **kw)
+
+    x, w = (ts.Tensor(torch.randn(s).half(), device="hip", requires_grad=True) for s in ((4096, 64), (64, 64)))
+    out = F.linear(x, w)
+    with patch.object(torch, "empty", full):
+        _attend()
+        out.backward(ts.Tensor(torch.ones(4096, 64).half(), device="hip"))
+    assert not any(name == "tsattn_linear_wgrad" for name, _, _ in lib.calls)
+    assert lib.args["tsattn_sdpa_forward_split"][7:9] == (None, 0)  # workspace and its bytes
+    want = torch.ones(64, 4096).double() @ x._data.double()
+    assert ((w.grad._data.double() - want).norm() / want.norm()).item() <= 2e-3
