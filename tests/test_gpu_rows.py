@@ -11,6 +11,7 @@ sums (relative 2^-11 / 2^-8 of the result's scale a rounding).
 from __future__ import annotations
 
 import ctypes
+import importlib
 from unittest.mock import patch
 
 import pytest
@@ -25,6 +26,7 @@ import tensorsmith_hip as ts  # noqa: E402
 from tensorsmith_hip import _lib, nn  # noqa: E402
 from tensorsmith_hip.nn import functional as F  # noqa: E402
 
+T = importlib.import_module("tensorsmith_hip.nn.transformer")
 ULP = {torch.float16: 2.0**-11, torch.bfloat16: 2.0**-8}
 CODE = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}
 
@@ -133,6 +135,48 @@ def test_block_step_in_one_call_matches_the_layers(case):
     for a, b in zip(got["call"][1], got["layers"][1]):
         assert torch.equal(a, b)
     _close(got["call"][0], got["layers"][0].double(), dt, 8)
+
+
+MHA_STEPS = [
+    # (dtype, embed, heads, kv heads, batch, tokens, past, int8, bias, rotary, causal)
+    ("float16", 256, 4, 2, 3, 1, 140, False, True, True, True),
+    ("bfloat16", 256, 2, 1, 2, 3, 130, False, True, False, False),
+    ("float16", 512, 4, 4, 1, 4, 128, False, False, True, False),
+    ("float16", 256, 4, 2, 2, 1, 200, True, True, True, True),
+    ("bfloat16", 512, 4, 2, 2, 2, 150, True, True, False, False),
+    ("float16", 256, 2, 2, 33, 1, 127, True, False, False, True),
+]
+
+
+@pytest.mark.parametrize("case", MHA_STEPS, ids=lambda c: "-".join(map(str, c)))
+def test_attention_step_in_one_call_matches_the_layers(case):
+    """The attention layer alone: projection biases (of three weights side by side
+    over int8 caches), no rotation, tokens that see each other both ways."""
+    dtype, embed, heads, kv_heads, batch, tokens, past, int8, bias, rotary, causal = case
+    print("attention step", case, flush=True)
+    ts.seed(4)
+    dt = getattr(torch, dtype)
+    mha = nn.MultiHeadAttention(embed, heads, num_kv_heads=kv_heads, bias=bias, rotary=rotary, device="hip").eval()
+    mha.to(dtype=dtype)
+    gen = torch.Generator(device="cuda").manual_seed(past)
+    draw = lambda *s: ts.Tensor(torch.randn(s, generator=gen, device="cuda").to(dt), device="hip")
+    k, v, x = (draw(batch, kv_heads, past, embed // heads), draw(batch, kv_heads, past, embed // heads),
+               draw(batch, tokens, embed))
+    got, original, steps = {}, nn.KVCache._project_append, []
+    step = T._cached_step
+    for name in ("call", "layers"):
+        cache = mha.new_cache(batch, 256, dtype=dtype, quantized=int8)
+        with (ts.no_grad(), patch.object(T, "_cached_step", lambda *a, **kw: steps.append(step(*a, **kw)) or steps[-1]),
+              patch.object(nn.KVCache, "_project_append",
+                           original if name == "call" else lambda self, *a: original(self, *a))):
+            cache.append(k, v)
+            out = mha(x, cache=cache, is_causal=causal)
+        assert (steps.pop() is None) == (name == "layers")
+        assert cache.length == past + tokens
+        got[name] = (out._data, [t[:, :, past:past + tokens] for t in cache.storage if t is not None])
+    for a, b in zip(got["call"][1], got["layers"][1]):
+        assert torch.equal(a, b)
+    _close(got["call"][0], got["layers"][0].double(), dt, 6)
 
 
 def test_block_step_leaves_replaced_layers_alone():
