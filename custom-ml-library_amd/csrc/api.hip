@@ -506,16 +506,15 @@ int run_step(const tsattn_step_desc &d, const StepPlan &s, char *ws, hipStream_t
     // int8 caches: the quantiser needs a whole row, which a 32-channel tile of
     // the projection does not have: all rows first, then rotate and append
     // (the decode kernel rotates the queries)
-    tsattn::Probe pr_("qkv_rope_append_int8", st);
     const int kvw = d.heads_kv * D, n[3] = {static_cast<int>(W), kvw, kvw};
     const int64_t N = W + 2 * kvw;
-    if ((rc = hip_status(tsattn::launch_rows_linear(d.dtype, rows, E, n, x, E, w, bias, nullptr, 0, q, N, st, false),
+    if ((rc = hip_status(tsattn::launch_rows_linear(d.dtype, rows, E, n, x, E, w, bias, nullptr, 0, q, N, st),
                          "step projection launch")))
       return rc;
     vq = tsattn::View{q, L * N, D, N};
     const tsattn::View nk{q + W * 2, L * N, D, N}, nv{q + (W + kvw) * 2, L * N, D, N};
     rc = hip_status(tsattn::launch_rope_append(d.dtype, d.batch, d.heads_kv, L, D, d.cos ? D : 0, nk, nv, vk, vv,
-                                               &vks, &vvs, d.cos, d.sin, d.pos, st, false),
+                                               &vks, &vvs, d.cos, d.sin, d.pos, st),
                     "step append launch");
     if (rc) return rc;
   }

@@ -233,10 +233,10 @@ hipError_t launch_rope(int dtype, int B, int H, int T, int D, int R, View x, Vie
 
 hipError_t launch_rope_append(int dtype, int B, int H, int T, int D, int R, View k, View v, View kc,
                               View vc, const View *ks, const View *vs, const void *cos,
-                              const void *sin, int64_t pos, hipStream_t st, bool probed) {
+                              const void *sin, int64_t pos, hipStream_t st) {
   AppendArgs a{B, H, T, D, R, k, v, kc, vc, ks ? *ks : View{}, vs ? *vs : View{}, cos, sin, pos};
   const bool q8 = ks != nullptr;
-  Probe pr_(probed ? (q8 ? "rope_append_int8" : "rope_append") : nullptr, st);
+  Probe pr_(q8 ? "rope_append_int8" : "rope_append", st);
   const dim3 g = row_grid(B, H, T);
   if (dtype == TSATTN_F32) {
     if (q8) rope_append_kernel<float, true><<<g, NT, 0, st>>>(a);

@@ -204,10 +204,10 @@ void launch_t(const RowsArgs &a, bool dual, int tiles, hipStream_t st) {
 
 hipError_t launch_rows_linear(int dtype, int rows, int K, const int n[3], const void *x, int64_t xs,
                               const void *const w[3], const void *const bias[3], const void *res, int64_t rs,
-                              void *out, int64_t os, hipStream_t st, bool probed) {
+                              void *out, int64_t os, hipStream_t st) {
   RowsArgs a{rows, K, {n[0], n[1], n[2]}, x, {w[0], w[1], w[2]}, {bias[0], bias[1], bias[2]}, res, out, xs, rs, os};
   const int tiles = (n[0] + 31) / 32 + (n[1] + 31) / 32 + (n[2] + 31) / 32;
-  Probe pr_(probed ? "rows_linear" : nullptr, st);
+  Probe pr_("rows_linear", st);
   if (dtype == TSATTN_BF16) launch_t<bf16>(a, false, tiles, st);
   else launch_t<f16>(a, false, tiles, st);
   return hipGetLastError();

@@ -170,8 +170,7 @@ void probe_end(hipStream_t st);
 struct Probe {
   bool on;
   hipStream_t st;
-  // (name NULL: a launch under its caller's probe)
-  Probe(const char *name, hipStream_t s) : on(name && probes_on()), st(s) {
+  Probe(const char *name, hipStream_t s) : on(probes_on()), st(s) {
     if (on) probe_begin(name, st);
   }
   ~Probe() {
@@ -246,7 +245,7 @@ hipError_t launch_rope(int dtype, int B, int H, int T, int D, int R, View x, Vie
 // `pos`; ks / vs non-null for int8 caches (then quantised as the int8 append).
 hipError_t launch_rope_append(int dtype, int B, int H, int T, int D, int R, View k, View v, View kc,
                               View vc, const View *ks, const View *vs, const void *cos,
-                              const void *sin, int64_t pos, hipStream_t st, bool probed = true);
+                              const void *sin, int64_t pos, hipStream_t st);
 
 // The q / k / v projections of the `batch x len` rows of x (embed wide; a
 // [batch, 1, len, embed] view) with
@@ -289,7 +288,7 @@ hipError_t launch_silu_mul(int dtype, int64_t n, const void *gate, const void *u
 // W rows, 8-byte aligned out rows.  launch_rows_swiglu: silu(x gate^T) * (x up^T).
 hipError_t launch_rows_linear(int dtype, int rows, int K, const int n[3], const void *x, int64_t xs,
                               const void *const w[3], const void *const bias[3], const void *res, int64_t rs,
-                              void *out, int64_t os, hipStream_t st, bool probed = true);
+                              void *out, int64_t os, hipStream_t st);
 hipError_t launch_rows_swiglu(int dtype, int rows, int K, int N, const void *x, int64_t xs, const void *gate,
                               const void *up, void *out, int64_t os, hipStream_t st);
 

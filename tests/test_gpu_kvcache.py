@@ -207,10 +207,12 @@ def test_lm_with_int8_cache_decodes_through_the_int8_kernel():
         got, probes = run(False)
         want, probes_ref = run(True)
     assert probes["decode_split_int8"][0] == 4 * cfg.num_layers
-    # one fused projection + RoPE + quantising append (q, K and V) per layer and step
-    assert probes["qkv_rope_append_int8"][0] == 4 * cfg.num_layers
-    assert "kv_append_int8" not in probes and "rope_append_int8" not in probes
-    # the queries come out of it rotated: no separate RoPE launch
+    # one rotating, quantising append (K and V) per layer and step; with a mask the
+    # layers run one by one, the projections fused with it
+    assert probes["rope_append_int8"][0] == 4 * cfg.num_layers
+    assert probes_ref["qkv_rope_append_int8"][0] == 4 * cfg.num_layers
+    assert "kv_append_int8" not in probes and "kv_append_int8" not in probes_ref
+    # the queries are rotated in the decode or projection kernel: no separate RoPE launch
     assert "rope" not in probes and "rope" not in probes_ref
     assert "decode_split_int8" not in probes_ref and "decode_split" in probes_ref
     assert rel_l2(got, want) <= 5e-3
