@@ -31,7 +31,7 @@ from ctypes import POINTER, c_char_p, c_double, c_int, c_int32, c_int64, c_size_
 import numpy as np
 import torch
 
-ABI_VERSION = 8
+ABI_VERSION = 9
 OK, ERR_INVALID, ERR_UNSUPPORTED, ERR_HIP = 0, 1, 2, 3
 MASK_NONE, MASK_BOOL, MASK_ADDITIVE = 0, 1, 2
 BOOL_CODE = 4

@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define TSATTN_ABI_VERSION 8
+#define TSATTN_ABI_VERSION 9
 
 typedef enum {
   TSATTN_OK = 0,

@@ -41,7 +41,7 @@ def host(t):
 
 def test_binding_loads_abi():
     lib = B.load()
-    assert lib.tsattn_abi_version() == B.ABI_VERSION == 8
+    assert lib.tsattn_abi_version() == B.ABI_VERSION == 9
     assert B.Problem.dropout_bits.offset == 152
 
 
