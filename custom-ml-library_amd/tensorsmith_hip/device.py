@@ -54,7 +54,12 @@ def device(value: DeviceLike = None) -> Device:
         return Device("cpu")
     if isinstance(value, Device):
         return value
-    value = value.lower().strip()
+    return _parse(value.lower().strip())
+
+
+@cache
+def _parse(value: str) -> Device:
+    """One (immutable) object a device, so that most comparisons end at identity."""
     if value.startswith("hip:"):
         return Device("hip", int(value.split(":", 1)[1]))
     return Device(value)
@@ -189,21 +194,24 @@ def attention_dropout_key() -> int:
     return drawn
 
 
-def current_stream(dev: Device) -> int:
-    """Raw hipStream_t of torch's current stream on ``dev`` (0 = default)."""
+@cache
+def _cuda():
     import torch
 
-    return torch.cuda.current_stream(dev.torch).cuda_stream
+    return torch.cuda
+
+
+def current_stream(dev: Device) -> int:
+    """Raw hipStream_t of torch's current stream on ``dev`` (0 = default)."""
+    return _cuda().current_stream(dev.index).cuda_stream
 
 
 def launch(dev: Device, function, *args) -> int:
     """``function(*args, stream)``, a library call, on ``dev``'s current stream and
     with ``dev`` the current device: a kernel goes to the current device whatever
     its operands' is, and the default stream's handle (0) names no device."""
-    import torch
-
     stream = current_stream(dev)
-    if torch.cuda.current_device() == dev.index:
+    if _cuda().current_device() == dev.index:
         return function(*args, stream)
-    with torch.cuda.device(dev.index):
+    with _cuda().device(dev.index):
         return function(*args, stream)

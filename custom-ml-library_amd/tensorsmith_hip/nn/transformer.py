@@ -105,14 +105,15 @@ def _cached_step(x: Tensor, attention, cache, is_causal: bool = True, block=None
         return None
     if not all(_plain(m, Linear) for m in linear):
         return None
-    desc = _lib.StepDesc()
+    desc, dev = _lib.StepDesc(), x.device
     keep = [raw] if raw.is_contiguous() else [raw.contiguous()]
 
     def at(tensor, *shape):  # the pointer of a contiguous operand of the step's dtype and device, else 0
         if tensor is None:
             return None
         data = tensor._data
-        if tensor.device != x.device or data.dtype != raw.dtype or not data.is_contiguous() or tuple(data.shape) != shape:
+        if ((tensor.device is not dev and tensor.device != dev) or data.dtype != raw.dtype
+                or not data.is_contiguous() or tuple(data.shape) != shape):
             return 0
         keep.append(data)
         return data.data_ptr()
