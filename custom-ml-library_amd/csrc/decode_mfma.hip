@@ -5,15 +5,17 @@
 //
 // Why: on the vector units every row costs a key 16 multiplies and a
 // cross-lane sum a lane, so from a few rows on the kernel is bound by them and
-// not by HBM (4 rows, B64 Hkv8 D128 over 1025 f16 keys: 90 us for 268 MB, 3.0
+// not by HBM (4 rows, B64 Hkv8 D128 over 1025 f16 keys: 92 us for 268 MB, 2.9
 // TB/s; over int8 codes 48 us for 66 MB).  Here a 32-key tile of D = 128 takes
 // 8 MFMAs (16x16x32) for the scores and 24 for the values whatever the
-// rows (up to 16, of which 2 .. 8 are used): about 500 cycles for 16 KB, a
-// fifth of its share of HBM.
+// rows (up to 16, of which 2 .. 8 are used): about 500 cycles of one SIMD for
+// 16 KB, which leaves the matrix cores 95% idle at HBM's rate.
 //
-// Measured, vector kernel -> this one: that f16 case 90 -> 48 us (5.6 TB/s), the
-// int8 one 48 -> 23 us (2.9 TB/s).  One row, and two over large caches
-// (decode_mfma_applies), stay on the vector kernel, which reaches 6.5 TB/s there.
+// Measured in a kernel trace, vector kernel -> this one: that f16 case 92 -> 52
+// us (5.2 TB/s), the int8 one 48 -> 23 us (2.8 TB/s, by the codes' conversion: 19
+// vector instructions an MFMA).  K and V by non-temporal DMA were 3 - 5% slower.
+// One row, and two over large caches (decode_mfma_applies), stay on the vector
+// kernel, which reaches 6.5 TB/s there.
 //
 // Precision: q k products are exact in the MFMA and sum in fp32.  The
 // probabilities are fp32 and stay so: each enters the value product as a sum

@@ -35,7 +35,7 @@
 // log2 e would overflow to -inf and turn a row of such keys, whose softmax is
 // their mean, into an empty one.  B4 H8 S777 D64, a [B,1,S,S] mask of three
 // documents a row and the causal flag, forward + backward: on the generic
-// kernels these problems ran on before 1455 us, here 180 us.
+// kernels these problems ran on before 1456 us, here 189 us.
 #include <type_traits>
 
 #include "mfma_common.h"
