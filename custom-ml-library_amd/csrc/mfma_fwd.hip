@@ -696,15 +696,17 @@ bool mfma_supported(const Problem &p, int dtype) {
 
 // Key splits of a forward: as many as fill the two workgroups a CU runs (512; so
 // none above 256 row blocks), each of 11 key tiles (352 keys) or more of an
-// average row, where that pays.  It takes the longest row block down from all its
-// keys to its part of them, or to what the whole chip has to do (two workgroups a CU
-// run 1.25 times as fast as one); it costs a merge kernel and two passes over
-// the partial rows, the time of 8 key tiles and one more for every 1024 rows (24
-// at most).  Unsplit / split, bf16 D128: causal, 32 heads, 16 rows over 8192 keys 137
-// / 25 us, 256 rows 149 / 51; 8 heads of 4096 x 4096 76 / 57; 16 heads of 2048 x 2048
-// 44 / 41.  Not causal, 1024 rows: 32 heads over 1024 keys 25 / 34 us, over 2048 43 /
-// 47, over 4096 80 / 74; 16 heads over 1024 23 / 26, over 2048 40 / 34; 8 heads over 1024
-// 22.6 / 21.8.
+// average row, where that pays on the GPU.  It takes the longest row block down from
+// all its keys to its part of them, or to what the chip has to do: with more than one
+// workgroup a CU two parts share one, 1.25 times as fast as one after the other, and
+// causal blocks end unevenly (half way from the average to the longest).  It costs
+// a merge kernel, the time of 9 key tiles, and the partial rows, of one key for
+// every 66 rows and further part.  Unsplit / split, bf16 D128: causal, 32 heads, 16
+// rows over 8192 keys 137 / 25 us, 256 rows 149 / 51; 8 heads of 4096 x 4096 76 / 57;
+// 16 heads of 2048 x 2048 44 / 41.  Not causal, 1024 rows: 32 heads over 1024 keys 25
+// / 34 us, over 2048 43 / 47, over 4096 80 / 74; 16 heads over 1024 23 / 26, over 2048
+// 40 / 34, 1000 rows over 1600 32.5 / 35.6; 8 heads over 1024 22.6 / 21.8.  Of 956 sizes
+// none that this splits is 1.5% slower than unsplit.
 int mfma_forward_splits(const Problem &p) {
   if (p.drop.on || mfma_mask_mode(p) != 0) return 1;
   const int64_t total = static_cast<int64_t>((p.Sq + BM - 1) / BM) * p.Hq * p.B;
@@ -715,9 +717,9 @@ int mfma_forward_splits(const Problem &p) {
   if (s > most) s = most;
   if (s < 2) return 1;
   const int64_t longest = p.causal && p.Sq + p.offset < p.Sk ? p.Sq + p.offset : p.Sk;
-  const int64_t part = longest / s, chip = total * keys / 320;
-  const int64_t rows = static_cast<int64_t>(p.B) * p.Hq * p.Sq;
-  const int64_t cost = BN * (rows < 16 * 1024 ? 8 + rows / 1024 : 24);
+  const int64_t part = longest / s, uneven = (keys + longest) / 2;
+  const int64_t chip = total * s > 256 ? uneven * 8 / (5 * s) : total * uneven / 320;
+  const int64_t cost = 9 * BN + static_cast<int64_t>(p.B) * p.Hq * p.Sq * (s - 1) / 66;
   return longest - (part > chip ? part : chip) < cost ? 1 : static_cast<int>(s);
 }
 

@@ -52,7 +52,9 @@ def test_norms(rows, dim, pays):
     (1, 32, 16, 8192, True, 16), (1, 32, 500, 8192, True, 4), (1, 8, 16, 704, False, 2), (1, 8, 1024, 1024, False, 2),
     (1, 16, 1024, 1024, False, 1), (1, 32, 1024, 1024, False, 1), (1, 32, 1024, 2048, False, 1),
     (1, 32, 1024, 4096, False, 2), (1, 16, 1024, 2048, False, 4), (1, 16, 2048, 2048, True, 2),
-    (1, 8, 4096, 4096, True, 2), (4, 32, 128, 800, False, 1), (4, 32, 128, 3000, False, 4), (1, 33, 1024, 8192, False, 1)])
+    (1, 8, 4096, 4096, True, 2), (4, 32, 128, 800, False, 1), (4, 32, 128, 3000, False, 4), (1, 33, 1024, 8192, False, 1),
+    (1, 16, 800, 1100, False, 1), (1, 16, 1000, 1600, False, 1), (1, 32, 500, 1600, False, 1),
+    (1, 32, 1024, 2400, True, 1), (3, 8, 1000, 1600, True, 1), (8, 8, 244, 1254, False, 1)])
 def test_split_forwards(b, h, sq, sk, causal, parts):
     p = _lib.Problem()
     p.dtype, p.batch, p.heads_q, p.heads_kv = _lib.BF16, b, h, h
