@@ -91,18 +91,28 @@ def _problem(b, hq, hkv, sq, sk, dqk, dv, dtype_code, scale, is_causal, offset):
     return p
 
 
+def _split_pays(prob) -> bool:
+    """Whether a split of the keys can be the faster call: 16-bit problems without
+    dropout or a general mask, of at most 256 blocks of 128 rows, whose unsplit kernel
+    takes longer than the host does over a split call (the question, the scratch, the
+    second launch: 21 - 24 us against 17 - 19).  Unsplit / split calls, 16 rows of 16
+    bf16 heads: D128 over 1024 keys 21 / 21 us, 1500 29 / 21; D64 over 1024 17 / 22,
+    1500 22 / 22, 2500 35 / 22; D32, 2 heads, over 1767 23 / 23."""
+    if (prob.dtype not in (_lib.F16, _lib.BF16) or prob.dropout_p
+            or not (prob.mask_kind == _lib.MASK_NONE or prob.kv_len)
+            or -(-prob.len_q // 128) * prob.heads_q * prob.batch > 256):
+        return False
+    longest = min(prob.len_kv, prob.len_q + prob.causal_offset) if prob.is_causal else prob.len_kv
+    return longest >= 1950 - 3 * (prob.dim_qk + prob.dim_v)
+
+
 def _forward(lib, prob, rope, vq, vk, vv, vo, lse_ptr, tdev, stream) -> None:
     """The forward, with scratch for splitting the keys where the problem has
-    too few query row blocks to fill the chip.  The library is asked (about 1 us
-    of host time) only for what it can split: 16-bit problems without dropout or
-    a general mask, of at most 256 blocks of 128 rows."""
+    too few query row blocks to fill the chip (the library is asked, where a split
+    can pay)."""
     import torch
 
-    nbytes = 0
-    if (prob.dtype in (_lib.F16, _lib.BF16) and not prob.dropout_p
-            and (prob.mask_kind == _lib.MASK_NONE or prob.kv_len)
-            and -(-prob.len_q // 128) * prob.heads_q * prob.batch <= 256):
-        nbytes = lib.tsattn_sdpa_forward_workspace(ctypes.byref(prob))
+    nbytes = lib.tsattn_sdpa_forward_workspace(ctypes.byref(prob)) if _split_pays(prob) else 0
     ws = None
     if nbytes:
         try:

@@ -77,21 +77,38 @@ def test_layers_launch_on_their_tensors_device(lib, index):
     assert lib.current == 0
 
 
-def _attend(dtype=torch.float16, heads=2, s=200, mask=None, dropout=0.0):
-    q, k, v = (ts.Tensor(torch.randn(1, heads, s, 64).to(dtype), device="hip") for _ in range(3))
+def _attend(dtype=torch.float16, heads=2, s=2000, mask=None, dropout=0.0, q_len=16, causal=True):
+    q, k, v = (ts.Tensor(torch.randn(1, heads, n, 64).to(dtype), device="hip") for n in (q_len, s, s))
     mask = None if mask is None else ts.Tensor(mask, device="hip")
-    return nn.scaled_dot_product_attention(q, k, v, mask, dropout, dropout == 0.0)
+    return nn.scaled_dot_product_attention(q, k, v, mask, dropout, causal and dropout == 0.0,
+                                           causal_offset=s - q_len if causal and dropout == 0.0 else 0)
 
 
 def test_split_scratch_is_asked_for_where_a_forward_can_split(lib):
     _attend()
-    _attend(mask=torch.ones(1, 1, 1, 200, dtype=torch.bool))  # key padding
+    _attend(mask=torch.ones(1, 1, 1, 2000, dtype=torch.bool))  # key padding
     assert lib.asked.count("tsattn_sdpa_forward_workspace") == 2
-    for kw in (dict(dtype=torch.float32), dict(dropout=0.5), dict(mask=torch.ones(200, 200, dtype=torch.bool)),
-               dict(mask=torch.ones(200, 200)), dict(heads=129)):
+    for kw in (dict(dtype=torch.float32), dict(dropout=0.5), dict(mask=torch.ones(16, 2000, dtype=torch.bool)),
+               dict(mask=torch.ones(16, 2000)), dict(heads=257), dict(heads=129, q_len=129), dict(s=1500)):
         _attend(**kw)
     assert lib.asked.count("tsattn_sdpa_forward_workspace") == 2
-    assert [name for name, _, _ in lib.calls].count("tsattn_sdpa_forward_split") == 7
+    assert [name for name, _, _ in lib.calls].count("tsattn_sdpa_forward_split") == 9
+
+
+@pytest.mark.parametrize("dims,q_len,kv_len,causal,offset,pays", [
+    # a split call is 21 - 24 us of host time: over fewer keys the unsplit kernel is through before
+    ((128, 128), 16, 1181, False, 0, False), ((128, 128), 16, 1182, False, 0, True),
+    ((64, 64), 16, 1565, True, 1549, False), ((64, 64), 16, 1566, True, 1550, True),
+    ((32, 32), 16, 1757, False, 0, False), ((32, 32), 16, 1758, False, 0, True),
+    ((64, 128), 16, 1373, False, 0, False), ((128, 64), 16, 1374, False, 0, True),
+    # a causal window that ends before the keys do
+    ((128, 128), 1000, 8000, True, 0, False), ((128, 128), 1000, 8000, True, 182, True)])
+def test_splits_that_their_host_time_hides(dims, q_len, kv_len, causal, offset, pays):
+    p = _lib.Problem()
+    p.dtype, p.batch, p.heads_q, p.heads_kv = _lib.BF16, 1, 4, 4
+    p.len_q, p.len_kv, p.dim_qk, p.dim_v = q_len, kv_len, *dims
+    p.is_causal, p.causal_offset, p.mask_kind = int(causal), offset, _lib.MASK_NONE
+    assert A._split_pays(p) == pays
 
 
 def test_without_room_for_scratch_the_unsplit_paths_run(lib):
