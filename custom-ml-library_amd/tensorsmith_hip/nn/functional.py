@@ -14,7 +14,7 @@ import ctypes
 import math
 
 from .. import _lib
-from ..amp import _cast_inputs
+from ..amp import _autocast, _cast_inputs
 from ..device import launch, random_uniform
 from ..tensor import Tensor, _sum_to_shape, is_grad_enabled, is_torch, no_grad
 from .attention import rotary_embedding, scaled_dot_product_attention
@@ -58,20 +58,23 @@ def linear(input: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
     """x @ W^T + b as one node (reference ``functional.py:63-90``), autocast-aware:
     the casts belong to the node, its gradients are rounded as the cast operands'
     would be and returned in the dtypes of the operands given."""
-    given = tuple(t for t in (input, weight, bias) if t is not None)
-    with no_grad():
-        input, weight, bias = _cast_inputs(input, weight, bias)
+    given = (input, weight) if bias is None else (input, weight, bias)
+    casts = bool(_autocast.get())
+    if casts:
+        with no_grad():
+            input, weight, bias = _cast_inputs(input, weight, bias)
     if input.ndim < 1 or weight.ndim != 2 or input.shape[-1] != weight.shape[1]:
         raise ValueError("linear expects [...,in_features] and [out_features,in_features]")
     parents = (input, weight) if bias is None else (input, weight, bias)
-    if any(p.device != input.device for p in parents):
+    dev = input.device
+    if any(p.device is not dev and p.device != dev for p in parents):
         raise ValueError("linear tensors must be on the same device")
     if bias is not None and bias.shape != (weight.shape[0],):
         raise ValueError("linear bias must have shape [out_features]")
     _require_hip(input, "linear")
     w = weight._data
     x = input._data.reshape(-1, weight.shape[1])
-    out = _rows_linear(x, w, None if bias is None else bias._data, input.device)
+    out = _rows_linear(x, w, None if bias is None else bias._data, dev)
     if out is None:
         out = x @ w.t()
         if bias is not None:
@@ -81,10 +84,10 @@ def linear(input: Tensor, weight: Tensor, bias: Tensor | None = None) -> Tensor:
     def backward(g):
         flat = g.reshape(-1, weight.shape[0])
         grads = [(flat @ w).reshape(input.shape).to(input.dtype),
-                 _weight_grad(flat, x, input.device, weight.dtype, given[1].dtype)]
+                 _weight_grad(flat, x, dev, weight.dtype, given[1].dtype)]
         if bias is not None:
             grads.append(flat.sum(0).to(bias.dtype))
-        return tuple(d.to(t.dtype) for d, t in zip(grads, given))
+        return tuple(d.to(t.dtype) for d, t in zip(grads, given)) if casts else tuple(grads)
 
     return Tensor._from_op(out, given, backward, "linear")
 
@@ -106,9 +109,11 @@ def _weight_grad(g, x, dev, dtype, store):
     """``g^T x`` over the tokens, rounded to ``dtype`` and given in ``store`` (that
     or float32, into which the kernel widens the rounded sums): one split contraction
     kernel (``tsattn_linear_wgrad``) where that pays, else the library's product."""
+    tokens, m = g.shape
+    if g.dtype.itemsize != 2 or tokens < 4096:
+        return (g.t() @ x).to(dtype)
     import torch
 
-    tokens, m = g.shape
     n = x.shape[1]
     if (g.dtype not in (torch.float16, torch.bfloat16) or x.dtype != g.dtype or not _wgrad_pays(tokens, m, n)
             or m % 8 or n % 8 or m == 0 or n == 0
@@ -148,11 +153,13 @@ def _rows_linear(x, w, bias, dev):
     """``x W^T (+ bias)`` of a few 16-bit rows in one kernel
     (``tsattn_rows_linear``), or None outside it.  The kernel's offsets are
     32-bit: rows picked out of a tensor of 2^31 bytes and more are the library's."""
+    rows, k = x.shape
+    if x.dtype.itemsize != 2 or rows > 64:
+        return None
     import torch
 
-    rows, k = x.shape
     n = w.shape[0]
-    if (x.dtype not in (torch.float16, torch.bfloat16) or w.dtype != x.dtype or not 0 < rows <= 64
+    if (x.dtype not in (torch.float16, torch.bfloat16) or w.dtype != x.dtype or rows == 0
             or not _rows_pays(rows, k, n) or k % 8 or n % 4 or k == 0 or n == 0 or x.stride(1) != 1
             or x.stride(0) % 8 or (rows * x.stride(0) + k) * 2 >= 2**31
             or not w.is_contiguous() or x.data_ptr() % 16 or w.data_ptr() % 16
@@ -202,11 +209,12 @@ def _norm(input: Tensor, weight: Tensor, bias: Tensor | None, eps: float, rms: b
     if bias is not None and bias.shape != weight.shape:
         raise ValueError("normalization bias and weight must have equal shapes")
     parents = (input, weight) if bias is None else (input, weight, bias)
-    if any(p.device != input.device for p in parents):
+    dev = input.device
+    if any(p.device is not dev and p.device != dev for p in parents):
         raise ValueError("normalization tensors must be on the same device")
     _require_hip(input, "rms_norm" if rms else "layer_norm")
     dim = math.prod(weight.shape)
-    if (_code(input._data) >= 0 and _code(weight._data) >= 0 and 0 < dim <= 8192 and dim % 8 == 0
+    if (0 < dim <= 8192 and dim % 8 == 0 and _code(input._data) >= 0 and _code(weight._data) >= 0
             and input.size > 0 and (bias is None or bias.dtype == weight.dtype)
             and _norm_pays(input.size // dim, dim)):
         return _norm_kernel(input, weight, bias, eps, rms, dim, parents)

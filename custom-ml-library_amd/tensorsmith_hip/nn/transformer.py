@@ -72,16 +72,16 @@ def _cached_step(x: Tensor, attention, cache, is_causal: bool = True, block=None
 
     raw = x._data
     if (raw.dtype not in (torch.float16, torch.bfloat16) or type(cache) is not KVCache
-            or _step_methods() != _STEP_METHODS or "_project_append" in vars(cache)
-            or cache.dtype != raw.dtype
-            or cache.device != x.device or attention.backend == "native"):
+            or cache.dtype != raw.dtype or attention.backend == "native"):
         return None
     b, t, e = raw.shape
     pos, stop = cache.length, cache.length + t
     heads, kv_heads, dim = attention.num_heads, attention.num_kv_heads, attention.head_dim
     if (stop > cache.max_seq_len or stop < DECODE_MIN_KEYS or b * t > 64 or (heads // kv_heads) * t > 8
             or dim not in (64, 128) or b != cache.batch_size or kv_heads != cache.num_heads
-            or dim != cache.head_dim or dim != cache.value_dim or t == 0):
+            or dim != cache.head_dim or dim != cache.value_dim or t == 0
+            or _step_methods() != _STEP_METHODS or "_project_append" in vars(cache)
+            or cache.device != x.device):
         return None
     linear = [attention.q_proj, attention.k_proj, attention.v_proj, attention.out_proj]
     hidden, widest = 0, e

@@ -130,3 +130,18 @@ def test_without_room_for_scratch_the_unsplit_paths_run(lib):
     assert lib.args["tsattn_sdpa_forward_split"][7:9] == (None, 0)  # workspace and its bytes
     want = torch.ones(64, 4096).double() @ x._data.double()
     assert ((w.grad._data.double() - want).norm() / want.norm()).item() <= 2e-3
+
+
+def test_layers_outside_the_kernels_take_the_plain_path(lib):
+    """Host time is what bounds small layers: without autocast a linear layer enters no
+    cast context, and what the kernels' first condition rules out asks nothing more."""
+    def refuse(*a, **kw):
+        raise AssertionError("asked")
+
+    draw = lambda *s: ts.Tensor(torch.randn(s), device="hip", requires_grad=True)
+    with patch.object(F, "no_grad", refuse), patch.object(F, "_rows_pays", refuse), \
+            patch.object(F, "_wgrad_pays", refuse), patch.object(F, "_code", refuse):
+        F.linear(draw(3, 100), draw(50, 100), draw(50)).backward(draw(3, 50))
+        F.linear(draw(5000, 8), draw(8, 8)).backward(draw(5000, 8))
+        F.rms_norm(draw(5, 100), draw(100)).backward(draw(5, 100))
+    assert not lib.calls and not lib.asked
