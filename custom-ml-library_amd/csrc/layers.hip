@@ -14,7 +14,7 @@
 // 2048): 1534 us with the chains (8 launches a norm and 11 its VJP, 5 and 7 the
 // activation), 1157 us with these (norm 10 us, its VJP 13 and the reduction 12);
 // a 6-layer model's cached step on 4 rows, which the launches bound, 2399 -> 1611 us
-// (and with the linear layers in rows.hip 340).
+// (and with the linear layers in rows.hip 315 - 350).
 #include <type_traits>
 
 #include "tsattn_internal.h"

@@ -19,7 +19,7 @@
 // 4096 x 4096 10.6 (3.2 TB/s; 64 rows 12.8); 4096 x 16384 29.7 us (4.5 TB/s).  The library's product
 // takes 12 us on the GPU at 4096 x 4096 and 64 rows and 18 us of host time a call,
 // which bounds it on every smaller layer.  The 6-layer model's cached step on 4
-// rows, with a block's step in one call: 1611 -> 340 us (51 launches, 238 us of GPU
+// rows, with a block's step in one call: 1611 -> 315 - 350 us (51 launches, 238 us of GPU
 // time); the attention layer's over int8 codes (B16 E2048, 4001 positions) 94 -> 41 us.
 #include <type_traits>
 
